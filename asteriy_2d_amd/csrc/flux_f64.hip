@@ -67,7 +67,7 @@ AST_DEV void store_face(double* __restrict__ out, size_t n, size_t i, double n1,
   out[n + i] = f.e;
   out[2 * n + i] = f.un * n1 - f.ut * n2;
   out[3 * n + i] = f.un * n2 + f.ut * n1;
-  const double t = krad / UU;
+  const double t = div64(krad, UU);
   out[4 * n + i] = METHOD == AST_HLL ? min2(1e7, t) : t;
 }
 
@@ -97,19 +97,37 @@ __global__ __launch_bounds__(FNT) void flux_kernel(size_t n, const double* __res
 // in LDS and solves them in that order, so that a wave's lanes mostly take
 // the same wave pattern and iteration loop (the faces of one wave otherwise
 // run the branches of every pattern one after another).  Each face's result
-// depends only on its own data.
-constexpr int SORT_PER = 4;
+// depends only on its own data.  The tile's faces stay in LDS (32 KiB) from
+// the coalesced classifying loads on: the solve reads its permuted faces
+// there and leaves its fluxes in their place, and the tile's fluxes go out
+// with coalesced stores.
+// Bound by the FP64 issue of the solvers, 104 B/face: 2^22 faces in 191 us
+// (22 Gfaces/s, 2.3 TB/s; 701 us with pow, the evaluated bisection and the
+// sorted faces re-read from global memory).  512-face tiles, one a
+// workgroup: four workgroups (of 34 KiB of LDS) and 16 waves a CU.
+constexpr int SORT_PER = 2;
 constexpr int STILE = FNT * SORT_PER;
 
+// the face's eight words in the frame of the normal (n1, n2)
+AST_DEV void face_frame(const double* w, double n1, double n2, PrimD& L, PrimD& R) {
+  L = PrimD{w[0], w[1], w[2] * n1 + w[3] * n2, -w[2] * n2 + w[3] * n1};
+  R = PrimD{w[4], w[5], w[6] * n1 + w[7] * n2, -w[6] * n2 + w[7] * n1};
+}
+
+// STATS: the variant that counts (the counters hold ten registers a lane).
+// G: the gas, with its order 1/gm compiled in or not.
+template <class G, bool STATS>
 __global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const double* __restrict__ in,
                                                            double n1, double n2, double krad,
-                                                           GasD gas, double* __restrict__ out,
+                                                           GasD gas0, double* __restrict__ out,
                                                            ast_stats_t* stats) {
+  const G gas(gas0);
   __shared__ uint32_t redi[(FNT / 64) * 10];
   __shared__ unsigned short perm[STILE];
   __shared__ int cnt[kPatternKeys + 1], cur[kPatternKeys + 1];
+  __shared__ double stage[8][STILE];  // the tile's faces, then (5 planes) its fluxes
   LaneStats st;
-  st.clear();
+  if constexpr (STATS) st.clear();
   const size_t ntiles = (n + STILE - 1) / STILE;
   for (size_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {  // workgroup-uniform
     const size_t base = tile * STILE;
@@ -122,8 +140,14 @@ __global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const doubl
       const int li = j * FNT + threadIdx.x;
       key[j] = kPatternKeys;  // past the end of the batch
       if (li < nv) {
+        double w[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          w[k] = in[k * n + base + li];
+          stage[k][li] = w[k];
+        }
         PrimD L, R;
-        load_face(in, n, base + li, n1, n2, L, R);
+        face_frame(w, n1, n2, L, R);
         key[j] = pattern_key(L, R, gas);
       }
       atomicAdd(&cnt[key[j]], 1);
@@ -149,27 +173,47 @@ __global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const doubl
     for (int j = 0; j < SORT_PER; j++) {
       const int pos = j * FNT + threadIdx.x;
       if (pos < nfaces) {
-        const size_t i = base + perm[pos];
+        const int li = perm[pos];
+        double w[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) w[k] = stage[k][li];
         PrimD L, R;
-        load_face(in, n, i, n1, n2, L, R);
+        face_frame(w, n1, n2, L, R);
         double UU;
         ExactInfo ei;
         const FluxD f = exact(L, R, gas, UU, ei);
-        st.add(ei);
-        store_face<AST_EXACT>(out, n, i, n1, n2, f, krad, UU);
+        if constexpr (STATS) st.add(ei);
+        // this lane alone holds face li: its words are read, its fluxes take
+        // their place
+        stage[0][li] = f.m;
+        stage[1][li] = f.e;
+        stage[2][li] = f.un * n1 - f.ut * n2;
+        stage[3][li] = f.un * n2 + f.ut * n1;
+        stage[4][li] = div64(krad, UU);
       }
     }
-    __syncthreads();  // perm and the counters are reused by the next tile
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < SORT_PER; j++) {
+      const int li = j * FNT + threadIdx.x;
+      if (li < nv) {
+#pragma unroll
+        for (int k = 0; k < 5; k++) out[k * n + base + li] = stage[k][li];
+      }
+    }
+    __syncthreads();  // stage, perm and the counters are reused by the next tile
   }
-  if (stats != nullptr) block_stats_to(st, redi, stats);
+  if constexpr (STATS) block_stats_to(st, redi, stats);
 }
 
 // The exact solver with per-face newton starting points and diagnostics.
+template <class G>
 __global__ __launch_bounds__(FNT) void guess_kernel(size_t n, const double* __restrict__ in,
-                                                    double n1, double n2, double krad, GasD gas,
+                                                    double n1, double n2, double krad, GasD gas0,
                                                     const float* __restrict__ guess,
                                                     double* __restrict__ out, ast_stats_t* stats,
                                                     int* __restrict__ info) {
+  const G gas(gas0);
   __shared__ uint32_t redi[(FNT / 64) * 10];
   LaneStats st;
   st.clear();
@@ -220,10 +264,15 @@ template <int METHOD>
 static int launch_flux(size_t n, const double* in, double n1, double n2, double krad,
                        const GasD& gas, double* out, ast_stats_t* stats, hipStream_t stream) {
   if constexpr (METHOD == AST_EXACT) {
+    // one tile per workgroup, a loop over tiles beyond 2^20 workgroups
     size_t blocks = (n + STILE - 1) / STILE;
-    if (blocks > 256 * 16) blocks = 256 * 16;
-    hipLaunchKernelGGL(exact_sorted_kernel, dim3((unsigned)blocks), dim3(FNT), 0, stream, n, in,
-                       n1, n2, krad, gas, out, stats);
+    if (blocks > (size_t(1) << 20)) blocks = size_t(1) << 20;
+    using G5 = GasN<5>;
+    const auto kernel =
+        gas.n == 5 ? (stats ? exact_sorted_kernel<G5, true> : exact_sorted_kernel<G5, false>)
+                   : (stats ? exact_sorted_kernel<GasD, true> : exact_sorted_kernel<GasD, false>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(FNT), 0, stream, n, in, n1, n2, krad,
+                       gas, out, stats);
     AST_LAUNCH_CHECK("ast_flux_f64 launch");
     return AST_OK;
   } else {
@@ -264,7 +313,8 @@ extern "C" int ast_flux_f64_guess(size_t n, const double* in, double n1, double 
   if (!in || !out) return ast_fail(AST_ERR_ARG, "ast_flux_f64_guess: null in/out");
   if (!(gamma > 1.0)) return ast_fail(AST_ERR_ARG, "ast_flux_f64_guess: gamma must be > 1");
   const GasD gas = ast::d64::make_gas(gamma);
-  hipLaunchKernelGGL(guess_kernel, dim3(flux_blocks(n)), dim3(FNT), 0, (hipStream_t)stream, n, in,
+  const auto kernel = gas.n == 5 ? guess_kernel<ast::d64::GasN<5>> : guess_kernel<GasD>;
+  hipLaunchKernelGGL(kernel, dim3(flux_blocks(n)), dim3(FNT), 0, (hipStream_t)stream, n, in,
                      n1, n2, krit * rad, gas, guess, out, stats, info);
   AST_LAUNCH_CHECK("ast_flux_f64_guess launch");
   return AST_OK;

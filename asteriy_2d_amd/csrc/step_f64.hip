@@ -25,6 +25,8 @@
 // direction, turns them into dt once, and workgroup minima lower *T with one
 // 64-bit atomicMin on the IEEE bits (positive doubles order like their
 // bits): the exact minimum over all faces, independent of the order.
+#include <type_traits>
+
 #include "common.hpp"
 #include "flux64.hpp"
 
@@ -151,8 +153,8 @@ AST_DEV void block_counters_to(const Counters& c, uint32_t* red, ast_stats_t* st
 // (kernel.cu:2812, 2838-2839, 2856).  Returns the flux in the face frame
 // (un: momentum along the normal, ut: along the other axis) and the face's
 // largest |wave speed|.
-template <int METHOD, bool WINDOW, bool NX>
-AST_DEV FluxD face(const Q& lv, const Q& rv, const Q& l, const Q& r, bool ho, const GasD& a,
+template <int METHOD, bool WINDOW, bool NX, class G>
+AST_DEV FluxD face(const Q& lv, const Q& rv, const Q& l, const Q& r, bool ho, const G& a,
                    double& UU, ExactInfo& info) {
   info.pat = -3;  // no exact solve
   if (WINDOW && !ho) {
@@ -186,12 +188,19 @@ struct StepArgs {
   int nwg;     // workgroups
 };
 
-template <int METHOD, int GEOM, bool WINDOW, bool STATS>
-__global__ __launch_bounds__(NT) void strip_kernel(StepArgs A) {
+// G: the gas, with its order 1/gm compiled in (the exact solver) or not.
+// Three waves a SIMD; the exact solver with the general power (232 VGPRs)
+// would spill 244 B a lane for the third, so it keeps two.
+template <int METHOD, class G>
+constexpr int step_waves() {
+  return METHOD == AST_EXACT && std::is_same<G, GasD>::value ? 2 : 3;
+}
+template <int METHOD, int GEOM, bool WINDOW, bool STATS, class G>
+__global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(StepArgs A) {
   __shared__ double red[WPB];
   __shared__ uint32_t redc[WPB * 10];
   const ast_grid_t& g = A.g;
-  const GasD& gas = A.gas;
+  const G gas(A.gas);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wg = xcd_tile(blockIdx.x, A.nwg);
   const int band = wg % A.nbands;
@@ -347,10 +356,16 @@ constexpr int kDefaultRows = 6;
 
 template <int METHOD, int GEOM, bool WINDOW>
 static int launch3(const StepArgs& a, bool stats, hipStream_t st) {
-  if (stats && METHOD == AST_EXACT)
-    hipLaunchKernelGGL((strip_kernel<METHOD, GEOM, WINDOW, true>), dim3(a.nwg), dim3(NT), 0, st, a);
-  else
-    hipLaunchKernelGGL((strip_kernel<METHOD, GEOM, WINDOW, false>), dim3(a.nwg), dim3(NT), 0, st, a);
+  auto kernel = strip_kernel<METHOD, GEOM, WINDOW, false, GasD>;
+  if constexpr (METHOD == AST_EXACT) {
+    using G5 = GasN<5>;
+    if (a.gas.n == 5)
+      kernel = stats ? strip_kernel<METHOD, GEOM, WINDOW, true, G5>
+                     : strip_kernel<METHOD, GEOM, WINDOW, false, G5>;
+    else if (stats)
+      kernel = strip_kernel<METHOD, GEOM, WINDOW, true, GasD>;
+  }
+  hipLaunchKernelGGL(kernel, dim3(a.nwg), dim3(NT), 0, st, a);
   AST_LAUNCH_CHECK("ast_step_f64 launch");
   return AST_OK;
 }
