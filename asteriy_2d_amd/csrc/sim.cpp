@@ -437,12 +437,12 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
   // default: strips of 4-16 rows, and the tilings that give every SIMD 2 to
   // 5 waves of (nearly) equal height, S strips per band with S * bands
   // waves (a wave strip has 60 output columns; a CU has 4 SIMDs); the FP64
-  // step takes strips of 4 to 32 rows
+  // step takes strips of 1 to 32 rows
   int dflt[8] = {4, 8, 12, 16};
-  static const int dflt64[6] = {4, 6, 8, 12, 16, 32};
+  static const int dflt64[11] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
   if ((!candidates || ncand <= 0) && S->precision == 0) {
     candidates = dflt64;
-    ncand = 6;
+    ncand = 11;
   }
   if (!candidates || ncand <= 0) {
     int nd = 4, dev = 0, cus = 0;

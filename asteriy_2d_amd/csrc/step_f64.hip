@@ -17,14 +17,22 @@
 // barrier inside the strip.  Slopes are the minmod of neighbour differences,
 // c +- minmod(c - a, b - c)/2, which is the reference's coordinate-difference
 // form (linear/linear2, kernel.cu:35-50) on a uniform grid without its
-// divisions.  Ghost cells follow the rules of ast_grid_t (fetch_cell).
+// divisions.
 //
 // The state stays in the reference's layout (two planes of double pairs);
-// loads and stores are 16-byte accesses of consecutive columns.  dt: each
+// loads and stores are 16-byte accesses of consecutive columns.  Row m+3 is
+// fetched while row m is computed.  Ghost cells follow the rules of
+// fetch_cell (common.hpp), split so that they cost the other cells nothing:
+// each lane loads the column its x rule names and each ghost row the row its
+// y rule names, and the rule's transform (mirrored, clamped or fixed state)
+// is applied a row later, when the fetch has arrived, under wave-uniform
+// branches that only the bands and rows with ghosts take.  Frozen cells are
+// looked for only by waves whose columns and rows can meet the region.  dt: each
 // wave keeps the largest |wave speed| of the faces it solved for each
 // direction, turns them into dt once, and workgroup minima lower *T with one
 // 64-bit atomicMin on the IEEE bits (positive doubles order like their
 // bits): the exact minimum over all faces, independent of the order.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -78,40 +86,86 @@ AST_DEV double minmod(double a, double b) { return fmax(fmin(a, b), fmin(fmax(a,
 // Face values c + s and c - s with s = minmod(c - a, b - c)/2 (dl = c - a,
 // dr = b - c).  A density or pressure face value <= 0 falls back to the cell
 // value (kernel.cu:2706-2788); that can only happen for a cell state that is
-// itself not positive.
+// itself not positive, so the four tests run only in waves where one of the
+// face values is not positive (c - |s| <= 0; wave-uniform).
 AST_DEV void face_values(const Q& c, const Q& dl, const Q& dr, Q& hi, Q& lo) {
-  const double sr = 0.5 * minmod(dl.r, dr.r), sp = 0.5 * minmod(dl.p, dr.p);
-  const double sx = 0.5 * minmod(dl.vx, dr.vx), sy = 0.5 * minmod(dl.vy, dr.vy);
-  hi = Q{c.r + sr, c.p + sp, c.vx + sx, c.vy + sy};
-  lo = Q{c.r - sr, c.p - sp, c.vx - sx, c.vy - sy};
-  if (hi.r <= 0.0) hi.r = c.r;
-  if (hi.p <= 0.0) hi.p = c.p;
-  if (lo.r <= 0.0) lo.r = c.r;
-  if (lo.p <= 0.0) lo.p = c.p;
+  const double sr = minmod(dl.r, dr.r), sp = minmod(dl.p, dr.p);
+  const double sx = minmod(dl.vx, dr.vx), sy = minmod(dl.vy, dr.vy);
+  // 0.5 s is exact: one fma rounds as c +- (0.5 s) does
+  hi = Q{fma(0.5, sr, c.r), fma(0.5, sp, c.p), fma(0.5, sx, c.vx), fma(0.5, sy, c.vy)};
+  lo = Q{fma(-0.5, sr, c.r), fma(-0.5, sp, c.p), fma(-0.5, sx, c.vx), fma(-0.5, sy, c.vy)};
+  const bool low = fma(-0.5, fabs(sr), c.r) <= 0.0 || fma(-0.5, fabs(sp), c.p) <= 0.0;
+  if (__builtin_amdgcn_ballot_w64(low) != 0) {
+    if (hi.r <= 0.0) hi.r = c.r;
+    if (hi.p <= 0.0) hi.p = c.p;
+    if (lo.r <= 0.0) lo.r = c.r;
+    if (lo.p <= 0.0) lo.p = c.p;
+  }
 }
 
-// Cell (n, m) with the ghost rules of ast_grid_t; positions that no output
-// cell reads (corners, columns past the halo of a partial band) take the
-// nearest grid cell, so every lane holds a finite, positive-where-the-grid-is
-// state.
-AST_DEV Q load_q(const ast_grid_t& g, const double2* __restrict__ s,
-                 const double2* __restrict__ u, int n, int m, double pulse) {
-  const bool xin = (n >= 0) & (n < g.N), yin = (m >= 0) & (m < g.M);
-  double2 a, b;
-  if (xin & yin) {
-    const size_t k = (size_t)m * g.N + n;
-    a = s[k];
-    b = u[k];
-  } else if ((xin | yin) & (n >= -2) & (n <= g.N + 1) & (m >= -2) & (m <= g.M + 1)) {
-    fetch_cell(g, s, u, n, m, a, b, pulse);
-  } else {
-    const int cn = n < 0 ? 0 : (n >= g.N ? g.N - 1 : n);
-    const int cm = m < 0 ? 0 : (m >= g.M ? g.M - 1 : m);
-    const size_t k = (size_t)cm * g.N + cn;
-    a = s[k];
-    b = u[k];
+// The column lane `n` of a row loads: itself, its ghost rule's source for
+// the two ghost columns of a side, else the nearest grid column (columns
+// past the halo of a partial band, read by no output cell).
+AST_DEV int source_column(const ast_grid_t& g, int n) {
+  if (n < 0) return g.bc[AST_XLO] == AST_BC_REFLECT ? -1 - n : 0;
+  if (n < g.N) return n;
+  return n <= g.N + 1 && g.bc[AST_XHI] == AST_BC_REFLECT ? 2 * g.N - 1 - n : g.N - 1;
+}
+// The row that row m loads, the same way (m >= -2; wave-uniform).
+AST_DEV int source_row(const ast_grid_t& g, int m) {
+  if (m < 0) return g.bc[AST_YLO] == AST_BC_REFLECT ? -1 - m : 0;
+  if (m < g.M) return m;
+  return m <= g.M + 1 && g.bc[AST_YHI] == AST_BC_REFLECT ? 2 * g.M - 1 - m : g.M - 1;
+}
+
+// The ghost rules' transforms of a loaded cell of row m (kernel.cu:2549-2698,
+// 2328-2377): x_ghosts: the wave's band has ghost columns (wave-uniform).
+// Corner ghosts, read by no cell, may take both.
+AST_DEV void apply_ghost_rules(const ast_grid_t& g, Q& q, int n, int m, bool x_ghosts,
+                               double pulse) {
+  if (x_ghosts) {
+    auto side = [&](int k, bool here) {
+      const int bc = g.bc[k];  // wave-uniform
+      if (bc == AST_BC_DIRICHLET || bc == AST_BC_DIRICHLET_PULSED) {
+        const double r = bc == AST_BC_DIRICHLET_PULSED && pulsed_row(g, m)
+                             ? g.bc_state[k][0] * pulse : g.bc_state[k][0];
+        q.r = here ? r : q.r;
+        q.p = here ? g.bc_state[k][1] : q.p;
+        q.vx = here ? g.bc_state[k][2] : q.vx;
+        q.vy = here ? g.bc_state[k][3] : q.vy;
+      } else if (bc == AST_BC_REFLECT) {
+        q.vx = here ? -q.vx : q.vx;
+      } else if (bc == AST_BC_OUTFLOW_CLAMPED) {
+        const double c = g.bc_vclamp[k];
+        q.vx = here && (k == AST_XLO ? q.vx > c : q.vx < c) ? c : q.vx;
+      }
+    };
+    side(AST_XLO, n < 0);
+    side(AST_XHI, n >= g.N && n <= g.N + 1);
   }
-  return Q{a.x, a.y, b.x, b.y};
+  if (m < 0 || m >= g.M) {
+    const int k = m < 0 ? AST_YLO : AST_YHI, bc = g.bc[k];
+    if (bc == AST_BC_DIRICHLET || bc == AST_BC_DIRICHLET_PULSED) {
+      const double r = bc == AST_BC_DIRICHLET_PULSED && pulsed_row(g, m)
+                           ? g.bc_state[k][0] * pulse : g.bc_state[k][0];
+      q = Q{r, g.bc_state[k][1], g.bc_state[k][2], g.bc_state[k][3]};
+    } else if (bc == AST_BC_REFLECT) {
+      q.vy = -q.vy;
+    } else if (bc == AST_BC_OUTFLOW_CLAMPED) {
+      const double c = g.bc_vclamp[k];
+      if (k == AST_YLO ? q.vy > c : q.vy < c) q.vy = c;
+    }
+  }
+}
+
+// Can any cell of columns [n0, n1] x rows [m0, m1] lie in the frozen
+// ellipse?  (wave-uniform; with a margin, so that rounding cannot matter)
+AST_DEV bool frozen_possible(const ast_grid_t& g, int n0, int n1, int m0, int m1) {
+  if (!(g.frozen_ax > 0.0)) return false;
+  const double x0 = g.x_min + n0 * g.dx, x1 = g.x_min + n1 * g.dx;
+  const double y0 = g.y_min + m0 * g.dy, y1 = g.y_min + m1 * g.dy;
+  const double ax = g.frozen_ax * 1.01, ay = fabs(g.frozen_ay) * 1.01;
+  return x1 >= g.frozen_x0 - ax && x0 <= g.frozen_x0 + ax && y1 >= -ay && y0 <= ay;
 }
 
 // Exact-solver counters of one lane (the STATS kernels), ast_stats_t order.
@@ -201,7 +255,9 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
   __shared__ uint32_t redc[WPB * 10];
   const ast_grid_t& g = A.g;
   const G gas(A.gas);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  // wave index made explicitly uniform: rows and the loop stay scalar
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wg = xcd_tile(blockIdx.x, A.nwg);
   const int band = wg % A.nbands;
   const int m0 = ((wg / A.nbands) * WPB + wave) * A.rows;
@@ -217,65 +273,107 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
   // pulsed Dirichlet sides: the density factor at the time before the step
   const double pulse = A.TT != nullptr ? pulse_factor(g, *A.TT) : 1.0;
   const double kx = T_do / g.dx, ky = T_do / g.dy;
-  const bool frz = g.frozen_ax > 0.0;
+  const bool any_out = m0 < g.M;  // wave-uniform (every band holds columns)
   // frozen grid cells are copied (kernel.cu:2317-2324); a face votes for dt
   // when one of its cells is a grid cell that is not frozen (frozen cells
-  // return before their faces)
+  // return before their faces).  Without frozen cells that is every face of
+  // an output cell, so the lanes are masked once, after the rows.
+  const bool frz = any_out && frozen_possible(g, band * WOUT - 3, band * WOUT + 62, m0 - 1, m1);
   auto in_grid = [&](int nn, int mm) { return nn >= 0 && nn < g.N && mm >= 0 && mm < g.M; };
   auto frozen = [&](int nn, int mm) {
     return frz && in_grid(nn, mm) && is_frozen(g, g.x_min + nn * g.dx, g.y_min + mm * g.dy);
   };
-  auto voter = [&](int nn, int mm) { return in_grid(nn, mm) && !frozen(nn, mm); };
   double UUx = 0.0, UUy = 0.0;
   Counters cnt;
   if constexpr (STATS) cnt.clear();
 
-  if (m0 < g.M && band * WOUT < g.N) {  // wave-uniform
-    // prologue: rows m0-2 .. m0+2; the south face of row m0
-    const Q qa = load_q(g, A.s, A.u, n, m0 - 2, pulse);
-    const Q qb = load_q(g, A.s, A.u, n, m0 - 1, pulse);
-    Q q0 = load_q(g, A.s, A.u, n, m0, pulse);
-    Q q1 = load_q(g, A.s, A.u, n, m0 + 1, pulse);
-    Q q2 = load_q(g, A.s, A.u, n, m0 + 2, pulse);
-    Q d1 = q_sub(q1, q0);  // q(m+1) - q(m)
-    Q vn;                  // north face value of row m
-    FluxD Gs;              // flux through the south face of row m
+  if (any_out) {  // wave-uniform
+    const bool x_ghosts = band * WOUT < 2 || band * WOUT + 61 >= g.N;
+    const unsigned off = (unsigned)source_column(g, n);
+    const unsigned out_off = (unsigned)max(n, 0);
+    const int last = m1 + 1;  // the last row a fetch may name
+    auto fetch = [&](int m) {
+      const size_t row = (size_t)source_row(g, m) * g.N;
+      const double2 a = A.s[row + off], b = A.u[row + off];
+      return Q{a.x, a.y, b.x, b.y};
+    };
+    auto ghosts = [&](Q& q, int m) { apply_ghost_rules(g, q, n, m, x_ghosts, pulse); };
+    // prologue: rows m0-2 .. m0+1 and the fetch of m0+2; the south face of
+    // row m0.  w[k & 3] holds row m0 + k: the window slides by a change of
+    // names in the unrolled rows below
+    Q w[4], vn[2], dd[2];
+    FluxD Gf[2];
+    bool fr[2] = {false, false};
     {
-      const Q db = q_sub(q0, qb);
+      Q qa = fetch(m0 - 2), qb = fetch(m0 - 1);
+      w[0] = fetch(m0);
+      w[1] = fetch(m0 + 1);
+      w[2] = fetch(min(m0 + 2, last));
+      ghosts(qa, m0 - 2);
+      ghosts(qb, m0 - 1);
+      ghosts(w[0], m0);
+      ghosts(w[1], m0 + 1);
+      dd[0] = q_sub(w[1], w[0]);
+      const Q db = q_sub(w[0], qb);
       Q nb, sb, s0;
       face_values(qb, q_sub(qb, qa), db, nb, sb);
-      face_values(q0, db, d1, vn, s0);
+      face_values(w[0], db, dd[0], vn[0], s0);
       double uu;
       ExactInfo ei;
-      Gs = face<METHOD, WINDOW, false>(nb, s0, qb, q0, ho_y, gas, uu, ei);
-      if (out_col && (voter(n, m0 - 1) || voter(n, m0))) UUy = fmax(UUy, uu);
+      Gf[0] = face<METHOD, WINDOW, false>(nb, s0, qb, w[0], ho_y, gas, uu, ei);
+      if (frz) {
+        fr[0] = frozen(n, m0);
+        const bool vote = (in_grid(n, m0 - 1) && !frozen(n, m0 - 1)) || (in_grid(n, m0) && !fr[0]);
+        if (vote) UUy = fmax(UUy, uu);
+      } else {
+        UUy = fmax(UUy, uu);
+      }
       if constexpr (STATS) cnt.add(ei, out_col && m0 == 0);
     }
-    bool fr_m = frozen(n, m0);
-    for (int m = m0; m < m1; m++) {
-      const Q q3 = load_q(g, A.s, A.u, n, m + 3, pulse);  // for the next row
+    // -T_do/y of the r-source: row m0 + 64 j + k in lane k, read back per row
+    double tyl = 0.0;
+
+    auto row = [&](auto tag, int m) {
+      constexpr int J = decltype(tag)::value;
+      const Q& q0 = w[J & 3];
+      const Q& q1 = w[(J + 1) & 3];
+      Q& q2 = w[(J + 2) & 3];
+      ghosts(q2, min(m + 2, last));
+      w[(J + 3) & 3] = fetch(min(m + 3, last));  // for the next row
       // y: face values of row m+1; the north face of row m
       const Q d2 = q_sub(q2, q1);
       Q vn1, vs1;
-      face_values(q1, d1, d2, vn1, vs1);
+      face_values(q1, dd[J & 1], d2, vn1, vs1);
+      dd[(J + 1) & 1] = d2;
       double uuy;
       ExactInfo eiy;
-      const FluxD Gn = face<METHOD, WINDOW, false>(vn, vs1, q0, q1, ho_y, gas, uuy, eiy);
+      const FluxD Gn = face<METHOD, WINDOW, false>(vn[J & 1], vs1, q0, q1, ho_y, gas, uuy, eiy);
+      vn[(J + 1) & 1] = vn1;
+      const FluxD Gs = Gf[J & 1];
+      Gf[(J + 1) & 1] = Gn;
       // x: face values of row m; the west face (left value from lane - 1)
       const Q ql = from_left(q0);
-      const Q qr = from_right(q0);
+      const Q dl = q_sub(q0, ql);
       Q ve, vw;
-      face_values(q0, q_sub(q0, ql), q_sub(qr, q0), ve, vw);
+      face_values(q0, dl, from_right(dl), ve, vw);
       double uux;
       ExactInfo eix;
       const FluxD Fw = face<METHOD, WINDOW, true>(from_left(ve), vw, ql, q0, ho_x, gas, uux, eix);
       const FluxD Fe = from_right(Fw);
       // votes
-      const bool vote_here = voter(n, m);
-      const bool vote_up = voter(n, m + 1);
-      const bool vote_left = from_left(vote_here);
-      if (out_col && (vote_here || vote_up)) UUy = fmax(UUy, uuy);
-      if (west_face && (vote_here || vote_left)) UUx = fmax(UUx, uux);
+      const bool fr_m = fr[J & 1];
+      if (frz) {
+        const bool fr_up = frozen(n, m + 1);
+        const bool vote_here = in_grid(n, m) && !fr_m;
+        const bool vote_up = in_grid(n, m + 1) && !fr_up;
+        const bool vote_left = from_left(vote_here);
+        if (vote_here || vote_up) UUy = fmax(UUy, uuy);
+        if (vote_here || vote_left) UUx = fmax(UUx, uux);
+        fr[(J + 1) & 1] = fr_up;
+      } else {
+        UUy = fmax(UUy, uuy);
+        UUx = fmax(UUx, uux);
+      }
       if constexpr (STATS) {
         cnt.add(eiy, out_col);
         cnt.add(eix, west_face);
@@ -290,17 +388,21 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
       const double mx = q0.r * q0.vx, my = q0.r * q0.vy;
       if constexpr (GEOM == AST_AXISYMMETRIC) {
         // KorolkovSolver.cu:13-32: -(T_do/y) v {rho, rho u, rho v, gamma p/(g-1) + KE}
-        const double ty = T_do / (g.y_min + m * g.dy);
+        const int k = (m - m0) & 63;
+        if (k == 0) tyl = div64(T_do, g.y_min + (m + lane) * g.dy);
+        const double ty = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(tyl), k),
+                                           __builtin_amdgcn_readlane(__double2loint(tyl), k));
         const double tr = ty * my;
         dr -= tr;
         dmx -= tr * q0.vx;
         dmy -= tr * q0.vy;
         dE -= ty * q0.vy * (gas.g * gas.ig1 * q0.p + ke);
       }
+      const size_t rowk = (size_t)m * g.N;
       if (A.nn2 != nullptr || A.nn3 != nullptr) {  // wave-uniform
         // neutral-H sources (kernel.cu:2495-2498): momentum T_do (rho kmom)
         // nn2.{x,y}, energy T_do ken nn3; output cells only (in bounds)
-        const size_t k = out_col ? (size_t)m * g.N + n : 0;
+        const size_t k = out_col ? rowk + out_off : 0;
         if (A.nn2 != nullptr) {
           const double tk = T_do * (q0.r * A.kmom);
           dmx += tk * (out_col ? A.nn2[3 * k] : 0.0);
@@ -313,37 +415,52 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
       const bool rfloor = q0.r + dr <= 0.0;
       const double drf = rfloor ? 0.0 : dr;
       const double r2 = q0.r + drf;
-      const double vx2 = (mx + dmx) / r2;
-      const double vy2 = (my + dmy) / r2;
+      const double ir2 = rcp64(r2);  // shared by the three quotients
+      const double vx2 = div64(mx + dmx, r2, ir2);
+      const double vy2 = div64(my + dmy, r2, ir2);
       // p' = (E' - rho'|u'|^2/2)(g-1) with the O(E) terms cancelled exactly:
       // KE' - KE = (m.dm + |dm|^2/2 - KE dr)/rho'
-      const double dke = (mx * dmx + my * dmy + 0.5 * (dmx * dmx + dmy * dmy) - ke * drf) / r2;
+      const double dke =
+          div64(mx * dmx + my * dmy + 0.5 * (dmx * dmx + dmy * dmy) - ke * drf, r2, ir2);
       double p2 = q0.p + gas.g1 * (dE - dke);
       if (p2 <= 0.0) p2 = 0.000001;  // kernel.cu:3070-3073
       if (out_col) {
-        const size_t k = (size_t)m * g.N + n;
-        if (fr_m) {  // frozen: copied (kernel.cu:2317-2324)
-          A.s2[k] = make_double2(q0.r, q0.p);
-          A.u2[k] = make_double2(q0.vx, q0.vy);
-        } else {
-          A.s2[k] = make_double2(r2, p2);
-          A.u2[k] = make_double2(vx2, vy2);
+        double2 so = make_double2(r2, p2), uo = make_double2(vx2, vy2);
+        if (frz && fr_m) {  // frozen: copied (kernel.cu:2317-2324)
+          so = make_double2(q0.r, q0.p);
+          uo = make_double2(q0.vx, q0.vy);
         }
+        A.s2[rowk + out_off] = so;
+        A.u2[rowk + out_off] = uo;
       }
-      // slide the window one row
-      fr_m = frozen(n, m + 1);
-      Gs = Gn;
-      vn = vn1;
-      d1 = d2;
-      q0 = q1;
-      q1 = q2;
-      q2 = q3;
+    };
+    // four rows a trip, so that the window slides by names; the exact solver
+    // (two inlined solvers a row, ~40 KB of code) takes one row a trip and
+    // moves the window
+    if constexpr (METHOD == AST_EXACT) {
+      for (int m = m0; m < m1; m++) {
+        row(std::integral_constant<int, 0>{}, m);
+        for (int k = 0; k < 3; k++) w[k] = w[k + 1];
+        vn[0] = vn[1];
+        dd[0] = dd[1];
+        Gf[0] = Gf[1];
+        fr[0] = fr[1];
+      }
+    } else {
+      for (int m = m0; m < m1; m += 4) {
+        row(std::integral_constant<int, 0>{}, m);
+        if (m + 1 >= m1) break;
+        row(std::integral_constant<int, 1>{}, m + 1);
+        if (m + 2 >= m1) break;
+        row(std::integral_constant<int, 2>{}, m + 2);
+        if (m + 3 >= m1) break;
+        row(std::integral_constant<int, 3>{}, m + 3);
+      }
     }
   }
   // per-face dt = krit*rad/UU (monotone in UU), capped at 1000 (kernel.cu:2530)
-  UUx = wave_max(UUx);
-  UUy = wave_max(UUy);
-  const bool any_out = m0 < g.M && band * WOUT < g.N;
+  UUx = wave_max(west_face ? UUx : 0.0);
+  UUy = wave_max(out_col ? UUy : 0.0);
   double tmin = any_out ? 1000.0 : INFINITY;
   if (UUx > 0.0) tmin = fmin(tmin, g.krit * g.dx / UUx);
   if (UUy > 0.0) tmin = fmin(tmin, g.krit * g.dy / UUy);
@@ -351,8 +468,48 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
   if constexpr (STATS) block_counters_to(cnt, redc, A.stats);
 }
 
-// rows per strip of the FP64 step (ast_step_f64_rows)
-constexpr int kDefaultRows = 6;
+// The default rows per strip (ast_step_f64_rows, rows = 0).  A wave's row is
+// one chain of dependent FP64 operations: 1.4 us a row for a wave alone on
+// its SIMD, 1.07 us of a SIMD's time from two waves on (HLLC); a strip costs
+// about 1.5 rows more than it holds (its south face, the first fetches).  So
+// small grids want one-row strips, which spread the chains over the chip,
+// and large ones taller strips in whole rounds of the 3 x 1024 waves that
+// are resident.  The rule takes the height with the least (rows + 1.5) x n,
+// n the load of a SIMD in waves fitted to the measured times: 1.3 / 2.15 /
+// 2.8 where one, two or three waves a SIMD all run at once, beyond that 0.8
+// of the mean count plus 0.4 and 0.6 of what the last round leaves empty.
+// Measured, us a step (HLLC; rows of the rule / the fixed 6 rows before):
+// 256x128 8.0 (1) / 14.7, 512x256 11.1 (3) / 15.2, 1024x512 19.5 (5) / 21.5,
+// 1500x750 29.7 (10) / 33.5, 2048x1024 45.7 (6), 4096x2048 148.4 (16) / 162.3.
+// The exact solver's rows differ by tens of times between waves (its
+// patterns and iterations diverge), so its strips stay short until 16384 of
+// them share the load: 256x128 26.0 (1) / 95.7, 1500x750 56.6 (2) / 106.4,
+// 2048x1024 82.1 (3) / 109.1, 4096x2048 about 243 (9) / 246.5.
+static int default_rows(const ast_grid_t& g, int method) {
+  const long long nbands = (g.N + WOUT - 1) / WOUT;
+  if (method == AST_EXACT) {
+    const long long rows = (nbands * g.M + 16383) / 16384;
+    return (int)std::min(rows, 32LL);
+  }
+  int best = 1;
+  double cost = INFINITY;
+  for (int rows = 1; rows <= 32; rows++) {
+    const long long strips = (g.M + rows - 1) / rows;
+    const double waves = (double)(nbands * ((strips + WPB - 1) / WPB) * WPB);
+    const double per = waves / 1024.0;
+    const double rounds = waves / 3072.0;
+    const double n = per <= 1.0   ? 1.3
+                     : per <= 2.0 ? 2.15
+                     : per <= 3.0 ? 2.8
+                                  : 0.8 * per + 0.4 + 0.6 * (ceil(rounds) - rounds);
+    const double c = n * (rows + 1.5);
+    if (c < cost) {
+      cost = c;
+      best = rows;
+    }
+  }
+  return best;
+}
 
 template <int METHOD, int GEOM, bool WINDOW>
 static int launch3(const StepArgs& a, bool stats, hipStream_t st) {
@@ -395,7 +552,7 @@ int ast_step_f64_rows(const ast_grid_t* g, const double* s, const double* u, dou
     return ast_fail(AST_ERR_ARG, "ast_step_f64: null state or time pointer");
   if (s == s2 || u == u2 || s == u2 || u == s2)
     return ast_fail(AST_ERR_ARG, "ast_step_f64: output planes must not alias the input planes");
-  if (rows == 0) rows = kDefaultRows;
+  if (rows == 0) rows = default_rows(*g, method);
   if (rows < 1 || rows > 4096) return ast_fail(AST_ERR_ARG, "ast_step_f64: %d rows per strip", rows);
   StepArgs a;
   a.g = *g;

@@ -415,11 +415,11 @@ int ast_sim_set_learned_mode(ast_sim_t* sim, int mode);
 /* Strip tiling of the step.  FP32: rows > 0 rows per wave strip, rows = -S
  * S strips of (nearly) equal height per band of 60 columns; strips of 4 to
  * 64 rows inside the grid take the fast strip path.  FP64: rows > 0 rows
- * per wave strip (default 6). */
+ * per wave strip (default: chosen from the grid's size and the method). */
 int ast_sim_set_tile_rows(ast_sim_t* sim, int rows);
 /* Times the step for each candidate tiling (NULL = a default list: FP32 4,
  * 8, 12, 16 rows and the tilings -S that give every SIMD 2, 3, 4 or 5 equal
- * waves; FP64 4, 6, 8, 12, 16, 32 rows), keeps the fastest; reports it (may
+ * waves; FP64 1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32 rows), keeps the fastest; reports it (may
  * be NULL).  State and time are left unchanged. */
 int ast_sim_autotune(ast_sim_t* sim, const int* candidates, int ncand, int reps,
                      int* best_rows, float* best_us);
