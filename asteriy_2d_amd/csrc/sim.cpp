@@ -7,9 +7,9 @@
 // (ping-pong A->B->A...) is captured once into a HIP graph on the
 // simulation's own stream and replayed; dt never leaves the device (T, T_do,
 // TT, i live in one device block, as in kernel.cu:3290-3293).  State is held
-// in FP64 (the reference layout: each step is Kernel_TVD + funk_time) or FP32
-// planes (each step is one kernel that also performs the previous step's time
-// advance, time_slots.h; one small kernel closes the run).
+// in FP64 (the reference layout) or FP32 planes; each step is one kernel that
+// also performs the previous step's time advance (time_slots.h), and one
+// small kernel closes the run.
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -33,7 +33,8 @@ int ast_step_f32_rows(const ast_grid_t* g, const float* s, const float* u, float
 int ast_funk_time_fold(double* T, int last, int nslots, uint32_t* flags, void* stream);
 int ast_step_f64_rows(const ast_grid_t* g, const double* s, const double* u, double* s2,
                       double* u2, double* T, const double* T_do, const double* TT, int method,
-                      ast_stats_t* stats, int rows, const ast_sources_t* src, void* stream);
+                      ast_stats_t* stats, int rows, const ast::StepTime* tm,
+                      const ast_sources_t* src, void* stream);
 extern "C" int ast_get_tile_rows(void);
 
 #define CK(call)                                              \
@@ -52,7 +53,7 @@ struct ast_sim {
   void* plane[4];  // s0, u0, s1, u1
   int cur;         // 0: state in (s0,u0); 1: in (s1,u1)
   double* scal;    // time block: T, T_do, TT (+ int i in the 4th word), then
-                   // the FP32 step's dt slots (time_slots.h)
+                   // the steps' dt slots (time_slots.h)
   ast_stats_t* stats;
   bool collect;  // count the exact solver's work into stats (counting kernels)
   const ast_mlp_t* mlp;
@@ -125,10 +126,10 @@ static ast::StepTime step_time(ast_sim_t* S, int j, int mode) {
   return tm;
 }
 
-// n steps from plane `from`.  FP32: step j lowers slot set j (mod 3), takes
-// its dt from set j-1 and advances the time; a fold of the last set closes
-// the run, so between runs the time block reads as after funk_time.  mode:
-// the run kind in the learned mode (-1: not in it).
+// n steps from plane `from`: step j lowers slot set j (mod 3), takes its dt
+// from set j-1 and advances the time; a fold of the last set closes the run,
+// so between runs the time block reads as after funk_time.  mode: the run
+// kind in the learned mode (-1: not in it).
 static int launch_steps(ast_sim_t* S, int from, int n, int mode) {
   double* T = S->scal;
   for (int j = 0; j < n; j++) {
@@ -138,14 +139,13 @@ static int launch_steps(ast_sim_t* S, int from, int n, int mode) {
     void* s2 = S->plane[2 * (1 - f)];
     void* u2 = S->plane[2 * (1 - f) + 1];
     int rc;
+    const ast::StepTime tm = step_time(S, j, mode);
     if (S->precision == 0) {
       rc = ast_step_f64_rows(&S->g, (const double*)s, (const double*)u, (double*)s2,
                              (double*)u2, T, T + 1, T + 2, S->method,
                              S->collect ? S->stats : nullptr,
-                             S->rows64, sources64(S), S->stream);
-      if (rc == AST_OK) rc = ast_funk_time(T, T + 1, T + 2, (int*)(T + 3), S->stream);
+                             S->rows64, &tm, sources64(S), S->stream);
     } else {
-      const ast::StepTime tm = step_time(S, j, mode);
       rc = ast_step_f32_rows(&S->g, (const float*)s, (const float*)u, (float*)s2, (float*)u2, T,
                              T + 1, T + 2, S->method, mode == kRunQuiet ? nullptr : S->mlp,
                              S->collect ? S->stats : nullptr, S->krows, &tm, sources32(S),
@@ -153,7 +153,7 @@ static int launch_steps(ast_sim_t* S, int from, int n, int mode) {
     }
     if (rc != AST_OK) return rc;
   }
-  if (S->precision == 1 && n > 0)
+  if (n > 0)
     return ast_funk_time_fold(T, n - 1, ast::kMaxSlots, mode >= 0 ? S->dflags : nullptr,
                               S->stream);
   return AST_OK;
@@ -483,7 +483,7 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
                                    sources32(S), S->stream)
                : ast_step_f64_rows(&S->g, (const double*)sp, (const double*)up, (double*)s2,
                                    (double*)u2, S->scal, S->scal + 1, S->scal + 2, S->method,
-                                   nullptr, kr, sources64(S), S->stream);
+                                   nullptr, kr, &tm, sources64(S), S->stream);
   };
   auto valid = [&](int kr) {
     if (S->precision == 0) return kr >= 1 && kr <= 4096;
