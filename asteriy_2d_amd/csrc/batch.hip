@@ -41,7 +41,7 @@ AST_DEV void batch_item(const BatchInst& I, int local, int from, double* red) {
   strip_rows(I.g.M, I.nbands, I.krows, local, wave, band, m0, m1);
   const double tmin = strip_of_wave<METHOD, GEOM, false>(
       I.g, I.c, I.ex, I.plane[2 * from], I.plane[2 * from + 1], I.plane[2 * (1 - from)],
-      I.plane[2 * (1 - from) + 1], I.scal[1], band, m0, m1, st);
+      I.plane[2 * (1 - from) + 1], [&]() { return I.scal[1]; }, band, m0, m1, st);
   block_min_uniform<NT>(tmin, red, I.scal, 0);
 }
 

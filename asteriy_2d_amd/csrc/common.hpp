@@ -118,15 +118,35 @@ AST_DEV bool is_frozen(const ast_grid_t& g, double x, double y) {
 AST_DEV bool high_order(const ast_grid_t& g, double xf) { return xf > g.ho_lo && xf < g.ho_hi; }
 
 // ---- wave64 / block reductions ------------------------------------------
+
+// v of the lane DPP control CTRL names, in the rows of ROWS (a lane without
+// a source, or in another row, keeps its own).
+template <int CTRL, int ROWS>
+AST_DEV double dpp64(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false),
+                          __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false));
+}
+// The minimum / maximum over the wave, wave-uniform (every lane active): row
+// shifts by 1, 2, 4, 8 leave each row's result in its lane 15, row_bcast:15
+// and :31 carry them to lane 63.  Six register moves in place of six rounds
+// through the LDS permute.
+template <class F>
+AST_DEV double wave_reduce(double v, F f) {
+  v = f(v, dpp64<0x111, 0xf>(v));
+  v = f(v, dpp64<0x112, 0xf>(v));
+  v = f(v, dpp64<0x114, 0xf>(v));
+  v = f(v, dpp64<0x118, 0xf>(v));
+  v = f(v, dpp64<0x142, 0xa>(v));
+  v = f(v, dpp64<0x143, 0xc>(v));
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
 AST_DEV double wave_min(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-  return v;
+  return wave_reduce(v, [](double a, double b) { return fmin(a, b); });
 }
 AST_DEV double wave_max(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-  return v;
+  return wave_reduce(v, [](double a, double b) { return fmax(a, b); });
 }
 AST_DEV uint32_t wave_sum(uint32_t v) {
 #pragma unroll
@@ -184,17 +204,22 @@ struct KTime {
   int nslots;
 };
 
-// dt of this step, in two parts.  step_dt_load (loads only): with a previous
-// slot set, dt is the minimum of its slots (every wave folds them itself: no
-// workgroup waits for another), else *T_do.  step_dt_commit (the writes):
-// with a previous set, wave 0 of workgroup 0 performs the previous step's
+// dt of this step, in three parts.  With a previous slot set dt is the
+// minimum of its slots (every wave folds them itself: no workgroup waits for
+// another), else *T_do: step_dt_load issues the loads, step_dt_fold takes
+// the minimum, where the kernel first needs it, so that the strip's own
+// first loads are under way meanwhile.  step_dt_commit (the writes): with a
+// previous set, wave 0 of workgroup 0 performs the previous step's
 // time advance, funk_time of kernel.cu:1525-1536 (T_do = that minimum,
 // TT += T_do, i += 1; T stays at its reset value); it clears the set `rst`
 // for the step after.
 AST_DEV double step_dt_load(const double* T_do, const KTime& kt) {
   const int lane = threadIdx.x & 63;
-  if (kt.prev != nullptr) return wave_min(lane < kt.nslots ? kt.prev[kSlotStride * lane] : INFINITY);
+  if (kt.prev != nullptr) return lane < kt.nslots ? kt.prev[kSlotStride * lane] : INFINITY;
   return *T_do;
+}
+AST_DEV double step_dt_fold(const KTime& kt, double loaded) {
+  return kt.prev != nullptr ? wave_min(loaded) : loaded;
 }
 AST_DEV void step_dt_commit(double* T, const KTime& kt, double t) {
   const int lane = threadIdx.x & 63;

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(NT) void step_kernel(ast_grid_t g, Consts c, ExactC
                                                   int nwg, SrcF src, const double* TT) {
   __shared__ double red[WPB];
   __shared__ uint32_t redi[WPB * 10];
-  const double tdo = step_dt_load(T_do, kt);
+  const double dt_loaded = step_dt_load(T_do, kt);
   // pulsed Dirichlet sides: the density factor at the time the reference's
   // step reads (TT after the previous step's funk_time).  With the runtime's
   // slots (kt), workgroup 0 advances T[2] during this step, so the step
@@ -73,14 +73,18 @@ __global__ __launch_bounds__(NT) void step_kernel(ast_grid_t g, Consts c, ExactC
   if (c.pulsed) {  // wave-uniform
     double tt;
     if (kt.cur != nullptr) {
-      tt = kt.prev != nullptr ? kt.prev[2] + tdo : T[2];
+      tt = kt.prev != nullptr ? kt.prev[2] + step_dt_fold(kt, dt_loaded) : T[2];
       if (blockIdx.x == 0 && threadIdx.x == 0) kt.cur[2] = tt;
     } else {
       tt = *TT;
     }
     pulse = pulse_factor(g, tt);
   }
-  step_dt_commit(T, kt, tdo);
+  auto dt = [&]() {  // (wave 0 of workgroup 0, which commits, has rows)
+    const double tdo = step_dt_fold(kt, dt_loaded);
+    step_dt_commit(T, kt, tdo);
+    return tdo;
+  };
   constexpr bool kDetects = METHOD == kExactLearned || METHOD == kExactDetect;
   typename std::conditional<STATS, StatsF32,
                             typename std::conditional<kDetects, StrongStats, NoStats>::type>::type st;
@@ -90,7 +94,7 @@ __global__ __launch_bounds__(NT) void step_kernel(ast_grid_t g, Consts c, ExactC
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int band, m0, m1;
   strip_rows(g.M, nbands, krows, xcd_tile(blockIdx.x, nwg), wave, band, m0, m1);
-  tmin = strip_of_wave<METHOD, GEOM, WINDOW, SRC, PULSE>(g, c, ex, s, u, s2, u2, tdo, band, m0,
+  tmin = strip_of_wave<METHOD, GEOM, WINDOW, SRC, PULSE>(g, c, ex, s, u, s2, u2, dt, band, m0,
                                                          m1, st, src, pulse);
   if (ex.strong != nullptr && st.any_strong() && (threadIdx.x & 63) == 0) atomicOr(ex.strong, 1u);
   if constexpr (STATS) block_stats_f32_to<NT>(st, redi, stats);

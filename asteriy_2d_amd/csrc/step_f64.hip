@@ -35,7 +35,8 @@
 // runtime spreads these atomics over 64 slots and lets the next step fold
 // them and advance the time (time_slots.h), so that a step is one kernel:
 // funk_time as a kernel of its own took 4.8 us of a step
-// (Sod 256x128: 13.0 -> 10.4 us a step, 2048x1024 HLLC 51.3 -> 50.5).
+// (Sod 256x128: 13.0 -> 9.5 us a step, 2048x1024 HLLC 51.3 -> 49.0,
+// both with the fold under the first rows' loads).
 #include <algorithm>
 #include <type_traits>
 
@@ -274,7 +275,7 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
   const double x = g.x_min + n * g.dx;
   const bool ho_x = high_order(g, x - g.dx / 2.0);  // west face (kernel.cu:2843)
   const bool ho_y = high_order(g, x);               // y faces: the cell x (kernel.cu:2816)
-  const double T_do = step_dt_load(A.T_do, A.kt);
+  const double dt_loaded = step_dt_load(A.T_do, A.kt);
   // pulsed Dirichlet sides: the density factor at the time before the step.
   // With the runtime's slots workgroup 0 advances TT during this step, so
   // the step takes the time the previous step of its run used (word 2 of
@@ -282,12 +283,10 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
   // records its own; the first step of a run reads TT.
   double pulse = 1.0;
   if (A.TT != nullptr) {  // wave-uniform
-    const double tt = A.kt.prev != nullptr ? A.kt.prev[2] + T_do : *A.TT;
+    const double tt = A.kt.prev != nullptr ? A.kt.prev[2] + step_dt_fold(A.kt, dt_loaded) : *A.TT;
     if (A.kt.cur != nullptr && blockIdx.x == 0 && threadIdx.x == 0) A.kt.cur[2] = tt;
     pulse = pulse_factor(g, tt);
   }
-  step_dt_commit(A.T, A.kt, T_do);
-  const double kx = T_do / g.dx, ky = T_do / g.dy;
   const bool any_out = m0 < g.M;  // wave-uniform (every band holds columns)
   // frozen grid cells are copied (kernel.cu:2317-2324); a face votes for dt
   // when one of its cells is a grid cell that is not frozen (frozen cells
@@ -319,11 +318,15 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
     Q w[4], vn[2], dd[2];
     FluxD Gf[2];
     bool fr[2] = {false, false};
+    double T_do;
     {
       Q qa = fetch(m0 - 2), qb = fetch(m0 - 1);
       w[0] = fetch(m0);
       w[1] = fetch(m0 + 1);
       w[2] = fetch(min(m0 + 2, last));
+      __builtin_amdgcn_sched_barrier(0);  // the fetches go out before the dt fold waits
+      T_do = step_dt_fold(A.kt, dt_loaded);
+      step_dt_commit(A.T, A.kt, T_do);  // (by wave 0 of workgroup 0, which has rows)
       ghosts(qa, m0 - 2);
       ghosts(qb, m0 - 1);
       ghosts(w[0], m0);
@@ -345,7 +348,8 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
       }
       if constexpr (STATS) cnt.add(ei, out_col && m0 == 0);
     }
-    // -T_do/y of the r-source: row m0 + 64 j + k in lane k, read back per row
+    const double kx = div64(T_do, g.dx), ky = div64(T_do, g.dy);
+    // T_do/y of the r-source: row m0 + 64 j + k in lane k, read back per row
     double tyl = 0.0;
 
     auto row = [&](auto tag, int m) {

@@ -358,8 +358,7 @@ struct StripArgs {
   bool yrefl[2], ydir[2];
   float ysign[2], ylo[2], yhi[2];
   float yq[2][4];
-  float ax, ay;   // -T_do/dx, -T_do/dy
-  float tdof, dxf, dyf, x, ymin;
+  float dxf, dyf, x, ymin;
   unsigned col_off;  // byte offset of the lane's column in a row (interior strips)
   unsigned st_off;   // the same for the stores, kOffDrop on lanes that write nothing
   unsigned row_bytes;
@@ -421,11 +420,15 @@ struct PulsePatch {
   }
 };
 
-template <int METHOD, int GEOM, bool WINDOW, int PATH, int SRC, class ST, class PF = NoPulse>
+//
+// dt() gives T_do, after the first rows' loads are issued (its own loads and
+// the fold of the slots then pass under theirs).
+template <int METHOD, int GEOM, bool WINDOW, int PATH, int SRC, class ST, class DT,
+          class PF = NoPulse>
 AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, const ExactCtx& ex,
                        const float2* __restrict__ s, const float2* __restrict__ u,
                        float2* __restrict__ s2, float2* __restrict__ u2, const StripArgs& a,
-                       float& UUx, float& UUy, ST& st, const PF& pf = PF{}) {
+                       float& UUx, float& UUy, ST& st, const DT& dt, const PF& pf = PF{}) {
   constexpr bool FAST = PATH != kEdge;
   const int n = a.n, m0 = a.m0, m1 = a.m1, N = g.N, M = g.M;
   const unsigned rb = a.row_bytes;
@@ -485,11 +488,17 @@ AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, c
   Q w[4], nv[2], dd[2];
   FaceF G[2];
   bool fr[2] = {false, false};
+  float tdof, tax, tay;  // T_do, -T_do/dx, -T_do/dy
   {
     const Q qa = pf(LD(m0 - 2), m0 - 2), qb = pf(LD(m0 - 1), m0 - 1);
     w[0] = pf(LD(m0), m0);
     w[1] = pf(LD(m0 + 1), m0 + 1);
     w[2] = pf(LD(m0 + 2), m0 + 2);
+    if constexpr (FAST) __builtin_amdgcn_sched_barrier(0);
+    const double tdo = dt();
+    tdof = (float)tdo;
+    tax = (float)(-tdo / g.dx);
+    tay = (float)(-tdo / g.dy);
     const Q d0 = sub(qb, qa), d1 = sub(w[0], qb);
     dd[0] = sub(w[1], w[0]);
     Q nvm1, svm1, sv0;
@@ -516,7 +525,7 @@ AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, c
   // an fma, a reciprocal and a product
   float tyl = 0.f;
   if constexpr (FAST && GEOM == AST_AXISYMMETRIC)
-    tyl = a.tdof * frcp(a.ymin + (m0 + (int)(threadIdx.x & 63)) * a.dyf);
+    tyl = tdof * frcp(a.ymin + (m0 + (int)(threadIdx.x & 63)) * a.dyf);
   Q pend = w[0];
   unsigned pend_vo = kOffDrop;
   // source planes: row m's values are fetched with row m-1's state fetch,
@@ -589,10 +598,10 @@ AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, c
     const CellFlux cW = in_cell_frame<ST1>(Fw, q0.vx, q0.vy);
     const CellFlux cN = in_cell_frame<ST1>(Gn, q0.vy, q0.vx);
     const CellFlux cS = in_cell_frame<ST1>(Gs, q0.vy, q0.vx);
-    float dr_ = a.ax * (Fe.m - Fw.m) + a.ay * (Gn.m - Gs.m);
-    float de = a.ax * (cE.e - cW.e) + a.ay * (cN.e - cS.e);
-    float d1x = a.ax * (cE.n - cW.n) + a.ay * (cN.t - cS.t);
-    float d1y = a.ax * (cE.t - cW.t) + a.ay * (cN.n - cS.n);
+    float dr_ = tax * (Fe.m - Fw.m) + tay * (Gn.m - Gs.m);
+    float de = tax * (cE.e - cW.e) + tay * (cN.e - cS.e);
+    float d1x = tax * (cE.n - cW.n) + tay * (cN.t - cS.t);
+    float d1y = tax * (cE.t - cW.t) + tay * (cN.n - cS.n);
     G[R::e1] = Gn;
     if constexpr (GEOM == AST_AXISYMMETRIC) {
       // KorolkovSolver.cu:13-32: -(T_do/y) v {rho, rho u, rho v, E + p}; in
@@ -600,7 +609,7 @@ AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, c
       // -(T_do/y) v (rho e + p) = -(T_do/y) v gamma p/(gamma-1)
       float ty;
       if constexpr (FAST) ty = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tyl), m - m0));
-      else ty = a.tdof * frcp(y);
+      else ty = tdof * frcp(y);
       const float f = ty * q0.vy;
       dr_ = fmaf(-f, q0.r, dr_);
       de = fmaf(-f, c.gig1 * q0.p, de);
@@ -609,10 +618,10 @@ AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, c
       // add_MK's neutral-hydrogen terms (kernel.cu:2495-2498), before the
       // floors: momentum T_do (rho kmom) nn2.{x, y}, energy T_do ken nn3;
       // seen from the cell the energy change loses u.(the momentum change)
-      const float tk = a.tdof * (q0.r * a.src.kmom);
+      const float tk = tdof * (q0.r * a.src.kmom);
       const float mx = tk * (float)scur.x;
       const float my = tk * (float)scur.y;
-      const float se = (a.tdof * a.src.ken) * (float)scur.e;
+      const float se = (tdof * a.src.ken) * (float)scur.e;
       scur = snext;
       d1x += mx;
       d1y += my;
@@ -689,10 +698,20 @@ AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, c
   bstore(pend.vx, pend.vy, wu, pend_vo, 0);
 }
 
+// the wave's maximum, wave-uniform (every lane active; wave_reduce's scheme)
+template <int CTRL, int ROWS>
+AST_DEV float max_dpp(float v) {
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(
+                      __float_as_int(v), __float_as_int(v), CTRL, ROWS, 0xf, false)));
+}
 AST_DEV float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
+  v = max_dpp<0x111, 0xf>(v);
+  v = max_dpp<0x112, 0xf>(v);
+  v = max_dpp<0x114, 0xf>(v);
+  v = max_dpp<0x118, 0xf>(v);
+  v = max_dpp<0x142, 0xa>(v);
+  v = max_dpp<0x143, 0xc>(v);
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
 // The band and rows [m0, m1) of wave `wave` of workgroup `wg` under a strip
@@ -734,10 +753,11 @@ AST_DEV void strip_rows(int M, int nbands, int tile, int wg, int wave, int& band
 // The strip of one wave given its band and rows (strip_rows): fills
 // StripArgs and runs the fast or the boundary variant.  Returns the wave's
 // dt candidate (wave-uniform).
-template <int METHOD, int GEOM, bool WINDOW, int SRC = kSrcNone, bool PULSE = false, class ST>
+template <int METHOD, int GEOM, bool WINDOW, int SRC = kSrcNone, bool PULSE = false, class ST,
+          class DT>
 AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCtx& ex,
                              const float2* __restrict__ s, const float2* __restrict__ u,
-                             float2* __restrict__ s2, float2* __restrict__ u2, double tdo,
+                             float2* __restrict__ s2, float2* __restrict__ u2, const DT& dt,
                              int band, int m0, int m1, ST& st,
                              const SrcF& src = SrcF{nullptr, nullptr, nullptr, nullptr, 0.f, 0.f},
                              double pulse = 1.0) {
@@ -750,9 +770,6 @@ AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCt
   a.cols_in = (band * WOUT - 2 >= 0) && (band * WOUT + 61 < g.N);  // wave-uniform
   a.out_col = (lane >= 2) & (lane < 2 + WOUT) & (a.n < g.N);
   a.xvote = (lane >= 2) & (lane <= 2 + WOUT) & (a.n <= g.N);
-  a.ax = (float)(-tdo / g.dx);
-  a.ay = (float)(-tdo / g.dy);
-  a.tdof = (float)tdo;
   a.dxf = (float)g.dx;
   a.dyf = (float)g.dy;
   a.x = (float)(g.x_min + a.n * g.dx);
@@ -813,9 +830,9 @@ AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCt
       a.gdir = a.gdir || gbc == AST_BC_DIRICHLET_PULSED;
       if (fast_rows && rows_in && !cw.frozen) {
         if (a.cols_in)
-          run_strip<METHOD, GEOM, WINDOW, kFast, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st);
+          run_strip<METHOD, GEOM, WINDOW, kFast, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt);
         else
-          run_strip<METHOD, GEOM, WINDOW, kFastX, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st,
+          run_strip<METHOD, GEOM, WINDOW, kFastX, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt,
                                                        pp);
       } else if (fast_rows && ((a.m1 - a.m0) & 3) == 0) {
         for (int k = 0; k < 2; k++) {
@@ -829,10 +846,10 @@ AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCt
           a.yhi[k] = (ybc == AST_BC_OUTFLOW_CLAMPED && k == 0) ? yc : 3.40282347e38f;
           for (int j = 0; j < 4; j++) a.yq[k][j] = (float)g.bc_state[ys][j];
         }
-        run_strip<METHOD, GEOM, WINDOW, kFastE, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st,
+        run_strip<METHOD, GEOM, WINDOW, kFastE, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt,
                                                      pp);
       } else {
-        run_strip<METHOD, GEOM, WINDOW, kEdge, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st);
+        run_strip<METHOD, GEOM, WINDOW, kEdge, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt);
       }
     } else {
       // kernels without the PULSE variants (the exact solver's): strips
@@ -844,9 +861,9 @@ AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCt
                                        g.bc[AST_YHI] == AST_BC_DIRICHLET_PULSED);
       if (fast_rows && rows_in && !cw.frozen && !xpulse) {
         if (a.cols_in)
-          run_strip<METHOD, GEOM, WINDOW, kFast, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st);
+          run_strip<METHOD, GEOM, WINDOW, kFast, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt);
         else
-          run_strip<METHOD, GEOM, WINDOW, kFastX, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st);
+          run_strip<METHOD, GEOM, WINDOW, kFastX, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt);
       } else if (fast_rows && ((a.m1 - a.m0) & 3) == 0 && !xpulse && !ypulse) {
         // the y-ghost rules of fetch_cell as row rules (only the first or last
         // strips of a band hold ghost rows)
@@ -861,9 +878,9 @@ AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCt
           a.yhi[k] = (ybc == AST_BC_OUTFLOW_CLAMPED && k == 0) ? yc : 3.40282347e38f;
           for (int j = 0; j < 4; j++) a.yq[k][j] = (float)g.bc_state[ys][j];
         }
-        run_strip<METHOD, GEOM, WINDOW, kFastE, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st);
+        run_strip<METHOD, GEOM, WINDOW, kFastE, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt);
       } else {
-        run_strip<METHOD, GEOM, WINDOW, kEdge, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st);
+        run_strip<METHOD, GEOM, WINDOW, kEdge, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt);
       }
     }
   }
