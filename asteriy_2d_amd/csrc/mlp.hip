@@ -7,10 +7,9 @@
 //  * forward: FP32 masters on the vector ALU (one sample per lane), or the
 //    BF16 MFMA path (one 64-sample tile per wave, mlp.hpp).
 //  * loss + gradient: mean squared error over the masked rows, forward and
-//    backward per lane in FP32, per-workgroup weight gradients reduced
-//    through LDS, per-workgroup partials summed in a fixed order by a second
-//    kernel (deterministic).
-//  * Adam on the FP32 masters, then the BF16 MFMA operands are rebuilt.
+//    backward on FP32 MFMA, per-workgroup partials summed in a fixed order by
+//    a second kernel (deterministic).
+//  * Adam on the FP32 masters, the BF16 MFMA operands rebuilt with it.
 #include "common.hpp"
 #include "flux64.hpp"
 #include "mlp.hpp"
@@ -85,214 +84,361 @@ __global__ void forward_bf16_kernel(const unsigned char* __restrict__ buf, size_
 }
 
 // ---- loss and gradient -----------------------------------------------------
-constexpr int GNT = 128;       // threads (samples per tile) of the gradient kernel
-constexpr int GBLOCKS = 256;   // workgroups: partial gradients to reduce
-constexpr int PW = NP + 2;     // partial: gradient, loss sum, row count
+//
+// Every product of the network runs on FP32 MFMA (FP32 operands, products
+// and accumulation).  A wave takes 16 samples at a time in the transposed
+// form of mlp.hpp, H_out^T = W H_in^T, on v_mfma_f32_16x16x4: lane (q, j) of
+// the accumulators holds the units 4q..4q+3 and 16+4q..16+4q+3 (slot_unit)
+// of sample j, which is the B operand of the next product as it stands when
+// that product's k index runs over the units in the same order -- forward
+// (W) and backward (W^T) alike, so activations and deltas never move between
+// lanes.  The weight gradients contract over samples instead,
+// dW[a][k] = sum_s g[s][a] h[s][k], so deltas and activations pass through a
+// wave-private LDS tile once and accumulate on v_mfma_f32_32x32x2.
+//
+// About 13 kflop a sample, bound by the FP32 MFMA issue (3456 cycles a block)
+// and, at the training batch of 65536 samples, by the start and the end of
+// the waves, which take two blocks each: 20 us with a trace on (78 us with
+// products on the vector ALU and weight gradients that each re-read 128
+// samples from LDS), 9.9 us more for every 65536 samples beyond.
+constexpr int GWAVES = 8;            // waves of a workgroup (two a SIMD)
+constexpr int GNT = 64 * GWAVES;
+constexpr int GBLOCKS = 256;         // most workgroups: partial gradients to reduce
+constexpr int PW = NP + 2;           // partial: gradient, loss sum, row count
+constexpr int TS = 36;               // row stride of the LDS tiles (16 samples x 32 units)
 
-__global__ __launch_bounds__(GNT) void grad_kernel(const float* __restrict__ P, size_t n,
-                                                   const float* __restrict__ feats,
-                                                   const float* __restrict__ target,
-                                                   const unsigned char* __restrict__ mask,
-                                                   float* __restrict__ partial) {
-  __shared__ float Ps[NP];
-  __shared__ float G[GNT][H + 1];
-  __shared__ float Hh[GNT][H + 1];
-  const int tid = threadIdx.x;
-  for (int k = tid; k < NP; k += GNT) Ps[k] = P[k];
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// v of lane l + the DPP row shifts' sums: lane 15 of each 16-lane row ends
+// with the row's sum
+AST_DEV float row_sum15(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x112, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x114, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118, 0xf, 0xf, true));
+  return v;
+}
+
+// orders a wave's LDS accesses before and after it (one wave's run in order)
+AST_DEV void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// the two 16-unit tiles of W x (A: 8 k-steps a tile; B: a unit vector in
+// slot order), added to c
+AST_DEV void product32(const float* A, const float* B, f32x4* c) {
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[k], B[k], c[0], 0, 0, 0);
+    c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[8 + k], B[k], c[1], 0, 0, 0);
+  }
+}
+
+__global__ __launch_bounds__(GNT, 2) void grad_kernel(const float* __restrict__ P, size_t n,
+                                                      const float* __restrict__ feats,
+                                                      const float* __restrict__ target,
+                                                      const unsigned char* __restrict__ mask,
+                                                      float* __restrict__ partial) {
+  // the waves' tiles (deltas, activations), then four partial gradients
+  constexpr int kTileFloats = 2 * 16 * TS;
+  constexpr int kShared = GWAVES * kTileFloats > 4 * PW ? GWAVES * kTileFloats : 4 * PW;
+  __shared__ __align__(16) float sh[kShared];
+  // W1, the biases and w4, read from here where they are used
+  constexpr int vB2 = oW2, vB3 = vB2 + H, vW4 = vB3 + H;
+  __shared__ __align__(16) float vec[vW4 + H];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, j = lane & 15;
+  float* tg = sh + wave * kTileFloats;
+  float* th = tg + 16 * TS;
+  // operands: A[8 t + k] = row 16 t + j of the matrix, unit slot_unit(8 q + k),
+  // gathered from an LDS copy of the masters whose rows are padded to 33
+  constexpr int HP = H + 1, kW2 = 0, kW3 = kW2 + H * HP;
+  static_assert(kW3 + H * HP <= kShared, "staged masters fit the tiles' space");
+  // a block's inputs, fetched a block ahead: the features of sample s0 + j
+  // for layer 1 (x0, x1), those of dW1's B operand (lane (q, j): feature j of
+  // sample s0 + 4 k + q, and a column of ones that sums db1), the target
+  const size_t blocks = (n + 15) / 16;
+  const size_t first = (size_t)blockIdx.x * GWAVES + wave, stride = (size_t)gridDim.x * GWAVES;
+  float x0 = 0.f, x1 = 0.f, xb[4] = {0.f, 0.f, 0.f, 0.f}, tv = 0.f;
+  bool valid = false;
+  auto fetch = [&](size_t blk) {
+    const size_t s0 = blk * 16, s = s0 + j, sc = s < n ? s : n - 1;
+    valid = s < n && (mask == nullptr || mask[s]);
+    x0 = feats[(size_t)q * n + sc];
+    x1 = q < IN - 4 ? feats[(size_t)(4 + q) * n + sc] : 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const size_t ss = s0 + 4 * k + q;
+      xb[k] = j < IN ? feats[(size_t)j * n + (ss < n ? ss : n - 1)] : (j == IN ? 1.f : 0.f);
+    }
+    tv = target[sc];
+  };
+  if (first < blocks) fetch(first);
+  float A2[16], A3[16], A2t[16], A3t[16];
+  for (int p = threadIdx.x; p < vW4 + H; p += GNT)
+    vec[p] = P[p < vB2 ? p : p < vB3 ? oB2 + (p - vB2) : p < vW4 ? oB3 + (p - vB3) : oW4 + (p - vW4)];
+  for (int p = threadIdx.x; p < H * H; p += GNT) {
+    sh[kW2 + (p >> 5) * HP + (p & 31)] = P[oW2 + p];
+    sh[kW3 + (p >> 5) * HP + (p & 31)] = P[oW3 + p];
+  }
   __syncthreads();
-  // owned gradient entries: dW3/dW2 rows i = tid/4, columns 8*(tid%4)..+7
-  const int oi = tid >> 2, oj = (tid & 3) * 8;
-  float aW3[8], aW2[8], aW1[2] = {0.f, 0.f}, aB = 0.f, aW4 = 0.f, aB4 = 0.f;
-  for (int c = 0; c < 8; c++) aW3[c] = aW2[c] = 0.f;
-  float lsum = 0.f, cnt = 0.f;
-  const size_t tiles = (n + GNT - 1) / GNT;
-  for (size_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-    const size_t i = t * GNT + tid;
-    const bool valid = i < n && (mask == nullptr || mask[i]);
-    float x[IN], h1[H], h2[H], h3[H], g[H];
-    for (int k = 0; k < IN; k++) x[k] = i < n ? feats[k * n + i] : 0.f;
-    for (int a = 0; a < H; a++) {
-      float s = Ps[oB1 + a];
-      for (int k = 0; k < IN; k++) s += Ps[oW1 + a * IN + k] * x[k];
-      h1[a] = tanh_f(s);
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int u = slot_unit(8 * q + k), r = 16 * t + j;
+      A2[8 * t + k] = sh[kW2 + r * HP + u];
+      A3[8 * t + k] = sh[kW3 + r * HP + u];
+      A2t[8 * t + k] = sh[kW2 + u * HP + r];
+      A3t[8 * t + k] = sh[kW3 + u * HP + r];
     }
-    for (int a = 0; a < H; a++) {
-      float s = Ps[oB2 + a];
-      for (int k = 0; k < H; k++) s += Ps[oW2 + a * H + k] * h1[k];
-      h2[a] = tanh_f(s);
+  }
+  __syncthreads();
+  const float b4 = P[oB4];
+  auto units = [&](int off, f32x4* c) {  // a unit vector of vec, in slot order
+    c[0] = *reinterpret_cast<const f32x4*>(vec + off + 4 * q);
+    c[1] = *reinterpret_cast<const f32x4*>(vec + off + 16 + 4 * q);
+  };
+  f32x16 dW3 = {0.f}, dW2 = {0.f};
+  f32x4 dW1[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  float s3[8], s2[8], s4[8], sb4 = 0.f, lsum = 0.f, cnt = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; k++) s3[k] = s2[k] = s4[k] = 0.f;
+
+  for (size_t blk = first; blk < blocks; blk += stride) {  // wave-uniform: EXEC stays full
+    f32x4 c[2];
+    float h1[8], h2[8], h3[8], g[8];
+    units(oB1, c);
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const float* r = vec + oW1 + (16 * t + j) * IN;
+      c[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(r[q], x0, c[t], 0, 0, 0);
+      c[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q < IN - 4 ? r[4 + q] : 0.f, x1, c[t], 0, 0, 0);
     }
-    float y = Ps[oB4];
-    for (int a = 0; a < H; a++) {
-      float s = Ps[oB3 + a];
-      for (int k = 0; k < H; k++) s += Ps[oW3 + a * H + k] * h2[k];
-      h3[a] = tanh_f(s);
-      y += Ps[oW4 + a] * h3[a];
+#pragma unroll
+    for (int k = 0; k < 8; k++) h1[k] = tanh_f(c[k >> 2][k & 3]);
+    units(vB2, c);
+    product32(A2, h1, c);
+#pragma unroll
+    for (int k = 0; k < 8; k++) h2[k] = tanh_f(c[k >> 2][k & 3]);
+    units(vB3, c);
+    product32(A3, h2, c);
+    float y = 0.f;
+    f32x4 w4[2];
+    units(vW4, w4);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      h3[k] = tanh_f(c[k >> 2][k & 3]);
+      y += w4[k >> 2][k & 3] * h3[k];
     }
-    const float e = valid ? (y - target[i]) : 0.f;
-    lsum += e * e;
-    cnt += valid ? 1.f : 0.f;
+    y += __shfl_xor(y, 16, 64);
+    y += __shfl_xor(y, 32, 64);
+    y += b4;
+    const float e = valid ? y - tv : 0.f;
+    if (q == 0) {
+      lsum += e * e;
+      cnt += valid ? 1.f : 0.f;
+    }
     const float dy = 2.f * e;  // d(e^2)/dy; the mean is taken in the reduction
-    // layer 4 and layer-3 deltas
-    for (int a = 0; a < H; a++) g[a] = dy * Ps[oW4 + a] * (1.f - h3[a] * h3[a]);
-    __syncthreads();
-    for (int a = 0; a < H; a++) {
-      G[tid][a] = g[a];
-      Hh[tid][a] = h2[a];
+    if (q == 0) sb4 += dy;
+    float xw[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) xw[k] = xb[k];
+    if (blk + stride < blocks) fetch(blk + stride);
+    // dW = sum over the block's samples of (the tile tg)^T th
+    auto contract = [&](f32x16& dW) {
+      const int half = lane >> 5, col = lane & 31;
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        dW = __builtin_amdgcn_mfma_f32_32x32x2f32(tg[(2 * k + half) * TS + col],
+                                                  th[(2 * k + half) * TS + col], dW, 0, 0, 0);
+    };
+    auto put = [&](float* T, const float* v) {  // sample j, units 4q.. and 16+4q..
+      *reinterpret_cast<f32x4*>(T + j * TS + 4 * q) = f32x4{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<f32x4*>(T + j * TS + 16 + 4 * q) = f32x4{v[4], v[5], v[6], v[7]};
+    };
+    // layer-3 deltas
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      s4[k] += dy * h3[k];
+      g[k] = dy * w4[k >> 2][k & 3] * (1.f - h3[k] * h3[k]);
+      s3[k] += g[k];
     }
-    G[tid][H] = dy;
-    Hh[tid][H] = 0.f;
-    __syncthreads();
-    for (int s = 0; s < GNT; s++) {
-      const float gi = G[s][oi];
-      for (int c = 0; c < 8; c++) aW3[c] += gi * Hh[s][oj + c];
+    put(tg, g);
+    put(th, h2);
+    wave_lds_fence();
+    contract(dW3);
+    // layer-2 deltas: (W3^T g3) (1 - h2^2)
+    c[0] = c[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    product32(A3t, g, c);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      g[k] = c[k >> 2][k & 3] * (1.f - h2[k] * h2[k]);
+      s2[k] += g[k];
     }
-    if (tid < H) {
-      float sb = 0.f;
-      for (int s = 0; s < GNT; s++) sb += G[s][tid];
-      aB += sb;  // db3 (tid < 32)
+    wave_lds_fence();
+    put(tg, g);
+    put(th, h1);
+    wave_lds_fence();
+    contract(dW2);
+    // layer-1 deltas: (W2^T g2) (1 - h1^2)
+    c[0] = c[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    product32(A2t, g, c);
+#pragma unroll
+    for (int k = 0; k < 8; k++) g[k] = c[k >> 2][k & 3] * (1.f - h1[k] * h1[k]);
+    wave_lds_fence();
+    put(tg, g);
+    wave_lds_fence();
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        dW1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(tg[(4 * k + q) * TS + 16 * t + j], xw[k],
+                                                      dW1[t], 0, 0, 0);
+    wave_lds_fence();
+  }
+
+  // this workgroup's partial gradient: four waves leave theirs in LDS, the
+  // others add theirs, and the four are summed in order
+  lsum = row_sum15(lsum);
+  cnt = row_sum15(cnt);
+  sb4 = row_sum15(sb4);
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    s3[k] = row_sum15(s3[k]);
+    s2[k] = row_sum15(s2[k]);
+    s4[k] = row_sum15(s4[k]);
+  }
+  float* R = sh + (wave & 3) * PW;
+  auto leave = [&](bool add) {
+    auto at = [&](int p, float v) { R[p] = add ? R[p] + v : v; };
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int row = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), col = lane & 31;
+      at(oW3 + row * H + col, dW3[r]);
+      at(oW2 + row * H + col, dW2[r]);
     }
-    // dW4 = sum dy h3 and db4: h3 is not in LDS; accumulate with a second pass
-    __syncthreads();
-    for (int a = 0; a < H; a++) Hh[tid][a] = h3[a];
-    __syncthreads();
-    if (tid >= 32 && tid < 64) {
-      float s4 = 0.f;
-      for (int s = 0; s < GNT; s++) s4 += G[s][H] * Hh[s][tid - 32];
-      aW4 += s4;
-    }
-    if (tid == 64) {
-      float s4 = 0.f;
-      for (int s = 0; s < GNT; s++) s4 += G[s][H];
-      aB4 += s4;
-    }
-    // layer-2 deltas: g2 = (W3^T g3) * (1 - h2^2)
-    float g2[H];
-    for (int k = 0; k < H; k++) {
-      float s = 0.f;
-      for (int a = 0; a < H; a++) s += Ps[oW3 + a * H + k] * g[a];
-      g2[k] = s * (1.f - h2[k] * h2[k]);
-    }
-    __syncthreads();
-    for (int a = 0; a < H; a++) {
-      G[tid][a] = g2[a];
-      Hh[tid][a] = h1[a];
-    }
-    __syncthreads();
-    for (int s = 0; s < GNT; s++) {
-      const float gi = G[s][oi];
-      for (int c = 0; c < 8; c++) aW2[c] += gi * Hh[s][oj + c];
-    }
-    if (tid >= 96 && tid < 128) {
-      float sb = 0.f;
-      for (int s = 0; s < GNT; s++) sb += G[s][tid - 96];
-      aB += sb;  // db2 (96 <= tid < 128)
-    }
-    // layer-1 deltas: g1 = (W2^T g2) * (1 - h1^2)
-    for (int k = 0; k < H; k++) {
-      float s = 0.f;
-      for (int a = 0; a < H; a++) s += Ps[oW2 + a * H + k] * g2[a];
-      g[k] = s * (1.f - h1[k] * h1[k]);
-    }
-    __syncthreads();
-    for (int a = 0; a < H; a++) G[tid][a] = g[a];
-    for (int k = 0; k < IN; k++) Hh[tid][k] = x[k];
-    __syncthreads();
-    for (int r = 0; r < 2; r++) {  // dW1: 192 entries, tid and tid + 128
-      const int e1 = tid + r * GNT;
-      if (e1 < H * IN) {
-        const int a = e1 / IN, k = e1 % IN;
-        float s1 = 0.f;
-        for (int s = 0; s < GNT; s++) s1 += G[s][a] * Hh[s][k];
-        aW1[r] += s1;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int row = 16 * t + 4 * q + v;
+        if (j < IN) at(oW1 + row * IN + j, dW1[t][v]);
+        else if (j == IN) at(oB1 + row, dW1[t][v]);
+      }
+    if (j == 15) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int u = slot_unit(8 * q + k);
+        at(oB3 + u, s3[k]);
+        at(oB2 + u, s2[k]);
+        at(oW4 + u, s4[k]);
+      }
+      if (q == 0) {
+        at(oB4, sb4);
+        at(NP, lsum);
+        at(NP + 1, cnt);
       }
     }
-    if (tid >= 64 && tid < 96) {
-      float sb = 0.f;
-      for (int s = 0; s < GNT; s++) sb += G[s][tid - 64];
-      aB += sb;  // db1 (64 <= tid < 96)
-    }
-  }
-  // this workgroup's partial gradient
+  };
+  __syncthreads();
+  if (wave >= 4) leave(false);
+  __syncthreads();
+  if (wave < 4) leave(true);
+  __syncthreads();
   float* out = partial + (size_t)blockIdx.x * PW;
-  for (int c = 0; c < 8; c++) {
-    out[oW3 + oi * H + oj + c] = aW3[c];
-    out[oW2 + oi * H + oj + c] = aW2[c];
+  for (int p = threadIdx.x; p < PW; p += GNT)
+    out[p] = (sh[p] + sh[PW + p]) + (sh[2 * PW + p] + sh[3 * PW + p]);
+}
+
+// Sums the workgroups' partials in a fixed order; grad = sum / count, loss =
+// mean.  A workgroup takes RCOLS entries, each summed by RSLICES threads over
+// every RSLICES-th partial (75 workgroups; one thread an entry over all
+// partials, 10 workgroups, took 114 us of latency for 256 of them).
+constexpr int RCOLS = 32, RSLICES = 16, RNT = RCOLS * RSLICES;
+
+__global__ __launch_bounds__(RNT) void grad_reduce_kernel(const float* __restrict__ partial,
+                                                          int nblocks, float* __restrict__ grad,
+                                                          float* __restrict__ loss) {
+  __shared__ float part[RSLICES][RCOLS], cpart[RNT];
+  const int col = threadIdx.x % RCOLS, slice = threadIdx.x / RCOLS;
+  const int k = blockIdx.x * RCOLS + col;
+  float s = 0.f, cnt = 0.f;
+  if (k < NP + 1) {
+#pragma unroll 8
+    for (int b = slice; b < nblocks; b += RSLICES) s += partial[(size_t)b * PW + k];
   }
-  for (int r = 0; r < 2; r++)
-    if (tid + r * GNT < H * IN) out[oW1 + tid + r * GNT] = aW1[r];
-  if (tid < 32) out[oB3 + tid] = aB;
-  if (tid >= 96) out[oB2 + tid - 96] = aB;
-  if (tid >= 64 && tid < 96) out[oB1 + tid - 64] = aB;
-  if (tid >= 32 && tid < 64) out[oW4 + tid - 32] = aW4;
-  if (tid == 64) out[oB4] = aB4;
-  // loss and count: wave sums, then one lane per wave adds in LDS order
+  for (int b = threadIdx.x; b < nblocks; b += RNT) cnt += partial[(size_t)b * PW + NP + 1];
+  part[slice][col] = s;
+  cpart[threadIdx.x] = cnt;
   __syncthreads();
-  G[tid][0] = lsum;
-  G[tid][1] = cnt;
-  __syncthreads();
-  if (tid == 0) {
-    float ls = 0.f, cs = 0.f;
-    for (int s = 0; s < GNT; s++) {
-      ls += G[s][0];
-      cs += G[s][1];
-    }
-    out[NP] = ls;
-    out[NP + 1] = cs;
+  for (int w = RNT / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) cpart[threadIdx.x] += cpart[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (slice == 0 && k < NP + 1) {
+    float t = part[0][col];
+#pragma unroll
+    for (int i = 1; i < RSLICES; i++) t += part[i][col];
+    const float inv = cpart[0] > 0.f ? 1.f / cpart[0] : 0.f;
+    if (k < NP) grad[k] = t * inv;
+    else if (loss) *loss = t * inv;
   }
 }
 
-// sums the partials in block order; grad = sum / count, loss = mean
-__global__ void grad_reduce_kernel(const float* __restrict__ partial, int nblocks,
-                                   float* __restrict__ grad, float* __restrict__ loss) {
-  float cnt = 0.f;
-  for (int b = 0; b < nblocks; b++) cnt += partial[(size_t)b * PW + NP + 1];
-  const float inv = cnt > 0.f ? 1.f / cnt : 0.f;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < NP + 1; k += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int b = 0; b < nblocks; b++) s += partial[(size_t)b * PW + k];
-    if (k < NP) grad[k] = s * inv;
-    else if (loss) *loss = s * inv;
+// The master parameter behind element v of lane `lane` of MFMA operand `op`
+// (-1: none, the element is zero).  No two elements share a parameter.
+AST_DEV int operand_param(int op, int lane, int v) {
+  const int i = lane & 15, s = 8 * (lane >> 4) + v;
+  if (op < 2) return s < IN ? oW1 + (op * 16 + i) * IN + s : -1;  // layer 1: feature slots 0..5
+  if (op < 6) {  // layers 2, 3: permuted hidden slots
+    const int off = op < 4 ? oW2 : oW3, mb = (op - 2) % 2;
+    return off + (mb * 16 + i) * H + slot_unit(s);
   }
+  return i == 0 ? oW4 + slot_unit(s) : -1;  // output: row 0 = w4
 }
+constexpr int OPELEMS = OPS * 64 * 8;
 
 // rebuilds the BF16 MFMA operands from the FP32 masters
 __global__ void refresh_bf16_kernel(unsigned char* buf) {
   const float* P = (const float*)buf;
-  bf16x8* A = (bf16x8*)(buf + BF_OFF);
-  const int lane = threadIdx.x & 63, op = threadIdx.x >> 6;  // 7 waves
-  if (op >= OPS) return;
-  const int i = lane & 15, q = lane >> 4;
-  bf16x8 a;
-  for (int v = 0; v < 8; v++) {
-    const int s = 8 * q + v;
-    float w = 0.f;
-    if (op < 2) {  // layer 1: feature slots 0..5
-      if (s < IN) w = P[oW1 + (op * 16 + i) * IN + s];
-    } else if (op < 6) {  // layers 2, 3: permuted hidden slots
-      const int layer = (op - 2) / 2, mb = (op - 2) % 2;
-      const int off = layer == 0 ? oW2 : oW3;
-      w = P[off + (mb * 16 + i) * H + slot_unit(s)];
-    } else {  // output: row 0 = w4
-      if (i == 0) w = P[oW4 + slot_unit(s)];
-    }
-    a[v] = (__bf16)w;
+  __bf16* A = (__bf16*)(buf + BF_OFF);
+  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < OPELEMS; e += gridDim.x * blockDim.x) {
+    const int k = operand_param(e >> 9, (e >> 3) & 63, e & 7);
+    A[e] = (__bf16)(k >= 0 ? P[k] : 0.f);
   }
-  A[op * 64 + lane] = a;
 }
 
-__global__ void adam_kernel(float* __restrict__ P, const float* __restrict__ g,
+// One Adam step on the masters and the rebuilt MFMA operands in one kernel:
+// thread e < OPELEMS owns operand element e and the parameter behind it, the
+// threads after them the biases, which have no operand.
+__global__ void adam_kernel(unsigned char* buf, const float* __restrict__ g,
                             float* __restrict__ st, int step, float lr) {
+  float* P = (float*)buf;
+  __bf16* A = (__bf16*)(buf + BF_OFF);
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < NP; k += gridDim.x * blockDim.x) {
+  auto update = [&](int k) {
     float m = st[k], v = st[NP + k];
     m = b1 * m + (1.f - b1) * g[k];
     v = b2 * v + (1.f - b2) * g[k] * g[k];
     st[k] = m;
     st[NP + k] = v;
-    P[k] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
+    const float p = P[k] - lr * (m / c1) / (sqrtf(v / c2) + eps);
+    P[k] = p;
+    return p;
+  };
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < OPELEMS) {
+    const int k = operand_param(e >> 9, (e >> 3) & 63, e & 7);
+    A[e] = (__bf16)(k >= 0 ? update(k) : 0.f);
+  } else {
+    const int b = e - OPELEMS;
+    if (b < 3 * H) update((b < H ? oB1 : b < 2 * H ? oB2 : oB3) + b % H);
+    else if (b == 3 * H) update(oB4);
   }
 }
+constexpr int ADAM_THREADS = OPELEMS + 3 * H + 1;
 
 }  // namespace mlp
 }  // namespace ast
@@ -345,18 +491,21 @@ extern "C" int ast_mlp_loss_grad(const ast_mlp_t* mlp, size_t n, const float* fe
   if (!mlp || !feats || !target || !grad || !work)
     return ast_fail(AST_ERR_ARG, "ast_mlp_loss_grad: null pointer");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(grad_kernel, dim3(GBLOCKS), dim3(GNT), 0, st, (const float*)mlp, n, feats,
-                     target, mask, work);
+  const size_t groups = (n + 16 * GWAVES - 1) / (16 * GWAVES);
+  const int wgs = groups < 1 ? 1 : groups > GBLOCKS ? GBLOCKS : (int)groups;
+  hipLaunchKernelGGL(grad_kernel, dim3(wgs), dim3(GNT), 0, st, (const float*)mlp, n, feats, target,
+                     mask, work);
   AST_LAUNCH_CHECK("ast_mlp_loss_grad launch");
-  hipLaunchKernelGGL(grad_reduce_kernel, dim3(10), dim3(256), 0, st, work, GBLOCKS, grad, loss);
+  hipLaunchKernelGGL(grad_reduce_kernel, dim3((NP + RCOLS) / RCOLS), dim3(RNT), 0, st, work, wgs,
+                     grad, loss);
   AST_LAUNCH_CHECK("ast_mlp_loss_grad reduce");
   return AST_OK;
 }
 
 extern "C" int ast_mlp_refresh(ast_mlp_t* mlp, void* stream) {
   if (!mlp) return ast_fail(AST_ERR_ARG, "ast_mlp_refresh: null pointer");
-  hipLaunchKernelGGL(refresh_bf16_kernel, dim3(1), dim3(64 * OPS), 0, (hipStream_t)stream,
-                     (unsigned char*)mlp);
+  hipLaunchKernelGGL(refresh_bf16_kernel, dim3((OPELEMS + 255) / 256), dim3(256), 0,
+                     (hipStream_t)stream, (unsigned char*)mlp);
   AST_LAUNCH_CHECK("ast_mlp_refresh launch");
   return AST_OK;
 }
@@ -364,10 +513,10 @@ extern "C" int ast_mlp_refresh(ast_mlp_t* mlp, void* stream) {
 extern "C" int ast_mlp_adam(ast_mlp_t* mlp, const float* grad, float* state, int step, float lr,
                             void* stream) {
   if (!mlp || !grad || !state || step < 1) return ast_fail(AST_ERR_ARG, "ast_mlp_adam: bad argument");
-  hipLaunchKernelGGL(adam_kernel, dim3(10), dim3(256), 0, (hipStream_t)stream, (float*)mlp, grad,
-                     state, step, lr);
+  hipLaunchKernelGGL(adam_kernel, dim3((ADAM_THREADS + 255) / 256), dim3(256), 0,
+                     (hipStream_t)stream, (unsigned char*)mlp, grad, state, step, lr);
   AST_LAUNCH_CHECK("ast_mlp_adam launch");
-  return ast_mlp_refresh(mlp, stream);
+  return AST_OK;
 }
 
 extern "C" int ast_mlp_set_params(ast_mlp_t* mlp, const float* host_params, void* stream) {
