@@ -35,7 +35,7 @@ int ast_step_f64_rows(const ast_grid_t* g, const double* s, const double* u, dou
                       double* u2, double* T, const double* T_do, const double* TT, int method,
                       ast_stats_t* stats, int rows, const ast::StepTime* tm,
                       const ast_sources_t* src, void* stream);
-extern "C" int ast_get_tile_rows(void);
+int ast_tile_rows_setting(void);
 
 #define CK(call)                                              \
   do {                                                        \
@@ -47,7 +47,7 @@ struct ast_sim {
   ast_grid_t g;
   int precision;  // 0: FP64 planes, 1: FP32 planes
   int method;
-  int krows;   // FP32 strip tiling (rows per strip, or -S strips per band)
+  int krows;   // FP32 strip tiling (rows per strip, -S strips per band, 0: by size)
   int rows64;  // FP64 rows per strip (0: the kernel's default)
   size_t cells;
   void* plane[4];  // s0, u0, s1, u1
@@ -193,7 +193,7 @@ extern "C" int ast_sim_create(const ast_grid_t* g, int precision, int method, as
   S->g = *g;
   S->precision = precision;
   S->method = method;
-  S->krows = ast_get_tile_rows();
+  S->krows = ast_tile_rows_setting();
   S->cells = (size_t)g->N * g->M;
   const size_t bytes = S->cells * 2 * elem(S);
   hipError_t e = hipSuccess;
@@ -436,13 +436,19 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
   if (!S) return ast_fail(AST_ERR_ARG, "ast_sim_autotune: null sim");
   // default: strips of 4-16 rows, and the tilings that give every SIMD 2 to
   // 5 waves of (nearly) equal height, S strips per band with S * bands
-  // waves (a wave strip has 60 output columns; a CU has 4 SIMDs); the FP64
-  // step takes strips of 1 to 32 rows
+  // waves (a wave strip has 60 output columns; a CU has 4 SIMDs); the FP32
+  // exact solver's strips are of 1 to 8 rows (its waves differ too much for
+  // taller ones), the FP64 step's of 1 to 32
   int dflt[8] = {4, 8, 12, 16};
+  static const int dflt_exact[5] = {1, 2, 3, 4, 8};
   static const int dflt64[11] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
   if ((!candidates || ncand <= 0) && S->precision == 0) {
     candidates = dflt64;
     ncand = 11;
+  }
+  if ((!candidates || ncand <= 0) && S->method == AST_EXACT) {
+    candidates = dflt_exact;
+    ncand = 5;
   }
   if (!candidates || ncand <= 0) {
     int nd = 4, dev = 0, cus = 0;

@@ -37,7 +37,9 @@
 using namespace ast;
 using namespace ast::f32;
 
-static int g_krows = 8;
+// The tiling set by ast_set_tile_rows (0: not set, the step takes
+// default_tile's)
+static int g_krows = 0;
 
 // krows > 0: rows per strip; krows = -S: S strips of (nearly) equal height
 // per band (strip_rows)
@@ -47,8 +49,57 @@ extern "C" int ast_set_tile_rows(int krows) {
   g_krows = krows;
   return AST_OK;
 }
-extern "C" int ast_get_tile_rows(void) { return g_krows; }
+extern "C" int ast_get_tile_rows(void) { return g_krows ? g_krows : 8; }
+int ast_tile_rows_setting(void) { return g_krows; }
 
+// The tiling of a step for which none was set, by the grid's size.
+//
+// HLL family: a row of a wave is a dependent chain, so a small grid wants its
+// rows spread over as many waves as there are (4-row strips, the shortest of
+// the fast paths), a larger one strips of equal height that fill every SIMD
+// with the 4 waves it holds, or 3, 2, 1 if their strips would be shorter
+// than 4 rows, and 8, 12, ... rounds of 4 if they would be taller than the
+// fast paths' 64 rows.  Measured, HLLC, us a step (the rule / 8-row strips
+// before): 256x128 7.2 / 10.1, 1024x512 10.1 / 12.4, 1500x750 14.4 / 18.4,
+// 2048x1024 20.5 / 22.9, 8192x400 26.9 / 29.1, 4096x2048 55.6 / 63.7.
+//
+// Exact solver: its waves differ by several times (patterns and iterations
+// diverge), so short strips balance them: 1 row up to 9400 wave rows
+// (bands x rows), 2 up to 20000, 4 up to 100000, 8 beyond, where the 5 rows
+// a strip reads and solves over those it holds weigh more.  Measured, us a
+// step (1 / 2 / 4 / 8 rows): 256x128 13.1 / 19.6 / 31.0 / 58.4, 1024x512
+// 20.5 / 21.0 / 32.4 / 56.3, 1500x750 34.5 / 27.6 / 36.0 / 63.5, 2048x1024
+// 58.1 / 43.8 / 40.0 / 61.1, 8192x400 85.3 / 62.5 / 53.5 / 63.6, 4096x2048
+// 209 / 149 / 121 / 111.
+static int default_tile(const ast_grid_t& g, int method) {
+  const long long nbands = (g.N + WOUT - 1) / WOUT;
+  int tile = 4;
+  if (method == AST_EXACT) {
+    const long long rows = nbands * g.M;
+    tile = rows <= 9400 ? 1 : rows <= 20000 ? 2 : rows <= 100000 ? 4 : 8;
+  } else {
+    auto strips = [&](long long waves) { return waves * 1024 / nbands; };
+    // the shortest strip of S a band: its middle ones (strip_rows)
+    auto shortest = [&](long long S) {
+      const long long e = std::max(4LL, (g.M / S + 2) / 4 * 4);
+      return S >= 3 && g.M - 2 * e >= S - 2 ? (g.M - 2 * e) / (S - 2) : g.M / S;
+    };
+    long long waves = 4;
+    while (strips(waves) < 1 || tallest_strip(g.M, (int)-std::min(strips(waves), (long long)g.M)) > 64)
+      waves += 4;
+    for (; waves >= 1; waves -= waves > 4 ? 4 : 1) {
+      const long long S = strips(waves);
+      if (S >= 1 && S <= g.M && shortest(S) >= 4) {
+        tile = (int)-S;
+        break;
+      }
+    }
+  }
+  // one buffer range covers a strip's rows: the 8-row strips of a wider grid
+  return strip_fits(g, tallest_strip(g.M, tile)) ? tile : 8;
+}
+
+// krows: the strip tiling (0: default_tile's).
 // tm (may be null): the runtime's time protocol (time_slots.h).  Null: the
 // reference protocol (the step lowers *T, dt is *T_do, a learned guess is
 // always on).  Otherwise the step lowers the slots of tm->cur and, with
@@ -67,7 +118,8 @@ int ast_step_f32_rows(const ast_grid_t* g, const float* s, const float* u, float
     return ast_fail(AST_ERR_ARG, "ast_step_f32: null state or time pointer");
   if (s == s2 || u == u2 || s == u2 || u == s2)
     return ast_fail(AST_ERR_ARG, "ast_step_f32: output planes must not alias the input planes");
-  if (krows == 0 || krows > 1024 || (krows < 0 && -(long long)krows > g->M))
+  if (krows == 0) krows = default_tile(*g, method);
+  if (krows > 1024 || (krows < 0 && -(long long)krows > g->M))
     return ast_fail(AST_ERR_ARG, "ast_step_f32: strip tiling %d for %d rows", krows, g->M);
   const int height = tallest_strip(g->M, krows);
   KTime kt = {nullptr, nullptr, nullptr, 0};

@@ -370,17 +370,17 @@ struct Row {
   static constexpr int e0 = J & 1, e1 = (J + 1) & 1;
 };
 
-// One wave's strip.  FAST (wave-uniform): the strip has 4 to 64 rows and its
-// columns are interior or its band's ghost columns follow a per-lane rule,
-// so rows are raw buffer loads at fixed per-lane offsets (kFast, kFastX: no
-// ghost row, no frozen cell either, rows in groups of four and a tail of 1-3
-// rows, the exact solver a multiple of 4 rows; kFastE: ghost rows by row
-// rules, frozen tests per row, a multiple of 4 rows);
+// One wave's strip.  FAST (wave-uniform): the strip has 4 (the exact solver:
+// 1) to 64 rows and its columns are interior or its band's ghost columns
+// follow a per-lane rule, so rows are raw buffer loads at fixed per-lane
+// offsets (kFast, kFastX: no ghost row, no frozen cell either, rows in groups
+// of four and a tail of 1-3 rows; kFastE: ghost rows by row rules, frozen
+// tests per row, a multiple of 4 rows; the exact solver any number of rows);
 // otherwise load() applies the boundary rules, the frozen tests run per row,
 // and the rows of the last group of four that lie past the strip vote for no
 // dt (their stores fall outside the store range).
 //
-// Rows are processed four per trip with the window held in w[4] (row r in
+// Rows are processed four per trip (the exact solver: one) with the window held in w[4] (row r in
 // slot (r - m0) & 3): the slide of the window is a change of names, not a
 // copy.  Row m + 3 is fetched while row m is computed; no branch separates
 // the four rows of a trip, so the fetch stays a row ahead of its use.  The
@@ -434,7 +434,7 @@ AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, c
   const unsigned rb = a.row_bytes;
   // loads: FAST strips read rows m0-2 .. m1+1 through one resource per plane
   // (kFastE: the rows of the grid among them, which hold every row a ghost
-  // row names; a strip of kFastE has at least 4 rows, so M >= 4)
+  // row names: M >= 4)
   const int rlo = PATH == kFastE ? max(m0 - 2, 0) : m0 - 2;
   const int rhi = PATH == kFastE ? min(m1 + 1, M - 1) : m1 + 1;
   const size_t b0 = FAST ? (size_t)rlo * N : 0;
@@ -664,35 +664,48 @@ AST_DEV void run_strip(const ast_grid_t& g, const Consts& c, const Consts& cw, c
     pend_vo = a.st_off + (unsigned)(m - m0) * rb;
   };
 
-  // kFast, kFastX: whole groups of four, then the 1-3 rows left
-  // (wave-uniform).  Whole groups only: kFastE strips (a tail there costs
-  // the kernel registers) and the exact solver's strips (a tail would inline
-  // the solver twice more into a kernel whose code size already matters);
-  // the boundary variant runs its last group whole (rows past m1 drop out).
-  constexpr bool TAIL = (PATH == kFast || PATH == kFastX) && !is_exact(METHOD);
-  const int mq = TAIL ? m0 + ((m1 - m0) & ~3) : m1;
-  for (int m = m0; m < mq; m += 4) {
-    if constexpr (FAST && !is_exact(METHOD)) {
-      // wave priority falls with the fraction of the strip done: a SIMD
-      // issues for its oldest wave first, so without this its waves finish
-      // one after another and the last runs alone; with it the waves that
-      // are behind catch up and the SIMD's waves end together
-      const int q = (4 * (m - m0)) / (m1 - m0);  // wave-uniform, 0..3
-      if (q == 0) __builtin_amdgcn_s_setprio(3);
-      else if (q == 1) __builtin_amdgcn_s_setprio(2);
-      else if (q == 2) __builtin_amdgcn_s_setprio(1);
-      else __builtin_amdgcn_s_setprio(0);
+  if constexpr (is_exact(METHOD)) {
+    // one row a trip, the window moved along: four rows inlined eight solvers
+    // a strip variant (230 KB of code against the 64 KB instruction cache),
+    // and strips of any height take this loop
+    for (int m = m0; m < m1; m++) {
+      row(Row<0>{}, m);
+      for (int k = 0; k < 3; k++) w[k] = w[k + 1];
+      nv[0] = nv[1];
+      dd[0] = dd[1];
+      G[0] = G[1];
+      fr[0] = fr[1];
     }
-    row(Row<0>{}, m);
-    row(Row<1>{}, m + 1);
-    row(Row<2>{}, m + 2);
-    row(Row<3>{}, m + 3);
-  }
-  if constexpr (TAIL) {
-    const int rest = m1 - mq;
-    if (rest > 0) row(Row<0>{}, mq);
-    if (rest > 1) row(Row<1>{}, mq + 1);
-    if (rest > 2) row(Row<2>{}, mq + 2);
+  } else {
+    // kFast, kFastX: whole groups of four, then the 1-3 rows left
+    // (wave-uniform).  kFastE strips take whole groups only (a tail there
+    // costs the kernel registers); the boundary variant runs its last group
+    // whole (rows past m1 drop out).
+    constexpr bool TAIL = PATH == kFast || PATH == kFastX;
+    const int mq = TAIL ? m0 + ((m1 - m0) & ~3) : m1;
+    for (int m = m0; m < mq; m += 4) {
+      if constexpr (FAST) {
+        // wave priority falls with the fraction of the strip done: a SIMD
+        // issues for its oldest wave first, so without this its waves finish
+        // one after another and the last runs alone; with it the waves that
+        // are behind catch up and the SIMD's waves end together
+        const int q = (4 * (m - m0)) / (m1 - m0);  // wave-uniform, 0..3
+        if (q == 0) __builtin_amdgcn_s_setprio(3);
+        else if (q == 1) __builtin_amdgcn_s_setprio(2);
+        else if (q == 2) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(0);
+      }
+      row(Row<0>{}, m);
+      row(Row<1>{}, m + 1);
+      row(Row<2>{}, m + 2);
+      row(Row<3>{}, m + 3);
+    }
+    if constexpr (TAIL) {
+      const int rest = m1 - mq;
+      if (rest > 0) row(Row<0>{}, mq);
+      if (rest > 1) row(Row<1>{}, mq + 1);
+      if (rest > 2) row(Row<2>{}, mq + 2);
+    }
   }
   bstore(pend.r, pend.p, ws, pend_vo, 0);
   bstore(pend.vx, pend.vy, wu, pend_vo, 0);
@@ -807,8 +820,12 @@ AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCt
               frozen_possible(g, band * WOUT - 3, band * WOUT + 62, a.m0 - 2, a.m1 + 1);
   if (a.m0 < g.M) {
     // wave-uniform
-    const bool fast_rows = (a.cols_in || xfast) && a.m1 - a.m0 >= 4 && a.m1 - a.m0 <= 64 &&
-                           (!is_exact(METHOD) || ((a.m1 - a.m0) & 3) == 0);
+    const bool fast_rows =
+        (a.cols_in || xfast) && a.m1 - a.m0 <= 64 && (is_exact(METHOD) || a.m1 - a.m0 >= 4);
+    // strips that may run kFastE: it runs groups of four rows (the exact
+    // solver single ones, on a grid that holds every row a ghost row names)
+    const bool fast_edge =
+        fast_rows && (is_exact(METHOD) ? g.M >= 4 : ((a.m1 - a.m0) & 3) == 0);
     const bool rows_in = a.m0 - 2 >= 0 && a.m1 + 1 < g.M;
     if constexpr (PULSE) {
       // a grid with a pulsed side: the strips that hold its ghosts run the
@@ -834,7 +851,7 @@ AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCt
         else
           run_strip<METHOD, GEOM, WINDOW, kFastX, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt,
                                                        pp);
-      } else if (fast_rows && ((a.m1 - a.m0) & 3) == 0) {
+      } else if (fast_edge) {
         for (int k = 0; k < 2; k++) {
           const int ys = k ? AST_YHI : AST_YLO;
           const int ybc = g.bc[ys];
@@ -864,7 +881,7 @@ AST_DEV double strip_of_wave(const ast_grid_t& g, const Consts& c, const ExactCt
           run_strip<METHOD, GEOM, WINDOW, kFast, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt);
         else
           run_strip<METHOD, GEOM, WINDOW, kFastX, SRC>(g, c, cw, ex, s, u, s2, u2, a, UUx, UUy, st, dt);
-      } else if (fast_rows && ((a.m1 - a.m0) & 3) == 0 && !xpulse && !ypulse) {
+      } else if (fast_edge && !xpulse && !ypulse) {
         // the y-ghost rules of fetch_cell as row rules (only the first or last
         // strips of a band hold ghost rows)
         for (int k = 0; k < 2; k++) {

@@ -413,14 +413,16 @@ int ast_sim_learned_modes(ast_sim_t* sim, int* modes);
  * the automatic choice to meet them). */
 int ast_sim_set_learned_mode(ast_sim_t* sim, int mode);
 /* Strip tiling of the step.  FP32: rows > 0 rows per wave strip, rows = -S
- * S strips of (nearly) equal height per band of 60 columns; strips of 4 to
- * 64 rows inside the grid take the fast strip path.  FP64: rows > 0 rows
+ * S strips of (nearly) equal height per band of 60 columns; strips of 4 (the
+ * exact solver: 1) to 64 rows inside the grid take the fast strip path
+ * (default: chosen from the grid's size and the method).  FP64: rows > 0 rows
  * per wave strip (default: chosen from the grid's size and the method). */
 int ast_sim_set_tile_rows(ast_sim_t* sim, int rows);
 /* Times the step for each candidate tiling (NULL = a default list: FP32 4,
  * 8, 12, 16 rows and the tilings -S that give every SIMD 2, 3, 4 or 5 equal
- * waves; FP64 1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32 rows), keeps the fastest; reports it (may
- * be NULL).  State and time are left unchanged. */
+ * waves, with the exact solver 1, 2, 3, 4, 8 rows; FP64 1 to 6, 8, 12, 16,
+ * 24, 32 rows), keeps the fastest; reports it (may be NULL).  State and time
+ * are left unchanged. */
 int ast_sim_autotune(ast_sim_t* sim, const int* candidates, int ncand, int reps,
                      int* best_rows, float* best_us);
 /* The simulation's stream (hipStream_t) for event timing. */
@@ -468,7 +470,10 @@ void* ast_batch_stream(ast_batch_t* b);
 long long ast_batch_cells(const ast_batch_t* b);
 
 /* ---- tile configuration of the stand-alone FP32 step entry point --------
- * Strip tiling as for ast_sim_set_tile_rows (default 8 rows per strip). */
+ * Strip tiling as for ast_sim_set_tile_rows, for the steps and for
+ * simulations created afterwards.  Until it is set (ast_get_tile_rows then
+ * returns 8) each step takes the tiling its rule gives for the grid's size
+ * and method; the tiling never changes a result. */
 int ast_set_tile_rows(int rows);
 int ast_get_tile_rows(void);
 /* Doubles of device memory ast_conservation_sums needs at `out` (the two
