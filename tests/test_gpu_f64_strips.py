@@ -83,3 +83,23 @@ def test_frozen_cells_in_some_waves(dev, ora, N, M, rows):
 def test_default_heights(dev, ora, N, M, rows):
     p = problems.wind(N, M)
     _check(dev, ora, p.grid, p.s, p.u, G.HLLC, T_do=1e-2, rows=rows)
+
+
+def test_time_left_below_the_steps_minimum(dev):
+    """A T set below what the first step would find is what that step leaves (Kernel_TVD lowers
+    the *T it is given), for that step alone."""
+    from asteriy_2d_amd.sim import Simulation
+    p = problems.wind(64, 32)
+    with Simulation(p.grid, G.HLLC, "f64", p.s, p.u) as sim:
+        sim.run(2)
+        free = sim.time()["T_do"]
+        for graph in (False, True):
+            sim.set_state(p.s, p.u)
+            sim.set_time(0.25 * free, 1e-9, 0.0, 0)
+            sim.run(1, graph=graph)
+            assert sim.time()["T_do"] == 0.25 * free
+            sim.set_state(p.s, p.u)
+            sim.set_time(0.25 * free, 1e-9, 0.0, 0)
+            sim.run(20, graph=graph)
+            t = sim.time()
+            assert t["T"] == 1e7 and t["T_do"] > 0.5 * free and t["i"] == 20
