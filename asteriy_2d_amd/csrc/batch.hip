@@ -6,10 +6,21 @@
 // capacity); workgroup b takes items b, b + G, b + 2G, ... (remapped within
 // each round so that one XCD gets a contiguous run of items, which keeps
 // neighbouring strips of an instance in one L2), runs the same wave strip as
-// the single-grid step and lowers its instance's T.  A second kernel advances
-// every instance's time (funk_time, kernel.cu:1525-1536, per instance).  The
-// two-step ping-pong of both kernels is captured in one HIP graph.  Strip
-// heights are per grid shape and chosen by timing the batch itself.
+// the single-grid step.
+//
+// Time: each instance has the four scalars of the reference's protocol and
+// three slots.  Step j of a run lowers slot j mod 3, takes its dt from slot
+// (j - 1) mod 3 (T_do at the start of a run) and, in the workgroup of the
+// instance's first item, advances the time (funk_time, kernel.cu:1525-1536)
+// and resets slot (j + 1) mod 3, which no workgroup of this launch reads; a
+// small kernel closes each run.  A step is then one kernel (the time advance
+// as a kernel after every step took 4 us of 17 on 8 instances of up to
+// 512x256).  Runs of kBatchChunk steps are captured in one HIP graph.
+//
+// The instances' strip tilings are chosen by the size of the sweep
+// (batch_default_tiles: 8 grids of 128x64 to 512x256 at 10.6 us a step, 11.5 on
+// 4-row strips and 17 on 8-row ones with the time kernel); ast_batch_autotune
+// chooses them per grid shape by timing the batch itself.
 #include <hip/hip_runtime.h>
 #include <string.h>
 
@@ -29,26 +40,47 @@ struct BatchInst {
   Consts c;
   ExactCtx ex;
   float2* plane[4];  // s0, u0, s1, u1
-  double* scal;      // T, T_do, TT, i
-  int nbands, krows, nsg, first_item;
+  double* scal;      // T, T_do, TT, i, then the three dt slots
+  int nbands, krows, items, first_item;  // krows: the strip tiling (strip_rows)
 };
 
+constexpr int kBatchSlot = 4;    // words of an instance's scalars before its slots
+constexpr int kBatchScal = 16;   // words an instance (128 B: no line is shared)
+constexpr int kBatchChunk = 20;  // steps of a captured run (even)
+
+// One item of step `j` of a run.
 template <int METHOD, int GEOM>
-AST_DEV void batch_item(const BatchInst& I, int local, int from, double* red) {
+AST_DEV void batch_item(const BatchInst& I, int local, int from, int j, double* red) {
   NoStats st;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int band, m0, m1;
   strip_rows(I.g.M, I.nbands, I.krows, local, wave, band, m0, m1);
-  const double tmin = strip_of_wave<METHOD, GEOM, false>(
+  double* slot = I.scal + kBatchSlot;
+  const double* prev = slot + (j + 2) % 3;  // step j - 1's
+  double tmin = strip_of_wave<METHOD, GEOM, false>(
       I.g, I.c, I.ex, I.plane[2 * from], I.plane[2 * from + 1], I.plane[2 * (1 - from)],
-      I.plane[2 * (1 - from) + 1], [&]() { return I.scal[1]; }, band, m0, m1, st);
-  block_min_uniform<NT>(tmin, red, I.scal, 0);
+      I.plane[2 * (1 - from) + 1], [&]() { return j > 0 ? *prev : I.scal[1]; }, band, m0, m1, st);
+  if (local == 0 && threadIdx.x == 0) {
+    double* T = I.scal;
+    slot[(j + 1) % 3] = kSlotEmpty;
+    if (j > 0) {
+      T[1] = *prev;
+      T[2] = T[2] + T[1];
+      int* i = reinterpret_cast<int*>(T + 3);
+      *i = *i + 1;
+    } else {
+      // the first step lowers the T it finds, which its slot then holds
+      tmin = fmin(tmin, T[0]);
+      T[0] = kSlotEmpty;
+    }
+  }
+  block_min_uniform<NT>(tmin, red, slot + j % 3, 0);
 }
 
 template <int METHOD>
 __global__ __launch_bounds__(NT) void batch_step_kernel(const BatchInst* __restrict__ inst,
                                                         const int* __restrict__ item_inst,
-                                                        int total, int from) {
+                                                        int total, int from, int j) {
   __shared__ double red[WPB];
   for (int base = 0; base < total; base += gridDim.x) {
     const int in_round = min((int)gridDim.x, total - base);
@@ -57,21 +89,25 @@ __global__ __launch_bounds__(NT) void batch_step_kernel(const BatchInst* __restr
     const int k = __builtin_amdgcn_readfirstlane(item_inst[item]);  // instance of the item
     const BatchInst& I = inst[k];
     const int local = item - I.first_item;
-    if (I.g.geometry == AST_AXISYMMETRIC) batch_item<METHOD, AST_AXISYMMETRIC>(I, local, from, red);
-    else batch_item<METHOD, AST_PLANAR>(I, local, from, red);
+    if (I.g.geometry == AST_AXISYMMETRIC) batch_item<METHOD, AST_AXISYMMETRIC>(I, local, from, j, red);
+    else batch_item<METHOD, AST_PLANAR>(I, local, from, j, red);
     __syncthreads();  // red[] is reused by the next item
   }
 }
 
-__global__ void batch_time_kernel(const BatchInst* __restrict__ inst, int count) {
+// Closes a run whose last step was step `last`: funk_time per instance, and
+// every slot reset for the next run.
+__global__ void batch_close_kernel(const BatchInst* __restrict__ inst, int count, int last) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < count) {  // funk_time per instance
+  if (k < count) {
     double* T = inst[k].scal;
-    T[1] = T[0];
+    double* slot = T + kBatchSlot;
+    T[1] = slot[last % 3];
     T[2] = T[2] + T[1];
-    T[0] = 10000000;
+    T[0] = kSlotEmpty;
     int* i = (int*)(T + 3);
     *i = *i + 1;
+    for (int s = 0; s < 3; s++) slot[s] = kSlotEmpty;
   }
 }
 
@@ -88,7 +124,7 @@ struct ast_batch {
   int* item_inst;  // instance of each work item
   int item_cap;
   float* pool;   // all planes
-  double* scal;  // count x 4
+  double* scal;  // count x kBatchScal
   int total_items, grid_wgs;
   hipStream_t stream;
   hipGraph_t graph;
@@ -109,17 +145,15 @@ static void batch_drop_graph(ast_batch_t* B) {
 static int batch_layout(ast_batch_t* B) {
   int item = 0;
   for (auto& I : B->h) {
-    const StripShape sh = strip_shape(I.g, I.krows);
-    I.nbands = sh.nbands;
-    I.nsg = sh.nsg;
+    I.nbands = (I.g.N + WOUT - 1) / WOUT;
+    I.items = (int)strip_groups(I.g, I.krows);
     I.first_item = item;
-    item += sh.nbands * sh.nsg;
+    item += I.items;
   }
   B->total_items = item;
   std::vector<int> map(item);
   for (int k = 0; k < B->count; k++) {
-    const int n = B->h[k].nbands * B->h[k].nsg;
-    for (int q = 0; q < n; q++) map[B->h[k].first_item + q] = k;
+    for (int q = 0; q < B->h[k].items; q++) map[B->h[k].first_item + q] = k;
   }
   if (item > B->item_cap) {
     if (B->item_inst) AST_HIP_CHECK(hipFree(B->item_inst));
@@ -133,27 +167,68 @@ static int batch_layout(ast_batch_t* B) {
   return AST_OK;
 }
 
+// The tilings of a batch before any autotuning, by the size of the whole
+// sweep.  HLL family: S strips a band in each instance, S in proportion to
+// its rows, so that all instances together give every SIMD 4 equal waves, or
+// 3, 2, 1 if the strips would be shorter than 4 rows (then strips of 4), or
+// 8-row strips taken in rounds where they would be taller than 64.  Exact
+// solver: rows by the wave rows of the sweep, as for one grid.
+static void batch_default_tiles(ast_batch_t* B) {
+  long long rows = 0;  // wave rows of the sweep
+  for (const auto& I : B->h) rows += (long long)((I.g.N + WOUT - 1) / WOUT) * I.g.M;
+  auto set = [&](auto tile) {
+    bool fits = true;
+    for (auto& I : B->h) {
+      I.krows = tile(I.g.M);
+      fits = fits && strip_fits(I.g, tallest_strip(I.g.M, I.krows));
+    }
+    return fits;
+  };
+  if (B->method == AST_EXACT) {
+    const int r = rows <= 9400 ? 1 : rows <= 20000 ? 2 : rows <= 100000 ? 4 : 8;
+    if (set([&](int) { return r; })) return;
+  }
+  for (int waves = 4; waves >= 1 && B->method != AST_EXACT; waves--) {
+    const double h = (double)rows / (1024.0 * waves);
+    if (h > 60.0) break;
+    if (h < 4.0) continue;
+    bool ok = set([&](int M) { return -std::max(1, (int)(M / h)); });
+    for (auto& I : B->h) ok = ok && (shortest_strip(I.g.M, I.krows) >= 4 || I.g.M < 8);
+    if (ok) return;
+  }
+  const int r = rows < 4 * 16 * 1024 ? 4 : 8;
+  set([&](int) { return r; });
+}
+
 template <int METHOD>
-static int launch_batch(ast_batch_t* B, int from) {
+static int launch_batch(ast_batch_t* B, int from, int j) {
   const int g = std::min(B->grid_wgs, B->total_items);
   hipLaunchKernelGGL(batch_step_kernel<METHOD>, dim3(g), dim3(NT), 0, B->stream, B->d,
-                     B->item_inst, B->total_items, from);
+                     B->item_inst, B->total_items, from, j);
   AST_LAUNCH_CHECK("ast_batch step launch");
   return AST_OK;
 }
 
-static int batch_step(ast_batch_t* B, int from, bool advance_time) {
-  int rc;
+// step j of a run, from plane `from`
+static int batch_step(ast_batch_t* B, int from, int j) {
   switch (B->method) {
-    case AST_HLL: rc = launch_batch<AST_HLL>(B, from); break;
-    case AST_HLLC: rc = launch_batch<AST_HLLC>(B, from); break;
-    case AST_HLLC_A: rc = launch_batch<AST_HLLC_A>(B, from); break;
-    default: rc = launch_batch<AST_EXACT>(B, from); break;
+    case AST_HLL: return launch_batch<AST_HLL>(B, from, j);
+    case AST_HLLC: return launch_batch<AST_HLLC>(B, from, j);
+    case AST_HLLC_A: return launch_batch<AST_HLLC_A>(B, from, j);
+    default: return launch_batch<AST_EXACT>(B, from, j);
   }
-  if (rc != AST_OK || !advance_time) return rc;
-  hipLaunchKernelGGL(batch_time_kernel, dim3((B->count + 63) / 64), dim3(64), 0, B->stream, B->d,
-                     B->count);
-  AST_LAUNCH_CHECK("ast_batch time launch");
+}
+
+// a run of n steps from plane `from`, closed
+static int batch_steps(ast_batch_t* B, int from, int n) {
+  if (n < 1) return AST_OK;
+  for (int j = 0; j < n; j++) {
+    const int rc = batch_step(B, from ^ (j & 1), j);
+    if (rc != AST_OK) return rc;
+  }
+  hipLaunchKernelGGL(batch_close_kernel, dim3((B->count + 63) / 64), dim3(64), 0, B->stream, B->d,
+                     B->count, n - 1);
+  AST_LAUNCH_CHECK("ast_batch close launch");
   return AST_OK;
 }
 
@@ -186,7 +261,7 @@ extern "C" int ast_batch_create(int count, const ast_grid_t* grids, int method, 
   B->method = method;
   B->h.resize(count);
   hipError_t e = hipMalloc((void**)&B->pool, floats * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&B->scal, sizeof(double) * 4 * count);
+  if (e == hipSuccess) e = hipMalloc((void**)&B->scal, sizeof(double) * kBatchScal * count);
   if (e == hipSuccess) e = hipMalloc((void**)&B->d, sizeof(BatchInst) * count);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -196,7 +271,7 @@ extern "C" int ast_batch_create(int count, const ast_grid_t* grids, int method, 
     delete B;
     return ast_hip_fail(e, "ast_batch_create: allocation");
   }
-  std::vector<double> init(4 * count, 0.0);
+  std::vector<double> init(kBatchScal * (size_t)count, 0.0);
   size_t off = 0;
   for (int k = 0; k < count; k++) {
     BatchInst& I = B->h[k];
@@ -208,12 +283,11 @@ extern "C" int ast_batch_create(int count, const ast_grid_t* grids, int method, 
       I.plane[q] = (float2*)(B->pool + off);
       off += pl;
     }
-    I.scal = B->scal + 4 * k;
-    I.krows = 8;
-    init[4 * k + 0] = 1e7;  // kernel.cu:3321-3324
-    init[4 * k + 1] = 1e-9;
-    init[4 * k + 2] = 0.0;
-    init[4 * k + 3] = 0.0;
+    I.scal = B->scal + kBatchScal * (size_t)k;
+    double* v = &init[kBatchScal * (size_t)k];
+    v[0] = 1e7;  // kernel.cu:3321-3324
+    v[1] = 1e-9;
+    for (int s = 0; s < 3; s++) v[kBatchSlot + s] = kSlotEmpty;
   }
   AST_HIP_CHECK(hipMemcpy(B->scal, init.data(), sizeof(double) * init.size(), hipMemcpyHostToDevice));
   // co-resident capacity: workgroups per CU x CUs
@@ -230,6 +304,7 @@ extern "C" int ast_batch_create(int count, const ast_grid_t* grids, int method, 
   }
   if (oe != hipSuccess || per_cu < 1) per_cu = 1;
   B->grid_wgs = cus * per_cu;
+  batch_default_tiles(B);
   int rc = batch_layout(B);
   if (rc != AST_OK) {
     ast_batch_destroy(B);
@@ -323,14 +398,13 @@ extern "C" int ast_batch_set_time(ast_batch_t* B, int k, double T, double T_do, 
 }
 
 // Per grid shape, tries each candidate strip height while the other shapes
-// keep theirs, timing `reps` launches of the whole batch step kernel (no
-// time advance: the launches read the current planes and write the spare
-// ones); keeps the fastest.  Time scalars are restored.
+// keep theirs, timing `reps` launches of the whole batch step kernel (the
+// first step of a run each: the launches read the current planes and write
+// the spare ones); keeps the fastest.  Time scalars are restored.
 extern "C" int ast_batch_autotune(ast_batch_t* B, int reps) {
   if (!B) return ast_fail(AST_ERR_ARG, "ast_batch_autotune: null batch");
   if (reps < 1) reps = 5;
-  static const int cand[] = {4, 8, 12, 16};  // multiples of 4 take the fast strip path
-  std::vector<double> saved(4 * B->count);
+  std::vector<double> saved(kBatchScal * (size_t)B->count);
   AST_HIP_CHECK(hipStreamSynchronize(B->stream));
   AST_HIP_CHECK(hipMemcpy(saved.data(), B->scal, sizeof(double) * saved.size(), hipMemcpyDeviceToHost));
   std::map<std::pair<int, int>, std::vector<int>> shapes;
@@ -341,13 +415,16 @@ extern "C" int ast_batch_autotune(ast_batch_t* B, int reps) {
   for (auto& sh : shapes) {
     int best = B->h[sh.second[0]].krows;
     float best_t = 1e30f;
-    for (int kr : cand) {
+    // the tiling it has, and strips of 4 rows (multiples take the fast strip
+    // path; the exact solver 1) and up
+    const int now = best, low = B->method == AST_EXACT ? 1 : 4;
+    for (int kr : {now, low, 2 * low, 8, 12, 16}) {
       for (int k : sh.second) B->h[k].krows = kr;
       int rc = batch_layout(B);
       if (rc != AST_OK) return rc;
       for (int r = -1; r < reps; r++) {
         if (r == 0) AST_HIP_CHECK(hipEventRecord(e0, B->stream));
-        if ((rc = batch_step(B, B->cur, false)) != AST_OK) return rc;
+        if ((rc = batch_step(B, B->cur, 0)) != AST_OK) return rc;
       }
       AST_HIP_CHECK(hipEventRecord(e1, B->stream));
       AST_HIP_CHECK(hipEventSynchronize(e1));
@@ -371,8 +448,7 @@ extern "C" int ast_batch_autotune(ast_batch_t* B, int reps) {
 static int batch_build_graph(ast_batch_t* B) {
   batch_drop_graph(B);
   AST_HIP_CHECK(hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
-  int rc = batch_step(B, 0, true);
-  if (rc == AST_OK) rc = batch_step(B, 1, true);
+  const int rc = batch_steps(B, 0, kBatchChunk);
   hipGraph_t gr = nullptr;
   hipError_t e = hipStreamEndCapture(B->stream, &gr);
   if (rc != AST_OK) {
@@ -390,26 +466,23 @@ extern "C" int ast_batch_run(ast_batch_t* B, int steps, int use_graph) {
   if (!B) return ast_fail(AST_ERR_ARG, "ast_batch_run: null batch");
   if (steps < 0) return ast_fail(AST_ERR_ARG, "ast_batch_run: steps %d", steps);
   int rc;
-  if (!use_graph) {
-    for (int k = 0; k < steps; k++) {
-      if ((rc = batch_step(B, B->cur, true)) != AST_OK) return rc;
-      B->cur ^= 1;
-    }
-    return AST_OK;
-  }
-  if (B->cur == 1 && steps > 0) {
-    if ((rc = batch_step(B, 1, true)) != AST_OK) return rc;
-    B->cur = 0;
+  auto direct = [&](int n) {  // n steps on plain launches
+    if ((rc = batch_steps(B, B->cur, n)) != AST_OK) return false;
+    B->cur ^= n & 1;
+    return true;
+  };
+  if (!use_graph) return direct(steps) ? AST_OK : rc;
+  // the captured run starts from plane 0
+  if (B->cur == 1 && steps > kBatchChunk) {
+    if (!direct(1)) return rc;
     steps--;
   }
-  if (steps >= 2 && !B->graph_ok)
-    if ((rc = batch_build_graph(B)) != AST_OK) return rc;
-  for (int k = 0; k + 1 < steps; k += 2) AST_HIP_CHECK(hipGraphLaunch(B->exec, B->stream));
-  if (steps & 1) {
-    if ((rc = batch_step(B, 0, true)) != AST_OK) return rc;
-    B->cur = 1;
+  if (steps >= kBatchChunk && B->cur == 0) {
+    if (!B->graph_ok && (rc = batch_build_graph(B)) != AST_OK) return rc;
+    for (; steps >= kBatchChunk; steps -= kBatchChunk)
+      AST_HIP_CHECK(hipGraphLaunch(B->exec, B->stream));
   }
-  return AST_OK;
+  return direct(steps) ? AST_OK : rc;
 }
 
 extern "C" int ast_batch_sync(ast_batch_t* B) {

@@ -79,17 +79,12 @@ static int default_tile(const ast_grid_t& g, int method) {
     tile = rows <= 9400 ? 1 : rows <= 20000 ? 2 : rows <= 100000 ? 4 : 8;
   } else {
     auto strips = [&](long long waves) { return waves * 1024 / nbands; };
-    // the shortest strip of S a band: its middle ones (strip_rows)
-    auto shortest = [&](long long S) {
-      const long long e = std::max(4LL, (g.M / S + 2) / 4 * 4);
-      return S >= 3 && g.M - 2 * e >= S - 2 ? (g.M - 2 * e) / (S - 2) : g.M / S;
-    };
     long long waves = 4;
     while (strips(waves) < 1 || tallest_strip(g.M, (int)-std::min(strips(waves), (long long)g.M)) > 64)
       waves += 4;
     for (; waves >= 1; waves -= waves > 4 ? 4 : 1) {
       const long long S = strips(waves);
-      if (S >= 1 && S <= g.M && shortest(S) >= 4) {
+      if (S >= 1 && S <= g.M && shortest_strip(g.M, (int)-S) >= 4) {
         tile = (int)-S;
         break;
       }

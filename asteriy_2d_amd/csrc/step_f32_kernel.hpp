@@ -108,13 +108,7 @@ int launch_f32(const ast_grid_t& g, const Consts& c, const ExactCtx& ex, const f
                       const SrcF* src, const double* TT) {
   // krows > 0: strips of krows rows; krows = -S: S strips per band (strip_rows)
   const int nbands = (g.N + WOUT - 1) / WOUT;
-  long long nwg;
-  if (krows > 0) {
-    const int nstrips = (g.M + krows - 1) / krows;
-    nwg = (long long)nbands * ((nstrips + WPB - 1) / WPB);
-  } else {
-    nwg = ((long long)nbands * -(long long)krows + WPB - 1) / WPB;
-  }
+  const long long nwg = strip_groups(g, krows);
   if (nwg > 0x7fffffffLL / NT) return ast_fail(AST_ERR_SIZE, "ast_step_f32: grid too large");
   const unsigned grid = (unsigned)nwg;
   const SrcF none{nullptr, nullptr, nullptr, nullptr, 0.f, 0.f};

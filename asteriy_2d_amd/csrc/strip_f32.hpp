@@ -136,18 +136,6 @@ static inline Consts make_consts(const ast_grid_t& g) {
   return c;
 }
 
-// Strip heights / band counts of one grid.
-struct StripShape {
-  int nbands, krows, nsg;
-};
-static inline StripShape strip_shape(const ast_grid_t& g, int krows) {
-  StripShape sh;
-  sh.krows = krows;
-  sh.nbands = (g.N + WOUT - 1) / WOUT;
-  const int nstrips = (g.M + krows - 1) / krows;
-  sh.nsg = (nstrips + WPB - 1) / WPB;
-  return sh;
-}
 // The tallest strip of a tiling (strip_rows): tile > 0 rows, or for S = -tile
 // strips per band the end strips (M/S rounded to a multiple of 4) or the
 // others (ceil of what is left over them).
@@ -156,6 +144,22 @@ static inline int tallest_strip(int M, int tile) {
   const int S = -tile, e = std::max(4, (M / S + 2) / 4 * 4), mid = M - 2 * e;
   if (S >= 3 && mid >= S - 2) return std::max(e, (mid + S - 3) / (S - 2));
   return (M + S - 1) / S;
+}
+// The shortest strip but the last of a tiling (S strips a band: their
+// middle ones).
+static inline int shortest_strip(int M, int tile) {
+  if (tile > 0) return tile;
+  const int S = -tile, e = std::max(4, (M / S + 2) / 4 * 4), mid = M - 2 * e;
+  return S >= 3 && mid >= S - 2 ? mid / (S - 2) : M / S;
+}
+// Workgroups of WPB waves that a tiling gives a grid.
+static inline long long strip_groups(const ast_grid_t& g, int tile) {
+  const long long nbands = (g.N + WOUT - 1) / WOUT;
+  if (tile > 0) {
+    const long long strips = (g.M + tile - 1) / tile;
+    return nbands * ((strips + WPB - 1) / WPB);
+  }
+  return (nbands * -(long long)tile + WPB - 1) / WPB;
 }
 // Do the buffer ranges of a strip fit one resource?  (rows krows + 4 of N
 // float2 cells)
