@@ -35,6 +35,7 @@ int ast_step_f64_rows(const ast_grid_t* g, const double* s, const double* u, dou
                       double* u2, double* T, const double* T_do, const double* TT, int method,
                       ast_stats_t* stats, int rows, const ast::StepTime* tm,
                       const ast_sources_t* src, void* stream);
+int ast_step_f64_default_tile(const ast_grid_t* g, int method);
 int ast_tile_rows_setting(void);
 
 #define CK(call)                                              \
@@ -48,7 +49,7 @@ struct ast_sim {
   int precision;  // 0: FP64 planes, 1: FP32 planes
   int method;
   int krows;   // FP32 strip tiling (rows per strip, -S strips per band, 0: by size)
-  int rows64;  // FP64 rows per strip (0: the kernel's default)
+  int rows64;  // FP64 strip tiling (rows per strip, -S strips per band, 0: by size)
   size_t cells;
   void* plane[4];  // s0, u0, s1, u1
   int cur;         // 0: state in (s0,u0); 1: in (s1,u1)
@@ -438,13 +439,16 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
   // 5 waves of (nearly) equal height, S strips per band with S * bands
   // waves (a wave strip has 60 output columns; a CU has 4 SIMDs); the FP32
   // exact solver's strips are of 1 to 8 rows (its waves differ too much for
-  // taller ones), the FP64 step's of 1 to 32
+  // taller ones), the FP64 step's of 1 to 32 or the tiling chosen by size
   int dflt[8] = {4, 8, 12, 16};
   static const int dflt_exact[5] = {1, 2, 3, 4, 8};
-  static const int dflt64[11] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
+  int dflt64[12] = {0, 1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
+  bool own64 = false;
   if ((!candidates || ncand <= 0) && S->precision == 0) {
+    dflt64[0] = ast_step_f64_default_tile(&S->g, S->method);
+    own64 = true;
     candidates = dflt64;
-    ncand = 11;
+    ncand = 12;
   }
   if ((!candidates || ncand <= 0) && S->method == AST_EXACT) {
     candidates = dflt_exact;
@@ -492,7 +496,7 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
                                    nullptr, kr, &tm, sources64(S), S->stream);
   };
   auto valid = [&](int kr) {
-    if (S->precision == 0) return kr >= 1 && kr <= 4096;
+    if (S->precision == 0) return (own64 || kr >= 1) && kr <= 4096;
     return !(kr == 0 || kr > 1024 || (kr < 0 && -kr > S->g.M));
   };
   const int n = ncand;
@@ -546,7 +550,8 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
     S->rows64 = best;
     drop_graph(S);
   }
-  if (best_rows) *best_rows = best;
+  // an FP64 tiling of equal strips is reported by their height
+  if (best_rows) *best_rows = S->precision == 0 && best < 0 ? (S->g.M - best - 1) / -best : best;
   if (best_us) *best_us = best_t;
   return AST_OK;
 }

@@ -243,10 +243,34 @@ struct StepArgs {
   const double* nn2;
   const double* nn3;
   double kmom, ken;
-  int rows;    // rows per strip
+  int rows;    // rows per strip, or -S strips per band (strip_of)
   int nbands;  // bands of WOUT columns
   int nwg;     // workgroups
 };
+
+// The band and rows [m0, m1) of wave `wave` of workgroup `wg` (wave-uniform).
+// rows > 0: strips of `rows` rows, WPB of them stacked per workgroup.  rows =
+// -S: every band cut into S strips of equal height (to one row), the waves
+// of all workgroups numbered band by band, so that the launch can hold
+// exactly the waves that are resident at once; waves past the last band get
+// no rows (m0 = M).
+AST_DEV void strip_of(int M, int nbands, int rows, int wg, int wave, int& band, int& m0, int& m1) {
+  if (rows > 0) {
+    band = wg % nbands;
+    m0 = ((wg / nbands) * WPB + wave) * rows;
+    m1 = min(m0 + rows, M);
+  } else {
+    const int S = -rows, gw = wg * WPB + wave;
+    band = gw / S;
+    const int k = gw - band * S, h = M / S, r = M - h * S;
+    m0 = k * h + min(k, r);
+    m1 = m0 + h + (k < r ? 1 : 0);
+    if (band >= nbands) {
+      band = nbands - 1;
+      m0 = m1 = M;
+    }
+  }
+}
 
 // G: the gas, with its order 1/gm compiled in (the exact solver) or not.
 // Three waves a SIMD; the exact solver with the general power (232 VGPRs)
@@ -265,9 +289,8 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
   // wave index made explicitly uniform: rows and the loop stay scalar
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wg = xcd_tile(blockIdx.x, A.nwg);
-  const int band = wg % A.nbands;
-  const int m0 = ((wg / A.nbands) * WPB + wave) * A.rows;
-  const int m1 = min(m0 + A.rows, g.M);
+  int band, m0, m1;
+  strip_of(g.M, A.nbands, A.rows, wg, wave, band, m0, m1);
   const int n = band * WOUT + lane - 2;
   const bool out_col = (lane >= 2) & (lane < 2 + WOUT) & (n < g.N);
   // the west face of this lane's column is a face of an output cell
@@ -467,6 +490,14 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
       }
     } else {
       for (int m = m0; m < m1; m += 4) {
+        // wave priority falls with the fraction of the strip done, so that
+        // the waves of a SIMD end together (a SIMD issues for its oldest
+        // wave first, and the last would run alone)
+        const int q = (4 * (m - m0)) / (m1 - m0);  // wave-uniform, 0..3
+        if (q == 0) __builtin_amdgcn_s_setprio(3);
+        else if (q == 1) __builtin_amdgcn_s_setprio(2);
+        else if (q == 2) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(0);
         row(std::integral_constant<int, 0>{}, m);
         if (m + 1 >= m1) break;
         row(std::integral_constant<int, 1>{}, m + 1);
@@ -491,49 +522,6 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
   }
   block_min_uniform<NT>(tmin, red, A.kt.cur ? A.kt.cur : A.T, A.kt.cur ? A.kt.nslots : 0);
   if constexpr (STATS) block_counters_to(cnt, redc, A.stats);
-}
-
-// The default rows per strip (ast_step_f64_rows, rows = 0).  A wave's row is
-// one chain of dependent FP64 operations: 1.4 us a row for a wave alone on
-// its SIMD, 1.07 us of a SIMD's time from two waves on (HLLC); a strip costs
-// about 1.5 rows more than it holds (its south face, the first fetches).  So
-// small grids want one-row strips, which spread the chains over the chip,
-// and large ones taller strips in whole rounds of the 3 x 1024 waves that
-// are resident.  The rule takes the height with the least (rows + 1.5) x n,
-// n the load of a SIMD in waves fitted to the measured times: 1.3 / 2.15 /
-// 2.8 where one, two or three waves a SIMD all run at once, beyond that 0.8
-// of the mean count plus 0.4 and 0.6 of what the last round leaves empty.
-// Measured, us a step (HLLC; rows of the rule / the fixed 6 rows before):
-// 256x128 8.0 (1) / 14.7, 512x256 11.1 (3) / 15.2, 1024x512 19.5 (5) / 21.5,
-// 1500x750 29.7 (10) / 33.5, 2048x1024 45.7 (6), 4096x2048 148.4 (16) / 162.3.
-// The exact solver's rows differ by tens of times between waves (its
-// patterns and iterations diverge), so its strips stay short until 16384 of
-// them share the load: 256x128 26.0 (1) / 95.7, 1500x750 56.6 (2) / 106.4,
-// 2048x1024 82.1 (3) / 109.1, 4096x2048 about 243 (9) / 246.5.
-static int default_rows(const ast_grid_t& g, int method) {
-  const long long nbands = (g.N + WOUT - 1) / WOUT;
-  if (method == AST_EXACT) {
-    const long long rows = (nbands * g.M + 16383) / 16384;
-    return (int)std::min(rows, 32LL);
-  }
-  int best = 1;
-  double cost = INFINITY;
-  for (int rows = 1; rows <= 32; rows++) {
-    const long long strips = (g.M + rows - 1) / rows;
-    const double waves = (double)(nbands * ((strips + WPB - 1) / WPB) * WPB);
-    const double per = waves / 1024.0;
-    const double rounds = waves / 3072.0;
-    const double n = per <= 1.0   ? 1.3
-                     : per <= 2.0 ? 2.15
-                     : per <= 3.0 ? 2.8
-                                  : 0.8 * per + 0.4 + 0.6 * (ceil(rounds) - rounds);
-    const double c = n * (rows + 1.5);
-    if (c < cost) {
-      cost = c;
-      best = rows;
-    }
-  }
-  return best;
 }
 
 template <int METHOD, int GEOM, bool WINDOW>
@@ -565,7 +553,44 @@ static int launch(const StepArgs& a, bool stats, bool window, hipStream_t st) {
 }  // namespace s64
 }  // namespace ast
 
-// The step with a given strip height (rows > 0; 0 = the default) and
+// The default strip tiling (ast_step_f64_rows, rows = 0; strip_of's
+// convention).  A wave's row is one chain of dependent FP64 operations, and a
+// SIMD holds three waves, so the launch is cut into S equal strips a band
+// that give every SIMD the same 1, 2 or 3 waves, or whole rounds of 3: few
+// waves of many rows leave the chains exposed, many short strips pay their
+// prologue (south face, first fetches) and the rounds' changes.  The rule
+// takes the count with the least time fitted to the measured ones (us, h the
+// tallest strip's rows): 1.5 h + 6, 1.85 h + 8 and 2.7 h + 8 for 1, 2 and 3
+// waves a SIMD, 2.6 r h + 4 r + 4 for r rounds of 3.
+// Measured, us a step (HLLC; the rule / 6-row strips): 256x128 8.0 / 14.7,
+// 512x256 10.7 / 15.7, 1024x512 17.5 / 19.4, 1500x750 26.5 / 34.3, 2048x1024
+// 39.3 / 46.6, 8192x400 60.7 / 73.0, 4096x2048 135 / 166, 32000x400 216 / 257.
+// The exact solver's rows differ by tens of times between waves (its
+// patterns and iterations diverge), so its strips stay short until 16384 of
+// them share the load: 256x128 26.0 (1 row) / 95.7, 1500x750 56.6 (2) / 106.4,
+// 2048x1024 82.1 (3) / 109.1, 4096x2048 about 243 (9) / 246.5.
+int ast_step_f64_default_tile(const ast_grid_t* g, int method) {
+  const long long nbands = (g->N + ast::s64::WOUT - 1) / ast::s64::WOUT, M = g->M;
+  if (method == AST_EXACT) return (int)std::min((nbands * M + 16383) / 16384, 32LL);
+  int best = 32;
+  double cost = INFINITY;
+  for (int waves = 1; waves <= 192; waves += waves < 3 ? 1 : 3) {
+    const long long S = std::min(M, waves * 1024 / nbands);
+    if (S < 1) continue;
+    const double h = (double)((M + S - 1) / S), r = waves / 3;
+    const double c = waves == 1   ? 1.5 * h + 6.0
+                     : waves == 2 ? 1.85 * h + 8.0
+                     : waves == 3 ? 2.7 * h + 8.0
+                                  : 2.6 * r * h + 4.0 * r + 4.0;
+    if (c < cost) {
+      cost = c;
+      best = (int)-S;
+    }
+  }
+  return best;
+}
+
+// The step with a given strip tiling (strip_of; 0 = the default) and
 // optional neutral-H source planes (src may be null).  tm (may be null): the
 // runtime's time protocol (time_slots.h); null: the reference protocol (the
 // step lowers *T, dt is *T_do).
@@ -580,8 +605,8 @@ int ast_step_f64_rows(const ast_grid_t* g, const double* s, const double* u, dou
     return ast_fail(AST_ERR_ARG, "ast_step_f64: null state or time pointer");
   if (s == s2 || u == u2 || s == u2 || u == s2)
     return ast_fail(AST_ERR_ARG, "ast_step_f64: output planes must not alias the input planes");
-  if (rows == 0) rows = default_rows(*g, method);
-  if (rows < 1 || rows > 4096) return ast_fail(AST_ERR_ARG, "ast_step_f64: %d rows per strip", rows);
+  if (rows == 0) rows = ast_step_f64_default_tile(g, method);
+  if (rows == 0 || rows > 4096 || rows < -g->M) return ast_fail(AST_ERR_ARG, "ast_step_f64: %d rows per strip", rows);
   StepArgs a;
   a.g = *g;
   a.gas = ast::d64::make_gas(g->gamma);
@@ -611,8 +636,9 @@ int ast_step_f64_rows(const ast_grid_t* g, const double* s, const double* u, dou
     return ast_fail(AST_ERR_ARG, "ast_step_f64: a source plane aliases a state plane");
   a.rows = rows;
   a.nbands = (g->N + WOUT - 1) / WOUT;
-  const long long strips = (g->M + rows - 1) / rows;
-  const long long nwg = (long long)a.nbands * ((strips + WPB - 1) / WPB);
+  const long long nwg = rows > 0
+      ? (long long)a.nbands * (((g->M + rows - 1) / rows + WPB - 1) / WPB)
+      : ((long long)a.nbands * -(long long)rows + WPB - 1) / WPB;
   if (nwg > 0x7fffffffLL) return ast_fail(AST_ERR_SIZE, "ast_step_f64: grid too large");
   a.nwg = (int)nwg;
   const bool window = !(g->ho_lo == -INFINITY && g->ho_hi == INFINITY);

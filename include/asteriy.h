@@ -421,8 +421,9 @@ int ast_sim_set_tile_rows(ast_sim_t* sim, int rows);
 /* Times the step for each candidate tiling (NULL = a default list: FP32 4,
  * 8, 12, 16 rows and the tilings -S that give every SIMD 2, 3, 4 or 5 equal
  * waves, with the exact solver 1, 2, 3, 4, 8 rows; FP64 1 to 6, 8, 12, 16,
- * 24, 32 rows), keeps the fastest; reports it (may be NULL).  State and time
- * are left unchanged. */
+ * 24, 32 rows and the tiling chosen by size, which is reported by its rows),
+ * keeps the fastest; reports it (may be NULL).  State and time are left
+ * unchanged. */
 int ast_sim_autotune(ast_sim_t* sim, const int* candidates, int ncand, int reps,
                      int* best_rows, float* best_us);
 /* The simulation's stream (hipStream_t) for event timing. */
