@@ -154,30 +154,16 @@ AST_DEV uint32_t wave_sum(uint32_t v) {
   return v;
 }
 
-// Lowers *T to the block minimum of tmin.  Positive IEEE doubles order like
-// their bit patterns, so one 64-bit atomicMin on the bits gives the exact,
-// order-independent minimum (the reference's store, kernel.cu:3013-3017, is
-// racy).  `red` is LDS of at least nwaves doubles.
-template <int NT>
-AST_DEV void block_min_to(double tmin, double* red, double* T) {
-  constexpr int NW = NT / 64;
-  tmin = wave_min(tmin);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) red[wave] = tmin;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = red[0];
-#pragma unroll
-    for (int i = 1; i < NW; i++) t = fmin(t, red[i]);
-    if (t < INFINITY)
-      atomicMin(reinterpret_cast<unsigned long long*>(T), (unsigned long long)__double_as_longlong(t));
-  }
-}
-
-// block_min_to for a tmin that is already uniform across each wave.  With
-// nslots > 0, T is a set of dt slots (time_slots.h) and workgroup b lowers
-// slot (b mod nslots), so that no single address takes every workgroup's
-// atomic; the time advance folds the slots.
+// Lowers *T to the block minimum of tmin, which is uniform across each wave.
+// Positive IEEE doubles order like their bit patterns, so one 64-bit
+// atomicMin on the bits gives the exact, order-independent minimum (the
+// reference's store, kernel.cu:3013-3017, is racy).  `red` is LDS of at least
+// nwaves doubles.  With nslots > 0, T is a set of dt slots (time_slots.h) and
+// workgroup b lowers slot (b mod nslots), so that no single address takes
+// every workgroup's atomic; the time advance folds the slots.  Without
+// slots the atomics of one address follow each other (about 17 ns each, and
+// workgroups of equal strips end together), so a workgroup looks first
+// whether *T is already as low, as it is for nearly all.
 template <int NT>
 AST_DEV void block_min_uniform(double tmin, double* red, double* T, int nslots) {
   constexpr int NW = NT / 64;
@@ -189,8 +175,11 @@ AST_DEV void block_min_uniform(double tmin, double* red, double* T, int nslots) 
 #pragma unroll
     for (int i = 1; i < NW; i++) t = fmin(t, red[i]);
     double* dst = nslots > 0 ? T + kSlotStride * (int)(blockIdx.x % (unsigned)nslots) : T;
-    if (t < INFINITY)
-      atomicMin(reinterpret_cast<unsigned long long*>(dst), (unsigned long long)__double_as_longlong(t));
+    auto* word = reinterpret_cast<unsigned long long*>(dst);
+    const auto bits = (unsigned long long)__double_as_longlong(t);
+    const bool lower = nslots > 0 || __hip_atomic_load(word, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT) > bits;
+    if (t < INFINITY && lower) atomicMin(word, bits);
   }
 }
 
