@@ -34,8 +34,9 @@ struct LaneStats {
   }
 };
 
+template <int NT>
 AST_DEV void block_stats_to(const LaneStats& c, uint32_t* red, ast_stats_t* stats) {
-  constexpr int NW = FNT / 64;
+  constexpr int NW = NT / 64;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int k = 0; k < 10; k++) {
     const uint32_t w = wave_sum(c.v[k]);
@@ -89,7 +90,7 @@ __global__ __launch_bounds__(FNT) void flux_kernel(size_t n, const double* __res
     if (METHOD == AST_EXACT) st.add(ei);
     store_face<METHOD>(out, n, i, n1, n2, f, krad, UU);
   }
-  if (METHOD == AST_EXACT && stats != nullptr) block_stats_to(st, redi, stats);
+  if (METHOD == AST_EXACT && stats != nullptr) block_stats_to<FNT>(st, redi, stats);
 }
 
 // The exact solver on pattern-sorted faces: each workgroup classifies a tile
@@ -100,13 +101,18 @@ __global__ __launch_bounds__(FNT) void flux_kernel(size_t n, const double* __res
 // depends only on its own data.  The tile's faces stay in LDS (32 KiB) from
 // the coalesced classifying loads on: the solve reads its permuted faces
 // there and leaves its fluxes in their place, and the tile's fluxes go out
-// with coalesced stores.
-// Bound by the FP64 issue of the solvers, 104 B/face: 2^22 faces in 191 us
-// (22 Gfaces/s, 2.3 TB/s; 701 us with pow, the evaluated bisection and the
-// sorted faces re-read from global memory).  512-face tiles, one a
-// workgroup: four workgroups (of 34 KiB of LDS) and 16 waves a CU.
+// with coalesced stores.  The waves take 64 sorted faces at a time, the
+// costliest patterns first, so that they reach the tile's end together.
+// Bound by the FP64 issue of the solvers, 104 B/face: 2^22 faces in 185 us
+// (23 Gfaces/s, 2.4 TB/s; 191 us with each wave's two groups of faces fixed,
+// 701 us with pow, the evaluated bisection and the sorted faces re-read from
+// global memory).  512-face tiles, one a workgroup: four workgroups (of 34
+// KiB of LDS) and 16 waves a CU; measured at 2^22 faces with fixed groups,
+// threads x faces a thread: 256x2 191, 512x2 198, 256x1 223, 512x1 241,
+// 256x4 261, 1024x1 272 us.
+constexpr int SORT_NT = 256;
 constexpr int SORT_PER = 2;
-constexpr int STILE = FNT * SORT_PER;
+constexpr int STILE = SORT_NT * SORT_PER;
 
 // the face's eight words in the frame of the normal (n1, n2)
 AST_DEV void face_frame(const double* w, double n1, double n2, PrimD& L, PrimD& R) {
@@ -117,14 +123,14 @@ AST_DEV void face_frame(const double* w, double n1, double n2, PrimD& L, PrimD& 
 // STATS: the variant that counts (the counters hold ten registers a lane).
 // G: the gas, with its order 1/gm compiled in or not.
 template <class G, bool STATS>
-__global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const double* __restrict__ in,
+__global__ __launch_bounds__(SORT_NT) void exact_sorted_kernel(size_t n, const double* __restrict__ in,
                                                            double n1, double n2, double krad,
                                                            GasD gas0, double* __restrict__ out,
                                                            ast_stats_t* stats) {
   const G gas(gas0);
-  __shared__ uint32_t redi[(FNT / 64) * 10];
+  __shared__ uint32_t redi[(SORT_NT / 64) * 10];
   __shared__ unsigned short perm[STILE];
-  __shared__ int cnt[kPatternKeys + 1], cur[kPatternKeys + 1];
+  __shared__ int cnt[kPatternKeys + 1], cur[kPatternKeys + 1], next;
   __shared__ double stage[8][STILE];  // the tile's faces, then (5 planes) its fluxes
   LaneStats st;
   if constexpr (STATS) st.clear();
@@ -133,11 +139,12 @@ __global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const doubl
     const size_t base = tile * STILE;
     const int nv = (int)min((size_t)STILE, n - base);
     if (threadIdx.x <= kPatternKeys) cnt[threadIdx.x] = 0;
+    if (threadIdx.x == 0) next = 0;
     __syncthreads();
     int key[SORT_PER];
 #pragma unroll
     for (int j = 0; j < SORT_PER; j++) {
-      const int li = j * FNT + threadIdx.x;
+      const int li = j * SORT_NT + threadIdx.x;
       key[j] = kPatternKeys;  // past the end of the batch
       if (li < nv) {
         double w[8];
@@ -148,7 +155,10 @@ __global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const doubl
         }
         PrimD L, R;
         face_frame(w, n1, n2, L, R);
-        key[j] = pattern_key(L, R, gas);
+        // the costliest pattern first: shock + rarefaction, two shocks, two
+        // rarefactions, vacuum, none
+        const int pk = pattern_key(L, R, gas);
+        key[j] = pk == 2 ? 0 : pk == 3 ? 1 : pk == 1 ? 2 : pk == 0 ? 3 : 4;
       }
       atomicAdd(&cnt[key[j]], 1);
     }
@@ -165,13 +175,16 @@ __global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const doubl
 #pragma unroll
     for (int j = 0; j < SORT_PER; j++) {
       const int slot = atomicAdd(&cur[key[j]], 1);
-      perm[slot] = (unsigned short)(j * FNT + threadIdx.x);
+      perm[slot] = (unsigned short)(j * SORT_NT + threadIdx.x);
     }
     __syncthreads();
     const int nfaces = cnt[0];
-#pragma unroll 1
-    for (int j = 0; j < SORT_PER; j++) {
-      const int pos = j * FNT + threadIdx.x;
+    for (;;) {
+      int chunk = 0;
+      if ((threadIdx.x & 63) == 0) chunk = atomicAdd(&next, 1);
+      chunk = __builtin_amdgcn_readfirstlane(chunk);
+      if (64 * chunk >= nfaces) break;  // wave-uniform
+      const int pos = 64 * chunk + (int)(threadIdx.x & 63);
       if (pos < nfaces) {
         const int li = perm[pos];
         double w[8];
@@ -195,7 +208,7 @@ __global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const doubl
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < SORT_PER; j++) {
-      const int li = j * FNT + threadIdx.x;
+      const int li = j * SORT_NT + threadIdx.x;
       if (li < nv) {
 #pragma unroll
         for (int k = 0; k < 5; k++) out[k * n + base + li] = stage[k][li];
@@ -203,7 +216,7 @@ __global__ __launch_bounds__(FNT) void exact_sorted_kernel(size_t n, const doubl
     }
     __syncthreads();  // stage, perm and the counters are reused by the next tile
   }
-  if constexpr (STATS) block_stats_to(st, redi, stats);
+  if constexpr (STATS) block_stats_to<SORT_NT>(st, redi, stats);
 }
 
 // The exact solver with per-face newton starting points and diagnostics.
@@ -232,7 +245,7 @@ __global__ __launch_bounds__(FNT) void guess_kernel(size_t n, const double* __re
       info[2 * i + 1] = (ei.pat == -9 ? -1 : ei.pat + 1) | (ei.capped ? 8 : 0);
     }
   }
-  if (stats != nullptr) block_stats_to(st, redi, stats);
+  if (stats != nullptr) block_stats_to<FNT>(st, redi, stats);
 }
 
 // HLLC with a passive scalar: 10 input planes (the 8 of load_face, Q_L,
@@ -271,7 +284,7 @@ static int launch_flux(size_t n, const double* in, double n1, double n2, double 
     const auto kernel =
         gas.n == 5 ? (stats ? exact_sorted_kernel<G5, true> : exact_sorted_kernel<G5, false>)
                    : (stats ? exact_sorted_kernel<GasD, true> : exact_sorted_kernel<GasD, false>);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(FNT), 0, stream, n, in, n1, n2, krad,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(SORT_NT), 0, stream, n, in, n1, n2, krad,
                        gas, out, stats);
     AST_LAUNCH_CHECK("ast_flux_f64 launch");
     return AST_OK;
