@@ -56,8 +56,7 @@ def _p(t):
 
 
 def _st(stream=None):
-    import torch
-    return _vp((stream or torch.cuda.current_stream()).cuda_stream)
+    return _vp(native.stream_handle(stream))
 
 
 def glorot_init(seed: int = 0) -> np.ndarray:

@@ -27,14 +27,15 @@ _STATS_WORDS = 10
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
-def _stream(stream):
-    import torch
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+def _grid(grid):
+    """The grid as the `const ast_grid_t*` argument of one call."""
+    return ctypes.byref(grid if isinstance(grid, native.CGrid) else grid.to_c())
+
+
+_stream = native.stream_handle
 
 
 def _check_state(t, dtype, cells, name):
@@ -98,7 +99,7 @@ def Kernel_TVD(grid, s, u, s2, u2, T, T_do, TT, method: int, stats=None, mlp=Non
         raise TypeError("state must be float64 or float32")
     for t, nm in ((s, "s"), (u, "u"), (s2, "s2"), (u2, "u2")):
         _check_state(t, dt, cells, nm)
-    gref = native.grid_ref(grid)
+    gref = _grid(grid)
     if dt == torch.float64:
         if mlp is not None:
             raise ValueError("the learned guess is served by the FP32 step only")
@@ -254,7 +255,7 @@ def mc_cell_exit(grid, particles, stream=None):
     t = torch.empty(n, dtype=torch.float64, device=p.device)
     mode = torch.empty(n, dtype=torch.int32, device=p.device)
     hit = torch.empty(n, dtype=torch.int32, device=p.device)
-    native.call("ast_mc_cell_exit_f64", native.grid_ref(grid), n, _ptr(p), _ptr(t), _ptr(mode),
+    native.call("ast_mc_cell_exit_f64", _grid(grid), n, _ptr(p), _ptr(t), _ptr(mode),
                 _ptr(hit), _stream(stream))
     return t, mode, hit
 
@@ -267,7 +268,7 @@ def mc_belong_point(grid, xy, stream=None):
         raise ValueError("xy must be a (2, n) float64 tensor")
     xy = xy.contiguous()
     nm = torch.empty((2, xy.shape[1]), dtype=torch.int32, device=xy.device)
-    native.call("ast_mc_belong_point_f64", native.grid_ref(grid), xy.shape[1], _ptr(xy), _ptr(nm),
+    native.call("ast_mc_belong_point_f64", _grid(grid), xy.shape[1], _ptr(xy), _ptr(nm),
                 _stream(stream))
     return nm
 
@@ -277,6 +278,6 @@ def conservation_sums(grid, s, u, stream=None):
     import torch
     work = torch.empty(int(native.load().ast_conservation_work_doubles()), dtype=torch.float64,
                        device=s.device)
-    native.call("ast_conservation_sums", native.grid_ref(grid), _ptr(s), _ptr(u),
+    native.call("ast_conservation_sums", _grid(grid), _ptr(s), _ptr(u),
                 1 if s.dtype == torch.float32 else 0, _ptr(work), _stream(stream))
     return work[:2]
