@@ -16,9 +16,14 @@
 // a = S_K in the star regions, b = S_K* in the Alfven regions (the
 // Rankine-Hugoniot chain from the side's outer state), and rotated back.
 #include "common.hpp"
+#include "flux64.hpp"
 
 namespace ast {
 namespace mhd {
+
+using d64::div64;
+using d64::rcp64;
+using d64::sqrt64;
 
 constexpr int MNT = 256;
 constexpr double kSqrt4Pi = 3.544907701811032;  // spi4, Header.h:69, as written there
@@ -50,9 +55,10 @@ AST_DEV Side load_side(const double* __restrict__ in, size_t n, size_t i, int k0
   // true divisions: the fast speed's inner root cancels for a field along
   // the normal with gamma p ~ b_n^2, where a one-ulp change of b moves c_f
   // by up to ~1e-8; dividing as the reference does keeps c_f and dt exact
-  const double bx = in[(k0 + 6) * n + i] / kSqrt4Pi;
-  const double by = in[(k0 + 7) * n + i] / kSqrt4Pi;
-  const double bz = in[(k0 + 8) * n + i] / kSqrt4Pi;
+  const double r4pi = rcp64(kSqrt4Pi);
+  const double bx = div64(in[(k0 + 6) * n + i], kSqrt4Pi, r4pi);
+  const double by = div64(in[(k0 + 7) * n + i], kSqrt4Pi, r4pi);
+  const double bz = div64(in[(k0 + 8) * n + i], kSqrt4Pi, r4pi);
   s.un = vx * f.n[0] + vy * f.n[1] + vz * f.n[2];
   s.ut = vx * f.t[0] + vy * f.t[1] + vz * f.t[2];
   s.um = vx * f.m[0] + vy * f.m[1] + vz * f.m[2];
@@ -62,10 +68,10 @@ AST_DEV Side load_side(const double* __restrict__ in, size_t n, size_t i, int k0
   const double bb = bx * bx + by * by + bz * bz;
   const double kin = (vx * vx + vy * vy + vz * vz) / 2.0;
   s.pT = s.p + bb / 2.0;
-  s.e = s.p / gas.g1 + s.r * kin + bb / 2.0;
+  s.e = div64(s.p, gas.g1) + s.r * kin + bb / 2.0;
   // c_f^2 = (gamma p + b^2 + sqrt((gamma p + b^2)^2 - 4 gamma p b_n^2)) / (2 rho)
   const double gpb = gas.g * s.p + bb;
-  s.cf = sqrt((gpb + sqrt(gpb * gpb - 4.0 * gas.g * s.p * (s.bn * s.bn))) / (2.0 * s.r));
+  s.cf = sqrt64(div64(gpb + sqrt64(gpb * gpb - 4.0 * gas.g * s.p * (s.bn * s.bn)), 2.0 * s.r));
   return s;
 }
 
@@ -101,6 +107,11 @@ struct Star {
   double r, q, v, w, bt, bm, e;
 };
 
+// Bound by HBM from 2^21 faces on (224 B/face): HLLD 2^21 faces in 99 us, 2^23
+// in 330 us (5.7 TB/s), 104 and 353 us with the compiler's divisions and
+// square roots; the chain of ~16 quotients and 6 roots is what few waves
+// expose below that (2^20: 54 / 58 us).  Three waves a SIMD (156 VGPRs): a
+// fourth spills 100 B a lane (168 us at 2^21).
 template <int METHOD>
 __global__ __launch_bounds__(MNT) void flux_mhd_kernel(size_t n, const double* __restrict__ in,
                                                        Frame fr, Gas gas,
@@ -114,17 +125,19 @@ __global__ __launch_bounds__(MNT) void flux_mhd_kernel(size_t n, const double* _
     const double SR = fmax(L.un, R.un) + fmax(L.cf, R.cf);
     const double sL = SL - L.un, sR = SR - R.un;
     const double den = sR * R.r - sL * L.r;
-    const double SM = (sR * R.r * R.un - sL * L.r * L.un - R.pT + L.pT) / den;
+    const double rden = rcp64(den);  // reciprocals that several quotients share
+    const double SM = div64(sR * R.r * R.un - sL * L.r * L.un - R.pT + L.pT, den, rden);
     const double dLR = SR - SL;
     const double dL = SL - SM, dR = SR - SM;
     // HLL averages of the field (b_n, b_t, b_m); b_n by a true division, as
     // it decides the Alfven switch |b_n| > 0.001 exactly as the reference
-    const double bn = (SR * R.bn - SL * L.bn) / dLR;
-    const double idLR = 1.0 / dLR;
+    const double rLR = rcp64(dLR), rL = rcp64(dL), rR = rcp64(dR);
+    const double bn = div64(SR * R.bn - SL * L.bn, dLR, rLR);
+    const double idLR = div64(1.0, dLR, rLR);
     const double bt = (SR * R.bt - SL * L.bt + flux_bt(L) - flux_bt(R)) * idLR;
     const double bm = (SR * R.bm - SL * L.bm + flux_bm(L) - flux_bm(R)) * idLR;
     Star sl, sr;
-    const double cL = sL / dL, cR = sR / dR;  // rho*_K / rho_K
+    const double cL = div64(sL, dL, rL), cR = div64(sR, dR, rR);  // rho*_K / rho_K
     sl.r = L.r * cL;
     sr.r = R.r * cR;
     sl.q = L.q * cL;
@@ -133,13 +146,14 @@ __global__ __launch_bounds__(MNT) void flux_mhd_kernel(size_t n, const double* _
     double v2 = 0.0, w2 = 0.0, bt2 = 0.0, bm2 = 0.0, de2L = 0.0, de2R = 0.0;
     int region;
     if constexpr (METHOD == AST_HLLD) {
-      const double PT = (sR * R.r * L.pT - sL * L.r * R.pT + L.r * R.r * sR * sL * (R.un - L.un)) / den;
+      const double PT =
+          div64(sR * R.r * L.pT - sL * L.r * R.pT + L.r * R.r * sR * sL * (R.un - L.un), den, rden);
       const double bbn = bn * bn;
       // outer star states (Gas_Dinamic.cu:1214-1259)
-      auto outer = [&](const Side& K, double sK, double dK, Star& s) {
+      auto outer = [&](const Side& K, double sK, double dK, double rK, Star& s) {
         const double tt = K.r * sK * dK - bbn;
         if (fabs(tt) >= 0.000001) {
-          const double itt = 1.0 / tt;
+          const double itt = div64(1.0, tt);
           const double f = (SM - K.un) * itt;
           const double g = (K.r * sK * sK - bbn) * itt;
           s.v = K.ut - bn * K.bt * f;
@@ -152,19 +166,21 @@ __global__ __launch_bounds__(MNT) void flux_mhd_kernel(size_t n, const double* _
           s.bt = 0.0;
           s.bm = 0.0;
         }
-        s.e = (K.e * sK + PT * SM - K.pT * K.un + bn * (vdotb(K) - (SM * bn + s.v * s.bt + s.w * s.bm))) / dK;
+        s.e = div64(K.e * sK + PT * SM - K.pT * K.un +
+                        bn * (vdotb(K) - (SM * bn + s.v * s.bt + s.w * s.bm)),
+                    dK, rK);
       };
-      outer(L, sL, dL, sl);
-      outer(R, sR, dR, sr);
+      outer(L, sL, dL, rL, sl);
+      outer(R, sR, dR, rR, sr);
       // inner (Alfven) states, shared velocity and field (Gas_Dinamic.cu:1261-1296)
-      const double qL = sqrt(sl.r), qR = sqrt(sr.r);
+      const double qL = sqrt64(sl.r), qR = sqrt64(sr.r);
       double sig = 0.0;
       if (fabs(bn) > 0.001) {
         sig = bn > 0.0 ? 1.0 : (bn < 0.0 ? -1.0 : 0.0);
-        SLs = SM - fabs(bn) / qL;
-        SRs = SM + fabs(bn) / qR;
+        SLs = SM - div64(fabs(bn), qL);
+        SRs = SM + div64(fabs(bn), qR);
       }
-      const double iqs = 1.0 / (qL + qR);
+      const double iqs = div64(1.0, qL + qR);
       v2 = (qL * sl.v + qR * sr.v + sig * (sr.bt - sl.bt)) * iqs;
       w2 = (qL * sl.w + qR * sr.w + sig * (sr.bm - sl.bm)) * iqs;
       bt2 = (qL * sr.bt + qR * sl.bt + sig * qL * qR * (sr.v - sl.v)) * iqs;
@@ -184,22 +200,27 @@ __global__ __launch_bounds__(MNT) void flux_mhd_kernel(size_t n, const double* _
       // HLLC for MHD: tangential velocity and field of the HLL average on
       // both sides, total pressure the mean of the two sides' star values
       // (Gas_Dinamic.cu:1051-1088)
-      const double z0 = (SR * R.r - SL * L.r + L.r * L.un - R.r * R.un) / dLR;
-      const double z1 = (SR * R.r * R.un - SL * L.r * L.un + (L.r * L.un * L.un + L.pT - L.bn * L.bn) -
-                         (R.r * R.un * R.un + R.pT - R.bn * R.bn)) / dLR;
-      const double z2 = (SR * R.r * R.ut - SL * L.r * L.ut + (L.r * L.un * L.ut - L.bn * L.bt) -
-                         (R.r * R.un * R.ut - R.bn * R.bt)) / dLR;
-      const double z3 = (SR * R.r * R.um - SL * L.r * L.um + (L.r * L.un * L.um - L.bn * L.bm) -
-                         (R.r * R.un * R.um - R.bn * R.bm)) / dLR;
+      const double z0 = div64(SR * R.r - SL * L.r + L.r * L.un - R.r * R.un, dLR, rLR);
+      const double z1 = div64(SR * R.r * R.un - SL * L.r * L.un +
+                                  (L.r * L.un * L.un + L.pT - L.bn * L.bn) -
+                                  (R.r * R.un * R.un + R.pT - R.bn * R.bn),
+                              dLR, rLR);
+      const double z2 = div64(SR * R.r * R.ut - SL * L.r * L.ut + (L.r * L.un * L.ut - L.bn * L.bt) -
+                                  (R.r * R.un * R.ut - R.bn * R.bt),
+                              dLR, rLR);
+      const double z3 = div64(SR * R.r * R.um - SL * L.r * L.um + (L.r * L.un * L.um - L.bn * L.bm) -
+                                  (R.r * R.un * R.um - R.bn * R.bm),
+                              dLR, rLR);
       const double ptz = ((R.pT + R.r * sR * (SM - R.un)) + (L.pT + L.r * sL * (SM - L.un))) / 2.0;
-      const double vz = z2 / z0, wz = z3 / z0;
-      const double vbz = (bn * z1 + bt * z2 + bm * z3) / z0;
+      const double rz = rcp64(z0);
+      const double vz = div64(z2, z0, rz), wz = div64(z3, z0, rz);
+      const double vbz = div64(bn * z1 + bt * z2 + bm * z3, z0, rz);
       sl.v = sr.v = vz;
       sl.w = sr.w = wz;
       sl.bt = sr.bt = bt;
       sl.bm = sr.bm = bm;
-      sl.e = L.e * (sL / dL) + (ptz * SM - L.pT * L.un + bn * (vdotb(L) - vbz)) / dL;
-      sr.e = R.e * (sR / dR) + (ptz * SM - R.pT * R.un + bn * (vdotb(R) - vbz)) / dR;
+      sl.e = L.e * cL + div64(ptz * SM - L.pT * L.un + bn * (vdotb(L) - vbz), dL, rL);
+      sr.e = R.e * cR + div64(ptz * SM - R.pT * R.un + bn * (vdotb(R) - vbz), dR, rR);
       // Gas_Dinamic.cu:1160-1187, in order
       if (SL >= 0.0) region = 0;
       else if (SL < 0.0 && SM >= 0.0) region = 1;
@@ -245,7 +266,7 @@ __global__ __launch_bounds__(MNT) void flux_mhd_kernel(size_t n, const double* _
     }
     out[7 * n + i] = F.c[4];
     out[8 * n + i] = F.c[8];
-    out[9 * n + i] = gas.krad / SN;
+    out[9 * n + i] = div64(gas.krad, SN);
   }
 }
 
