@@ -4,13 +4,12 @@
 // (pI <= pII), the same wave-pattern test on Uud/Urz/Uvk, the same sampling
 // at the face (w = 0) with the reference's region edges, and the same flux
 // and dt -- with the p* solve adapted to FP32:
-//  * two shocks: the reference's newton (kernel.cu:635-680) in FP32, its
-//    stopping scale pee the PVRS-type estimate as in the reference, the
-//    tolerance raised from 1e-9 to 1e-6 (FP32 resolution) and the starting
-//    point optionally a learned guess;
+//  * two shocks: the root of newton's equation (kernel.cu:635-680) by Newton
+//    in sqrt(p), to FP32 resolution, from the reference's PVRS-type estimate
+//    or a learned guess;
 //  * shock + rarefaction: the root of lev (kernel.cu:751-765) on the same
 //    bracket [pI, pII] as devtwo's bisection (kernel.cu:682-749), found by a
-//    bracket-safeguarded Newton iteration to 1e-6 relative;
+//    bracket-safeguarded Newton iteration in (p/pII)^((g-1)/2g);
 //  * FP64 islands: near vacuum and in strong rarefactions the p* equation
 //    subtracts two nearly equal numbers, and FP32 would lose the digits of
 //    p* there.  That difference -- and only it: every other term of these
@@ -23,6 +22,11 @@
 //        du = enI - enII, q = (p/pII)^((g-1)/2g)).
 //    Counted in ast_stats_t.fp64_faces.  (No FP64 pow: the islands keep the
 //    kernel's register budget, and so its occupancy, at the FP32 level.)
+// Bound: vector instructions.  Against the same solves in p (seven
+// transcendental operations a step, a pow among them, stopped at 1e-6) and a
+// sampling per pattern: 2^24 faces 345 -> 187 us, the step at 2047x1021
+// 41.5 -> 38.5; the error against 64 bits is the same (3.6e-8 of the flux, 99%
+// of the values within 3.5e-6 of theirs, was 3.6e-6).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -35,7 +39,7 @@ namespace ast {
 
 struct ExactCtx {
   float g, g1, g2, gp, gm, igm, ig1, c2g1, g1g2, c2g2;
-  double gd;
+  double gd, c2g1d;  // gamma, 2/(gamma - 1)
   int n;  // 1/gm = 2 gamma/(gamma - 1) when that is an integer in [1, 16] (5 for
           // gamma = 5/3, 7 for 7/5), else 0
   const unsigned char* mlp;  // learned-guess block (ast_mlp_t) in device memory, or null
@@ -59,6 +63,7 @@ static inline ExactCtx make_exact_ctx(double gamma, const void* mlp) {
   e.g1g2 = (float)(g1 / g2);
   e.c2g2 = (float)(2.0 / g2);
   e.gd = gamma;
+  e.c2g1d = 2.0 / g1;
   const double ig = 1.0 / gm, ni = floor(ig + 0.5);
   // (an FP32 gamma of 5/3 or 7/5 still counts: 1e-6 is its resolution)
   e.n = (fabs(ig - ni) <= 1e-6 * ig && ni >= 1.0 && ni <= 16.0) ? (int)ni : 0;
@@ -96,6 +101,20 @@ AST_DEV float geom_sum(float x, int n) {
 }
 // x^(1/gm): exact products for an integer 1/gm, else exp2/log2
 AST_DEV float pow_igm(const ExactCtx& e, float x) { return e.n ? ipow(x, e.n) : fpow(x, e.igm); }
+
+// x^(1/gm - 1), the same way
+AST_DEV float pow_igm1(const ExactCtx& e, float x) {
+  if (e.n == 5) {
+    const float x2 = x * x;
+    return x2 * x2;
+  }
+  if (e.n == 7) {
+    const float x2 = x * x;
+    return x2 * x2 * x2;
+  }
+  return e.n ? ipow(x, e.n - 1) : fpow(x, e.igm - 1.f);
+}
+AST_DEV float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
 
 // What the exact solver did on one face (pat: -1 vacuum, 0 two
 // rarefactions, 1 shock + rarefaction, 2 two shocks; kNoFace: not an exact
@@ -174,141 +193,305 @@ AST_DEV void block_stats_f32_to(const StatsF32& st, uint32_t* red, ast_stats_t* 
   }
 }
 
-constexpr float kNewtonTol32 = 1e-6f;
+constexpr float kBracket = 2e-7f;  // a bracket of y this narrow holds its root to 1e-6 in p
 // a two-shock face is served by the learned guess when the PVRS start is
 // poor: PVRS estimate above kStrongShock * pII (strong shocks)
 constexpr float kStrongShock = 3.f;
 constexpr float kVacuumIsland = 0.05f;
 constexpr float kRarefIsland = 1e-4f;
 
-// FP32 newton of kernel.cu:635-680 (two shocks), x^1.5 as x*sqrt(x).
-AST_DEV float newton_f32(const ExactCtx& e, float enI, float pI, float rI, float cI, float enII,
-                         float pII, float rII, float cII, float guess, bool use_guess,
-                         int& iters, bool& capped) {
-  const float g = e.g, gp = e.gp, gm = e.gm;
+// A Newton step stops the iterations below once it is at most kStep of the
+// iterate: its own remainder is then below kStep^2 (both equations bend by
+// less than that, curvature x / (2 slope) < 1), under the FP32 resolution.
+constexpr float kStep = 1e-4f;
+
+// Two shocks: the root of kernel.cu:635-680's equation
+//   fI(p) + fII(p) = enI - enII,  fK = (p - pK) hK,
+//   1/hK^2 = aK^2 = rK ((g+1) p + (g-1) pK)/2
+// (the reference's zK^2 (gp p/pK + gm) with zK = rK cK multiplied out: no
+// division by pK) by Newton in w = sqrt(p): a strong shock's fK grows like
+// sqrt(p), which is linear in w, so strong faces need no more steps than weak
+// ones.  dfK/dp = hK (1 + zK^2 hK^2)/2: three transcendental operations a
+// step.  pee: the PVRS-type estimate, kernel.cu:640, the start unless a
+// learned guess is used.  Every iterate is kept at or above pII (p* > pII in
+// this pattern).
+AST_DEV float newton_f32(const ExactCtx& e, float du, float pI, float rI, float cI, float pII,
+                         float rII, float cII, float guess, bool use_guess, int& iters,
+                         bool& capped) {
   const float zI = rI * cI, zII = rII * cII;
-  float pn = (pI * zII + pII * zI + (enI - enII) * zI * zII) * frcp(zI + zII);
-  const float pee = pn;
-  // a learned start is clamped into the two-shock range p* > pII: the
-  // function is concave and increasing in p, so Newton from at or below the
-  // root climbs to it monotonically, while a start far above the root would
-  // jump below zero (and sqrt of a negative argument is NaN); every iterate
-  // is clamped as well
-  const float plo = use_guess ? pII : -INFINITY;
-  if (use_guess) pn = fmaxf(guess, pII);
-  const float ipI = frcp(pI), ipII = frcp(pII);
-  const float k1 = g + 1.f, k3 = 3.f * g - 1.f, k4 = 4.f * g;
+  const float pee = (pI * zII + pII * zI + du * zI * zII) * frcp(zI + zII);
+  const float kI = 0.5f * e.g2 * rI, kII = 0.5f * e.g2 * rII;
+  const float jI = 0.5f * e.g1 * rI * pI, jII = 0.5f * e.g1 * rII * pII;
+  const float zzI = zI * zI, zzII = zII * zII, wlo = fsqrt(pII);
+  float w = fmaxf(fsqrt(use_guess ? guess : pee), wlo);
+  float p, dw;
   int k = 0;
-  float p, dprev = INFINITY;
   for (;;) {
-    p = pn;
+    p = w * w;
     k++;
-    const float aI = gp * p * ipI + gm, aII = gp * p * ipII + gm;
-    const float sI = fsqrt(aI), sII = fsqrt(aII);
-    const float fI = (p - pI) * frcp(zI * sI);
-    const float fII = (p - pII) * frcp(zII * sII);
-    const float dI = (k1 * p * ipI + k3) * frcp(k4 * zI * aI * sI);
-    const float dII = (k1 * p * ipII + k3) * frcp(k4 * zII * aII * sII);
-    pn = fmaxf(p - (fI + fII - (enI - enII)) * frcp(dI + dII), plo);
-    // the reference's rule |pn - p| < tol*pee, floored at the FP32
-    // resolution of the residual (pee can lie far below p* in strong
-    // shocks, where the residual's rounding moves p by ~2 ulp); close to
-    // the root (|dp| < 1e-4 p) it also stops once the steps stop shrinking,
-    // i.e. at the rounding floor
-    const float d = fabsf(pn - p);
-    if (!(d >= fmaxf(kNewtonTol32 * pee, 2e-6f * fabsf(pn)))) break;
-    if (k > 2 && d < 1e-4f * fabsf(pn) && !(d < 0.5f * dprev)) break;
-    dprev = d;
+    const float hI = frsq(fmaf(kI, p, jI)), hII = frsq(fmaf(kII, p, jII));
+    const float f = fmaf(p - pI, hI, fmaf(p - pII, hII, -du));
+    // 2 df/dp
+    const float d = fmaf(hI, fmaf(zzI * hI, hI, 1.f), hII * fmaf(zzII * hII, hII, 1.f));
+    dw = -f * frcp(w * d);  // df/dw = w d
+    if (!(fabsf(dw) > kStep * w)) break;
     if (k >= AST_ITER_CAP) { capped = true; break; }
+    w = fmaxf(w + dw, wlo);
   }
   iters = k;
-  return pn;
+  return fmaxf(fmaf(dw, fmaf(2.f, w, dw), p), pII);  // (w + dw)^2
 }
 
-template <typename R> struct FastM;
-template <> struct FastM<float> {
-  static AST_DEV float sqrt_(float a) { return fsqrt(a); }
-  static AST_DEV float pow_(float a, float b) { return fpow(a, b); }
-  static AST_DEV float div_(float a, float b) { return a * frcp(b); }
-};
-template <> struct FastM<double> {
-  static AST_DEV double sqrt_(double a) { return ::sqrt(a); }
-  static AST_DEV double pow_(double a, double b) { return ::pow(a, b); }
-  static AST_DEV double div_(double a, double b) { return a / b; }
-};
-
-// Root of lev(p) (left shock + right rarefaction) on [pI, pII]:
-// safeguarded Newton on fI(p) + c2 q(p) - D with D = c2 + du supplied by the
-// caller (FP64-formed in strong rarefactions).  R is float or double.
-template <typename R>
-AST_DEV R shock_raref(R g, R g1, R gp, R gm, R enI, R pI, R rI, R enII, R pII, R rII, R cI,
-                      R cII, R D, R tol, int& iters, bool& capped) {
-  typedef FastM<R> F;
-  const R zI = rI * cI, zII = rII * cII, du = enI - enII, c2 = F::div_(R(2), g1) * cII;
-  const R ipI = F::div_(R(1), pI), ipII = F::div_(R(1), pII);
-  R lo = pI, hi = pII;
-  // start: the linearised (PVRS-type) estimate, clipped into the bracket
-  R p = F::div_(pI * zII + pII * zI + du * zI * zII, zI + zII);
-  if (!(p > lo && p < hi)) p = R(0.5) * (lo + hi);
+// Shock + rarefaction: the root of lev (kernel.cu:751-765) on devtwo's
+// bracket [pI, pII] (kernel.cu:682-749) by safeguarded Newton in
+// y = (p/pII)^gm, in which the rarefaction is linear and p = pII y^n,
+// n = 1/gm (5 for gamma 5/3: products, no power function):
+//   (p - pI) hI + c2 y - D = 0,  c2 = 2 cII/(g - 1),  D = c2 + enI - enII
+// (D from the caller: FP64-formed in strong rarefactions).  hI and the
+// shock's derivative are newton_f32's, dp/dy = n p/y: two transcendental
+// operations a step.  q = (pI/pII)^gm; the start takes side I as a
+// rarefaction too, whose root is (cI + cII + (g-1)/2 du)/(cI/q + cII).
+// Returns y and p.
+AST_DEV float shock_raref_f32(const ExactCtx& e, float du, float D, float pI, float rI, float cI,
+                              float pII, float cII, float q, float& p, int& iters, bool& capped) {
+  const float kI = 0.5f * e.g2 * rI, jI = 0.5f * e.g1 * rI * pI, zI = rI * cI, zzI = zI * zI;
+  const float c2 = e.c2g1 * cII, hn = 0.5f * e.igm;
+  float lo = q, hi = 1.f;
+  float y = q * fmaf(0.5f * e.g1, du, cI + cII) * frcp(fmaf(q, cII, cI));
+  y = fminf(fmaxf(y, lo), hi);
+  if (!(y > 0.f)) y = 0.5f;  // pI / pII under the FP32 range
   int k = 0;
   for (;;) {
     k++;
-    const R a = gp * p * ipI + gm;
-    const R sa = F::sqrt_(a);
-    const R q = F::pow_(p * ipII, gm);
-    const R f = F::div_(p - pI, zI * sa) + c2 * q - D;
-    const R df = F::div_((g + R(1)) * p * ipI + (R(3) * g - R(1)), R(4) * g * zI * a * sa) +
-                 F::div_(cII * q, g * p);
-    if (f < R(0)) lo = p;
-    else hi = p;
-    R pn = p - F::div_(f, df);
-    if (!(pn > lo && pn < hi)) pn = R(0.5) * (lo + hi);
-    const R dp = pn - p;
-    p = pn;
-    if (!((dp < R(0) ? -dp : dp) > tol * p) || !(hi - lo > tol * p)) break;
+    const float m = pII * pow_igm1(e, y);  // p/y
+    p = m * y;
+    const float h = frsq(fmaf(kI, p, jI));
+    const float f = fmaf(p - pI, h, fmaf(c2, y, -D));
+    const float df = fmaf(hn * m * h, fmaf(zzI * h, h, 1.f), c2);
+    const float dy = -f * frcp(df);
+    if (f < 0.f) lo = y;
+    else hi = y;
+    float yn = y + dy;
+    if (!(fabsf(dy) > kStep * y)) {
+      y = fminf(fmaxf(yn, lo), hi);
+      break;
+    }
+    if (!(yn > lo && yn < hi)) yn = 0.5f * (lo + hi);
+    y = yn;
+    if (!(hi - lo > kBracket * y)) break;
     if (k >= AST_ITER_CAP) { capped = true; break; }
   }
   iters = k;
-  return p;
+  p = pII * pow_igm1(e, y) * y;
+  return y;
 }
 
-// The wave pattern exact_f32 will find for a face, as a schedule key for
-// sorting faces by pattern: 0 vacuum, 1 two rarefactions, 2 shock +
-// rarefaction, 3 two shocks, 4 two shocks that are strong (acoustic estimate
-// above kStrongShock * pII: the learned start's faces), 5 no pattern (NaN).
-// The same tests as exact_f32's, so the key is the pattern the solver takes.
-constexpr int kPatternKeys = 6;
-AST_DEV int pattern_key(const PrimF& L, const PrimF& R, const ExactCtx& e) {
+// A face with its sides swapped so that pI <= pII (kernel.cu:156-184; u turns
+// with them), the sides' sound speeds and q = (pI/pII)^gm.
+struct ExactFace {
+  float rI, pI, enI, teI, rII, pII, enII, teII, cI, cII, q;
+  bool sw;
+};
+AST_DEV ExactFace exact_sides(const PrimF& L, const PrimF& R, const ExactCtx& e) {
   const bool sw = L.p > R.p;
-  const float enI = sw ? -R.u : L.u, enII = sw ? -L.u : R.u;
-  const float pI = sw ? R.p : L.p, pII = sw ? L.p : R.p;
-  const float rI = sw ? R.r : L.r, rII = sw ? L.r : R.r;
-  const float cI = fsqrt(e.g * pI * frcp(rI)), cII = fsqrt(e.g * pII * frcp(rII));
-  const float q = fpow(pI * frcp(pII), e.gm);
-  const float a = fsqrt(rI * (e.g2 * pII + e.g1 * pI) * 0.5f);
-  const float Uud = (pII - pI) * frcp(a);
-  const float Urz = -e.c2g1 * cII * (1.f - q);
-  const float Uvk = -e.c2g1 * (cII + cI);
-  const float Udf = enI - enII;
-  if (Udf < Uvk) return 0;
-  if (Udf >= Uvk && Udf <= Urz) return 1;
-  if (Udf > Urz && Udf <= Uud) return 2;
-  if (Udf > Uud) {
-    const float zI = rI * cI, zII = rII * cII;
-    return (pI * zII + pII * zI + Udf * zI * zII) * frcp(zI + zII) > kStrongShock * pII ? 4 : 3;
-  }
-  return 5;
+  ExactFace f;
+  f.sw = sw;
+  f.rI = sw ? R.r : L.r;
+  f.pI = sw ? R.p : L.p;
+  f.enI = sw ? -R.u : L.u;
+  f.teI = sw ? R.v : L.v;
+  f.rII = sw ? L.r : R.r;
+  f.pII = sw ? L.p : R.p;
+  f.enII = sw ? -L.u : R.u;
+  f.teII = sw ? L.v : R.v;
+  f.cI = fsqrt(e.g * f.pI * frcp(f.rI));
+  f.cII = fsqrt(e.g * f.pII * frcp(f.rII));
+  f.q = fpow(f.pI * frcp(f.pII), e.gm);
+  return f;
 }
 
-// FP64 sound speed of an FP32 state (for the FP64-formed differences)
-AST_DEV double sound_speed_d(double g, float p, float r) { return sqrt(g * (double)p / (double)r); }
+// The wave pattern: vacuum, two rarefactions, shock + rarefaction or two
+// shocks.  Each pattern's whole interval is tested, so NaN input matches none.
+// Four lane masks, which live in scalar registers.
+struct WavePattern {
+  bool vac, rr, sr, ss;
+  // FaceInfo's number
+  AST_DEV int number() const { return vac ? -1 : rr ? 0 : sr ? 1 : ss ? 2 : kNoPattern; }
+};
+AST_DEV WavePattern wave_pattern(const ExactFace& f, const ExactCtx& e) {
+  const float Uud = (f.pII - f.pI) * frsq(f.rI * (e.g2 * f.pII + e.g1 * f.pI) * 0.5f);
+  const float Urz = -e.c2g1 * f.cII * (1.f - f.q);
+  const float Uvk = -e.c2g1 * (f.cII + f.cI);
+  const float Udf = f.enI - f.enII;
+  WavePattern w;
+  w.vac = Udf < Uvk;
+  w.rr = Udf >= Uvk && Udf <= Urz;
+  w.sr = Udf > Urz && Udf <= Uud;
+  w.ss = Udf > Uud;
+  if (w.vac) w.rr = w.sr = w.ss = false;  // the first pattern that matches
+  if (w.rr) w.sr = w.ss = false;
+  if (w.sr) w.ss = false;
+  return w;
+}
+// A two-shock face whose PVRS estimate is above kStrongShock * pII: the
+// learned start's faces.
+AST_DEV bool strong_shocks(const ExactFace& f) {
+  const float zI = f.rI * f.cI, zII = f.rII * f.cII;
+  return (f.pI * zII + f.pII * zI + (f.enI - f.enII) * zI * zII) * frcp(zI + zII) >
+         kStrongShock * f.pII;
+}
 
-// The exact face flux in the face frame (u normal, v tangential), kernel.cu:
-// 128-570 in FP32 (see the header), as the physical flux of the state it
-// samples at the face, written in that state's frame (FaceF: m = r un,
-// w = (un, ut), gn = p, gt = 0, ge = un p/(g-1)); UU is the largest |wave
-// speed| used for dt; fi reports the wave pattern, iterations and flags.
-// `guess` (finite, > 0) seeds newton.
+// A face's schedule key for sorting faces by pattern: 0 vacuum, 1 two
+// rarefactions, 2 shock + rarefaction, 3 two shocks, 4 (STRONG) strong two
+// shocks, 5 no pattern (NaN).
+constexpr int kPatternKeys = 6;
+template <bool STRONG>
+AST_DEV int pattern_key(const ExactFace& f, const WavePattern& w) {
+  return w.vac ? 0 : w.rr ? 1 : w.sr ? 2 : w.ss ? (STRONG && strong_shocks(f) ? 4 : 3) : 5;
+}
+
+// FP64 sound speed of an FP32 state (for the FP64-formed differences), c its
+// FP32 value: 1/r and the root refined from the FP32 ones by Newton steps
+// (1e-7 -> 1e-14 -> the last bits), a third of the double divide and square
+// root's instructions.
+AST_DEV double sound_speed_d(double g, float p, float r, float c) {
+  const double rd = r, i0 = frcp(r);
+  const double e0 = fma(-rd, i0, 1.0);
+  const double x = g * (double)p * fma(i0, fma(e0, e0, e0), i0);
+  const double h = c > 0.f ? 0.5f * frcp(c) : 0.f;
+  double cd = c;
+  cd = fma(fma(-cd, cd, x), h, cd);
+  return fma(fma(-cd, cd, x), h, cd);
+}
+
+// The flux of a face of pattern w (kernel.cu:128-570 in FP32, see the
+// header), as the physical flux of the state it samples at the face, written
+// in that state's frame (FaceF: m = r un, w = (un, ut), gn = p, gt = 0, ge =
+// un p/(g-1)); UU is the largest |wave speed| used for dt; fi reports the
+// iterations and flags.  `guess` (finite, > 0) seeds newton.
+//
+// The patterns differ only in their p* solve: the sampling (kernel.cu:
+// 234-544) is one code for all, with the side that holds w = 0 mirrored onto
+// side I, so that lanes of different patterns and regions share it.  Faces
+// outside both rarefactions take a side's state without a p*.
+AST_DEV FaceF exact_solve_f32(const ExactFace& s, const WavePattern& w, const ExactCtx& e,
+                              float& UU, FaceInfo& fi, float guess) {
+  const float g = e.g, g1 = e.g1, g2 = e.g2, gm = e.gm;
+  const float enI = s.enI, enII = s.enII, pI = s.pI, pII = s.pII, rI = s.rI, rII = s.rII;
+  const float cI = s.cI, cII = s.cII, Udf = enI - enII;
+  // heads of the waves, the rarefactions' until a shock is found; the tails
+  // lie between them, so the largest |speed| is a head's
+  float dI = enI - cI, dII = enII + cII;
+  // two rarefactions: t = (p/pI)^gm; Urz - Uvk = 2/(g-1) (cII q + cI) (no
+  // cancellation)
+  const float iden = frcp(e.c2g1 * fmaf(cII, s.q, cI));
+  float t = (Udf + e.c2g1 * (cII + cI)) * iden;
+  bool island = (w.rr && t < kVacuumIsland) || (w.sr && pI < kRarefIsland * pII);
+  int it = 0;
+  bool capped = false, learned = false;
+  const bool shock = w.sr || w.ss;
+  const bool outI = 0.f <= dI;
+  bool one = outI;
+  float en = outI ? enI : -enII, pp = outI ? pI : pII, r = outI ? rI : rII;
+  bool empty = false;
+  if (shock || !(outI || dII <= 0.f)) {
+    const float zI = rI * cI, zII = rII * cII;
+    float p = 0.f, aI = zI, aII = zII, y = 0.f;
+    if (w.rr) {
+      if (island) {  // FP64 island: near vacuum
+        const double num = fma(e.c2g1d, sound_speed_d(e.gd, pI, rI, cI) +
+                                        sound_speed_d(e.gd, pII, rII, cII),
+                               (double)enI - (double)enII);
+        t = fmaxf((float)num, 0.f) * iden;
+      }
+      y = t * s.q;
+      p = pI * pow_igm(e, t);
+    }
+    if (w.sr) {
+      float D = fmaf(e.c2g1, cII, Udf);
+      if (island)  // FP64 island: strong rarefaction
+        D = (float)fma(e.c2g1d, sound_speed_d(e.gd, pII, rII, cII), (double)enI - (double)enII);
+      y = shock_raref_f32(e, Udf, D, pI, rI, cI, pII, cII, s.q, p, it, capped);
+    }
+    if (w.ss) {
+      learned = guess > 0.f && guess < 3.0e38f;
+      p = newton_f32(e, Udf, pI, rI, cI, pII, rII, cII, guess, learned, it, capped);
+    }
+    // impedances: shocks aK^2 = rK ((g+1) p + (g-1) pK)/2, speed enI - aI/rI
+    // (enII + aII/rII); rarefactions (kernel.cu:369-388) aK = gm rK cK
+    // (1 - x)/(1 - x^gm), x = p/pK, with x^gm = t (side I) and y (side II):
+    // a geometric sum for an integer 1/gm
+    const float hp = 0.5f * g2 * p;
+    if (shock) {
+      aI = fsqrt(rI * fmaf(0.5f * g1, pI, hp));
+      dI = enI - aI * frcp(rI);
+    } else if (e.n) {
+      aI = gm * zI * geom_sum(t, e.n);
+    } else if (!(fabsf(p - pI) < 1e-6f * pI)) {
+      aI = gm * zI * (1.f - p * frcp(pI)) * frcp(1.f - t);
+    }
+    if (w.ss) {
+      aII = fsqrt(rII * fmaf(0.5f * g1, pII, hp));
+      dII = enII + aII * frcp(rII);
+    } else if (e.n) {
+      aII = gm * zII * geom_sum(y, e.n);
+    } else if (!(fabsf(p - pII) < 1e-6f * pII)) {
+      aII = gm * zII * (1.f - p * frcp(pII)) * frcp(1.f - y);
+    }
+    const float u = (aI * enI + aII * enII + pI - pII) * frcp(aI + aII);
+    // rarefactions' tails; a vacuum's edges
+    const float hg = 0.5f * g1;
+    const float tI = w.vac ? fmaf(e.c2g1, cI, enI) : u - fmaf(hg, enI - u, cI);
+    const float tII = w.vac ? fmaf(-e.c2g1, cII, enII) : u + fmaf(hg, u - enII, cII);
+    // the side of the face, mirrored onto side I
+    one = 0.f <= dI || (!shock && 0.f < tI) || (!w.vac && 0.f <= u);
+    const float en0 = one ? enI : -enII, c0 = one ? cI : cII, us = one ? u : -u;
+    const float head = one ? dI : -dII, tail = one ? tI : -tII;
+    const bool sh0 = one ? shock : w.ss;
+    en = en0;
+    pp = one ? pI : pII;
+    r = one ? rI : rII;
+    if (!(0.f <= head)) {
+      if (sh0) {
+        const float a0 = one ? aI : aII;
+        r = r * a0 * frcp(a0 - r * (en0 - us));
+        en = us;
+        pp = p;
+      } else {
+        const bool fan = 0.f < tail;
+        const float ce = fan ? fmaf(e.g1g2, en0, e.c2g2 * c0) : fmaf(hg, en0 - us, c0);
+        en = fan ? ce : us;
+        pp = fan ? pp * pow_igm(e, ce * frcp(c0)) : p;
+        r = g * pp * frcp(ce * ce);
+        empty = w.vac && !one && !fan;  // between a vacuum's edges
+      }
+    }
+  }
+  fi.pat = w.number();
+  fi.it = it;
+  fi.capped = capped;
+  fi.island = island;
+  fi.learned = learned;
+  UU = fmaxf(fabsf(dI), fabsf(dII));
+  float te = one ? s.teI : s.teII;
+  if (empty) en = pp = r = te = 0.f;
+  if (!(w.vac || w.rr || shock)) {  // no pattern (NaN input): NaN fluxes, dt 0
+    UU = INFINITY;
+    en = pp = r = te = __int_as_float(0x7fc00000);
+  }
+  if (!(UU > 1e-7f)) UU = 1e-7f;  // eps8 floor of the reference's dt, kernel.cu:246-253
+  if (one == s.sw) en = -en;      // side II mirrored, sides swapped: either turns u
+  FaceF f;
+  f.m = r * en;
+  f.wn = en;
+  f.wt = te;
+  f.gn = pp;
+  f.gt = 0.f;
+  f.ge = en * pp * e.ig1;
+  return f;
+}
+
+// The exact face flux of two states in the face frame (u normal, v tangential).
 // LEARNED (compiled only into the kernels that serve a learned guess; its
 // network needs registers the plain solver does not) with e.mlp set: the
 // caller guarantees a full wave (EXEC all ones); if any lane of the wave
@@ -319,172 +502,21 @@ AST_DEV double sound_speed_d(double g, float p, float r) { return sqrt(g * (doub
 template <bool LEARNED, bool DETECT = false>
 AST_DEV FaceF exact_frame_f32(const PrimF& L, const PrimF& R, const ExactCtx& e, float& UU,
                               FaceInfo& fi, float guess = -1.f) {
-  const float g = e.g, g1 = e.g1, g2 = e.g2, gm = e.gm;
-  // swap sides so that pI <= pII, kernel.cu:156-184
-  const bool sw = L.p > R.p;
-  const float enI = sw ? -R.u : L.u, enII = sw ? -L.u : R.u;
-  const float teI = sw ? R.v : L.v, teII = sw ? L.v : R.v;
-  const float pI = sw ? R.p : L.p, pII = sw ? L.p : R.p;
-  const float rI = sw ? R.r : L.r, rII = sw ? L.r : R.r;
-  const float cI = fsqrt(g * pI * frcp(rI)), cII = fsqrt(g * pII * frcp(rII));
-  const float q = fpow(pI * frcp(pII), gm);  // (pI/pII)^gm
-  const float a = fsqrt(rI * (g2 * pII + g1 * pI) * 0.5f);
-  const float Uud = (pII - pI) * frcp(a);
-  const float Urz = -e.c2g1 * cII * (1.f - q);
-  const float Uvk = -e.c2g1 * (cII + cI);
-  const float Udf = enI - enII;
-  // strong two-shock face: PVRS estimate above kStrongShock * pII (the
-  // learned kernel needs it before the branches for its wave ballot, the
-  // detecting one only in the two-shock branch)
+  const ExactFace s = exact_sides(L, R, e);
+  const WavePattern w = wave_pattern(s, e);
+  // strong two-shock face (the learned kernel needs it for its wave ballot)
   bool strong = false;
-  auto strong_pvrs = [&]() {
-    const float zI = rI * cI, zII = rII * cII;
-    return (pI * zII + pII * zI + Udf * zI * zII) * frcp(zI + zII) > kStrongShock * pII;
-  };
-  if constexpr (LEARNED) strong = (Udf > Uud) && strong_pvrs();
+  if constexpr (LEARNED || DETECT) strong = w.ss && strong_shocks(s);
   if (LEARNED && e.mlp != nullptr) {
     if (__builtin_amdgcn_ballot_w64(strong) != 0) {  // wave-uniform
       float fe[mlp::IN];
-      const float lp = mlp::features<float>(rI, pI, enI, rII, pII, enII, g, fe);
+      const float lp = mlp::features<float>(s.rI, s.pI, s.enI, s.rII, s.pII, s.enII, e.g, fe);
       const float y = mlp::forward_wave_bf16(e.mlp, fe);
       if (strong) guess = __expf(y + lp);
     }
   }
-  int pat;
-  float p = 0.f, t = 1.f;
-  int it = 0;
-  bool capped = false, island = false, learned = false;
-  // each pattern's whole interval is tested, so NaN input matches none
-  if (Udf < Uvk) {
-    pat = -1;
-  } else if (Udf >= Uvk && Udf <= Urz) {
-    // two rarefactions, Urz - Uvk = 2/(g-1) (cII q + cI) (no cancellation)
-    pat = 0;
-    const float den = e.c2g1 * (cII * q + cI);
-    t = (Udf - Uvk) * frcp(den);
-    if (t < kVacuumIsland) {  // FP64 island: near vacuum
-      const double gd = e.gd;
-      const double num = ((double)enI - (double)enII) +
-                         2.0 / (gd - 1.0) * (sound_speed_d(gd, pI, rI) + sound_speed_d(gd, pII, rII));
-      t = fmaxf((float)num, 0.f) * frcp(den);
-      island = true;
-    }
-    p = pI * pow_igm(e, t);
-  } else if (Udf > Urz && Udf <= Uud) {
-    pat = 1;
-    float D;
-    if (pI < kRarefIsland * pII) {  // FP64 island: strong rarefaction
-      const double gd = e.gd;
-      D = (float)(2.0 / (gd - 1.0) * sound_speed_d(gd, pII, rII) + ((double)enI - (double)enII));
-      island = true;
-    } else {
-      D = e.c2g1 * cII + Udf;
-    }
-    p = shock_raref<float>(g, g1, e.gp, gm, enI, pI, rI, enII, pII, rII, cI, cII, D, kNewtonTol32,
-                           it, capped);
-  } else if (Udf > Uud) {
-    pat = 2;
-    if constexpr (DETECT && !LEARNED) strong = strong_pvrs();
-    learned = guess > 0.f && guess < 3.0e38f;
-    p = newton_f32(e, enI, pI, rI, cI, enII, pII, rII, cII, guess, learned, it, capped);
-  } else {
-    pat = kNoPattern;  // NaN input
-  }
-  fi.pat = pat;
-  fi.it = it;
-  fi.capped = capped;
-  fi.island = island;
-  fi.learned = learned;
   fi.strong = strong;
-
-  // sample the solution at w = 0, kernel.cu:234-544
-  float en, pp, r, te;
-  if (pat == 2) {
-    const float aI = fsqrt(rI * (g2 * 0.5f * p + g1 * 0.5f * pI));
-    const float aII = fsqrt(rII * (g2 * 0.5f * p + g1 * 0.5f * pII));
-    const float u = (aI * enI + aII * enII + pI - pII) * frcp(aI + aII);
-    const float dI = enI - aI * frcp(rI), dII = enII + aII * frcp(rII);
-    UU = fmaxf(fabsf(dI), fabsf(dII));
-    if (0.f <= dI) { en = enI; pp = pI; r = rI; te = teI; }
-    else if (0.f <= u) { en = u; pp = p; r = rI * aI * frcp(aI - rI * (enI - u)); te = teI; }
-    else if (0.f < dII) { en = u; pp = p; r = rII * aII * frcp(aII + rII * (enII - u)); te = teII; }
-    else { en = enII; pp = pII; r = rII; te = teII; }
-  } else if (pat == 1) {
-    const float aI = fsqrt(rI * (g2 * 0.5f * p + g1 * 0.5f * pI));
-    float aII;
-    if (fabsf(p - pII) < 1e-6f * pII) aII = rII * cII;
-    else aII = gm * rII * cII * (1.f - p * frcp(pII)) * frcp(1.f - fpow(p * frcp(pII), gm));
-    const float u = (aI * enI + aII * enII + pI - pII) * frcp(aI + aII);
-    const float dI = enI - aI * frcp(rI), dII = enII + cII;
-    const float ddII = u + cII - g1 * (enII - u) * 0.5f;
-    UU = fmaxf(fmaxf(fabsf(dI), fabsf(dII)), fabsf(ddII));
-    if (0.f <= dI) { en = enI; pp = pI; r = rI; te = teI; }
-    else if (0.f <= u) { en = u; pp = p; r = rI * aI * frcp(aI - rI * (enI - u)); te = teI; }
-    else if (0.f <= ddII) {
-      const float ce = cII - g1 * 0.5f * (enII - u);
-      en = u; pp = p; r = g * p * frcp(ce * ce); te = teII;
-    } else if (0.f < dII) {
-      const float ce = -e.g1g2 * enII + e.c2g2 * cII;
-      en = -ce; pp = pII * pow_igm(e, ce * frcp(cII)); r = g * pp * frcp(ce * ce); te = teII;
-    } else { en = enII; pp = pII; r = rII; te = teII; }
-  } else if (pat == 0) {
-    // rarefaction impedances aK = gm rK cK (1 - x)/(1 - x^gm), x = p/pK
-    // (kernel.cu:369-388), with x^gm = t (side I) and t q (side II)
-    float aI, aII;
-    if (e.n) {
-      aI = gm * rI * cI * geom_sum(t, e.n);
-      aII = gm * rII * cII * geom_sum(t * q, e.n);
-    } else {
-      if (fabsf(p - pI) < 1e-6f * pI) aI = rI * cI;
-      else aI = gm * rI * cI * (1.f - p * frcp(pI)) * frcp(1.f - t);
-      if (fabsf(p - pII) < 1e-6f * pII) aII = rII * cII;
-      else aII = gm * rII * cII * (1.f - p * frcp(pII)) * frcp(1.f - t * q);
-    }
-    const float u = (aI * enI + aII * enII + pI - pII) * frcp(aI + aII);
-    const float dI = enI - cI, ddI = u - cI - g1 * (enI - u) * 0.5f;
-    const float dII = enII + cII, ddII = u + cII - g1 * (enII - u) * 0.5f;
-    UU = fmaxf(fmaxf(fabsf(dI), fabsf(dII)), fmaxf(fabsf(ddII), fabsf(ddI)));
-    if (0.f <= dI) { en = enI; pp = pI; r = rI; te = teI; }
-    else if (0.f < ddI) {
-      const float ce = e.g1g2 * enI + e.c2g2 * cI;
-      en = ce; pp = pI * pow_igm(e, ce * frcp(cI)); r = g * pp * frcp(ce * ce); te = teI;
-    } else if (0.f <= u) {
-      const float ce = cI + g1 * 0.5f * (enI - u);
-      en = u; pp = p; r = g * p * frcp(ce * ce); te = teI;
-    } else if (0.f <= ddII) {
-      const float ce = cII - g1 * 0.5f * (enII - u);
-      en = u; pp = p; r = g * p * frcp(ce * ce); te = teII;
-    } else if (0.f < dII) {
-      const float ce = -e.g1g2 * enII + e.c2g2 * cII;
-      en = -ce; pp = pII * pow_igm(e, ce * frcp(cII)); r = g * pp * frcp(ce * ce); te = teII;
-    } else { en = enII; pp = pII; r = rII; te = teII; }
-  } else if (pat == -1) {  // vacuum, kernel.cu:480-544
-    const float dI = enI - cI, ddI = enI + e.c2g1 * cI;
-    const float dII = enII + cII, ddII = enII - e.c2g1 * cII;
-    UU = fmaxf(fmaxf(fabsf(dI), fabsf(dII)), fmaxf(fabsf(ddII), fabsf(ddI)));
-    if (0.f <= dI) { en = enI; pp = pI; r = rI; te = teI; }
-    else if (0.f < ddI) {
-      const float ce = e.g1g2 * enI + e.c2g2 * cI;
-      en = ce; pp = pI * pow_igm(e, ce * frcp(cI)); r = g * pp * frcp(ce * ce); te = teI;
-    } else if (0.f <= ddII) { en = 0.f; pp = 0.f; r = 0.f; te = 0.f; }
-    else if (0.f < dII) {
-      const float ce = -e.g1g2 * enII + e.c2g2 * cII;
-      en = -ce; pp = pII * pow_igm(e, ce * frcp(cII)); r = g * pp * frcp(ce * ce); te = teII;
-    } else { en = enII; pp = pII; r = rII; te = teII; }
-  } else {  // no pattern (NaN input): NaN fluxes, dt 0
-    UU = INFINITY;
-    en = pp = r = te = __int_as_float(0x7fc00000);
-  }
-  if (!(UU > 1e-7f)) UU = 1e-7f;  // eps8 floor of the reference's dt, kernel.cu:246-253
-  if (sw) en = -en;
-  FaceF f;
-  f.m = r * en;
-  f.wn = en;
-  f.wt = te;
-  f.gn = pp;
-  f.gt = 0.f;
-  f.ge = en * pp * e.ig1;
-  return f;
+  return exact_solve_f32(s, w, e, UU, fi, guess);
 }
 
 // The same flux in the lab frame (face-frame axes).

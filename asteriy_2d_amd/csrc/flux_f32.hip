@@ -14,27 +14,12 @@ namespace f32 {
 
 constexpr int FNT = 256;
 
-// STATS: the variant that counts the exact solver's work into *stats;
-// LEARNED: the exact solver with the learned newton start compiled in
-template <int METHOD, bool STATS, bool LEARNED>
+template <int METHOD>
 __global__ __launch_bounds__(FNT) void flux_kernel(size_t n, const float* __restrict__ in,
                                                    float n1, float n2, float krad,
-                                                   ExactCtx ex, float* __restrict__ out,
-                                                   ast_stats_t* stats, int* __restrict__ info) {
-  __shared__ uint32_t redi[(FNT / 64) * 10];
-  typename std::conditional<STATS, StatsF32, NoStats>::type st;
-  st.clear();
-  // whole 64-face tiles per wave: every lane runs every iteration (EXEC full,
-  // as the wave-level learned guess needs); lanes past n compute on a clamped
-  // face and do not store
+                                                   ExactCtx ex, float* __restrict__ out) {
   const size_t stride = (size_t)gridDim.x * FNT;
-  const size_t nt = (n + 63) / 64 * 64;
-  const int lane = threadIdx.x & 63;
-  const size_t base0 = (size_t)blockIdx.x * FNT + 64 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (size_t base = base0; base < nt; base += stride) {  // wave-uniform
-    const size_t ii = base + lane;
-    const bool valid = ii < n;
-    const size_t i = valid ? ii : n - 1;
+  for (size_t i = (size_t)blockIdx.x * FNT + threadIdx.x; i < n; i += stride) {
     const float rl = in[i], pl = in[n + i], vxl = in[2 * n + i], vyl = in[3 * n + i];
     const float rr = in[4 * n + i], pr = in[5 * n + i], vxr = in[6 * n + i], vyr = in[7 * n + i];
     // face frame: normal (n1, n2), tangent (-n2, n1)
@@ -42,29 +27,17 @@ __global__ __launch_bounds__(FNT) void flux_kernel(size_t n, const float* __rest
     const PrimF R = {rr, pr, vxr * n1 + vyr * n2, -vxr * n2 + vyr * n1};
     float UU;
     FluxF f;
+    FaceInfo fi;
     if constexpr (METHOD == AST_HLL) f = hll_f32(L, R, ex.g, ex.ig1, UU);
     else if constexpr (METHOD == AST_HLLC) f = hllc_f32<false>(L, R, ex.g, ex.ig1, UU);
     else if constexpr (METHOD == AST_HLLC_A) f = hllc_f32<true>(L, R, ex.g, ex.ig1, UU);
-    else {
-      FaceInfo fi;
-      f = exact_f32<LEARNED>(L, R, ex, UU, fi);
-      if (!valid) fi = FaceInfo{kNoFace, 0, false, false, false, false};
-      st.add(fi);
-      if (info && valid) {
-        info[2 * i] = fi.it;
-        info[2 * i + 1] = (fi.pat == kNoPattern ? -1 : fi.pat + 1) | (fi.capped ? 8 : 0) |
-                          (fi.island ? 16 : 0);
-      }
-    }
-    if (valid) {
-      out[i] = f.m;
-      out[n + i] = f.e;
-      out[2 * n + i] = f.un * n1 - f.ut * n2;
-      out[3 * n + i] = f.un * n2 + f.ut * n1;
-      out[4 * n + i] = krad * frcp(UU);
-    }
+    else f = exact_f32<false>(L, R, ex, UU, fi);
+    out[i] = f.m;
+    out[n + i] = f.e;
+    out[2 * n + i] = f.un * n1 - f.ut * n2;
+    out[3 * n + i] = f.un * n2 + f.ut * n1;
+    out[4 * n + i] = krad * frcp(UU);
   }
-  if constexpr (STATS) block_stats_f32_to<FNT>(st, redi, stats);
 }
 
 // ---- the exact solver on pattern-sorted faces ------------------------------
@@ -78,11 +51,17 @@ __global__ __launch_bounds__(FNT) void flux_kernel(size_t n, const float* __rest
 // lanes of a wave mostly hold faces of one pattern.  Results depend only on
 // each face's own data: the order changes no bit.
 //
-// The tile's faces are kept in LDS from the classifying (coalesced) loads on:
-// the solve reads its permuted faces there and leaves its fluxes there, and
-// the tile's fluxes go out with coalesced stores (measured: re-reading the
-// faces from global memory in sorted order, 32 scattered loads per lane and
-// tile, took 60% of the kernel's time).
+// Bound: the solver's vector instructions (about 90% of issue at 2^24 faces,
+// 400 a face and wave; the 52 B a face take 155 us at a copy's rate).
+//
+// The tile's faces are kept in LDS from the classifying (coalesced) loads on,
+// swapped and with the sound speeds and the power the classes needed: the
+// solve reads its permuted faces there and leaves its fluxes there, and the
+// tile's fluxes go out with coalesced stores.  Measured at 2^24 faces: 345 us
+// with the p* solves and a sampling per pattern of before, 200 us with
+// exact_f32.hpp's, 188 us with the classes' values kept as well; re-reading
+// the faces from global memory in sorted order, 32 scattered loads per lane
+// and tile, took 60% of the kernel's time.
 //
 // With the learned newton start, a first kernel (kGuessPass) evaluates the
 // network for the strong two-shock faces only -- they are contiguous after
@@ -112,36 +91,47 @@ __global__ __launch_bounds__(SORT_NT) void exact_sorted_kernel(size_t n,
                                                                int* __restrict__ info) {
   constexpr bool STRONG = MODE != kSolve;  // strong faces form a group of their own
   __shared__ uint32_t redi[(SORT_NT / 64) * 10];
+  // slot -> face of the tile (low bits), its key and its swap
+  static_assert(STILE <= 1 << 9 && kPatternKeys < 8, "perm's fields");
   __shared__ unsigned short perm[STILE];
   __shared__ int cnt[kPatternKeys + 1], cur[kPatternKeys + 1];
-  __shared__ float stage[8][STILE];  // the tile's faces, then (5 planes) its fluxes
+  __shared__ float stage[11][STILE];  // the tile's ExactFaces, then (5 planes) its fluxes
   typename std::conditional<STATS, StatsF32, NoStats>::type st;
   st.clear();
+  auto staged = [&](int li) {
+    return ExactFace{stage[0][li], stage[1][li], stage[2][li], stage[3][li], stage[4][li],
+                     stage[5][li], stage[6][li], stage[7][li], stage[8][li], stage[9][li],
+                     stage[10][li], false};
+  };
   const size_t ntiles = (n + STILE - 1) / STILE;
   for (size_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {  // workgroup-uniform
     const size_t base = tile * STILE;
     const int nv = (int)min((size_t)STILE, n - base);
     if (threadIdx.x <= kPatternKeys) cnt[threadIdx.x] = 0;
     __syncthreads();
-    // classify (coalesced loads, kept in LDS) and count
-    int key[SORT_PER];
+    // classify (coalesced loads) and count
+    unsigned tag[SORT_PER];  // perm's entry
 #pragma unroll
     for (int j = 0; j < SORT_PER; j++) {
       const int li = j * SORT_NT + threadIdx.x;
-      key[j] = kPatternKeys;  // past the end of the batch
+      unsigned key = kPatternKeys;  // past the end of the batch
+      bool sw = false;
       if (li < nv) {
         float w[8];
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-          w[k] = in[k * n + base + li];
-          stage[k][li] = w[k];
-        }
+        for (int k = 0; k < 8; k++) w[k] = in[k * n + base + li];
         PrimF L, R;
         face_frame(w, n1, n2, L, R);
-        key[j] = pattern_key(L, R, ex);
-        if (!STRONG && key[j] == 4) key[j] = 3;  // no network: strong faces are plain ones
+        const ExactFace f = exact_sides(L, R, ex);
+        const float v[11] = {f.rI, f.pI, f.enI, f.teI, f.rII, f.pII, f.enII, f.teII, f.cI, f.cII,
+                             f.q};
+#pragma unroll
+        for (int k = 0; k < 11; k++) stage[k][li] = v[k];
+        key = pattern_key<STRONG>(f, wave_pattern(f, ex));
+        sw = f.sw;
       }
-      atomicAdd(&cnt[key[j]], 1);
+      tag[j] = (unsigned)li | key << 9 | (sw ? 1u << 12 : 0u);
+      atomicAdd(&cnt[key], 1);
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -157,8 +147,8 @@ __global__ __launch_bounds__(SORT_NT) void exact_sorted_kernel(size_t n,
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < SORT_PER; j++) {
-      const int slot = atomicAdd(&cur[key[j]], 1);
-      perm[slot] = (unsigned short)(j * SORT_NT + threadIdx.x);
+      const int slot = atomicAdd(&cur[tag[j] >> 9 & 7], 1);
+      perm[slot] = (unsigned short)tag[j];
     }
     __syncthreads();
     const int s0 = cnt[0], s1 = cnt[1], nfaces = cnt[2];
@@ -166,17 +156,11 @@ __global__ __launch_bounds__(SORT_NT) void exact_sorted_kernel(size_t n,
       // the network on the strong faces, whole waves of them (EXEC full)
       const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
       for (int w0 = s0 + 64 * wave; w0 < s1; w0 += SORT_NT) {  // wave-uniform
-        const int li = perm[min(w0 + lane, s1 - 1)];
-        float w[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) w[k] = stage[k][li];
-        PrimF L, R;
-        face_frame(w, n1, n2, L, R);
-        const bool sw = L.p > R.p;
+        const int li = perm[min(w0 + lane, s1 - 1)] & (STILE - 1);
+        const ExactFace f = staged(li);
         float fe[mlp::IN];
-        const float lp = mlp::features<float>(sw ? R.r : L.r, sw ? R.p : L.p, sw ? -R.u : L.u,
-                                              sw ? L.r : R.r, sw ? L.p : R.p, sw ? -L.u : R.u,
-                                              ex.g, fe);
+        const float lp =
+            mlp::features<float>(f.rI, f.pI, f.enI, f.rII, f.pII, f.enII, ex.g, fe);
         const float y = mlp::forward_wave_bf16(ex.mlp, fe);
         if (w0 + lane < s1) out[4 * n + base + li] = __expf(y + lp);
       }
@@ -187,22 +171,21 @@ __global__ __launch_bounds__(SORT_NT) void exact_sorted_kernel(size_t n,
         const int pos = j * SORT_NT + threadIdx.x;
         FaceInfo fi{kNoFace, 0, false, false, false, false};
         if (pos < nfaces) {
-          const int li = perm[pos];
+          const unsigned tg = perm[pos];
+          const int li = tg & (STILE - 1), key = tg >> 9 & 7;
           const size_t i = base + li;
-          float w[8];
-#pragma unroll
-          for (int k = 0; k < 8; k++) w[k] = stage[k][li];
-          PrimF L, R;
-          face_frame(w, n1, n2, L, R);
+          ExactFace f = staged(li);
+          f.sw = (tg >> 12) != 0;
+          const WavePattern wp{key == 0, key == 1, key == 2, key == 3 || key == 4};
           const float g = (MODE == kSolveGuessed && pos >= s0 && pos < s1) ? out[4 * n + i] : -1.f;
           float UU;
-          const FluxF f = exact_f32<false>(L, R, ex, UU, fi, g);
+          const FluxF q = lab_flux(exact_solve_f32(f, wp, ex, UU, fi, g));
           // this lane alone holds face li: its words are read, its fluxes
           // take their place
-          stage[0][li] = f.m;
-          stage[1][li] = f.e;
-          stage[2][li] = f.un * n1 - f.ut * n2;
-          stage[3][li] = f.un * n2 + f.ut * n1;
+          stage[0][li] = q.m;
+          stage[1][li] = q.e;
+          stage[2][li] = q.un * n1 - q.ut * n2;
+          stage[3][li] = q.un * n2 + q.ut * n1;
           stage[4][li] = krad * frcp(UU);
           if (info) {
             info[2 * i] = fi.it;
@@ -229,17 +212,28 @@ __global__ __launch_bounds__(SORT_NT) void exact_sorted_kernel(size_t n,
 }
 
 template <int METHOD>
-static int launch_unsorted(size_t n, const float* in, float n1, float n2, float krad,
-                           const ExactCtx& ex, float* out, ast_stats_t* stats, int* info,
-                           hipStream_t stream);
-
-template <int METHOD>
 static int launch(size_t n, const float* in, float n1, float n2, float krad, const ExactCtx& ex,
                   float* out, ast_stats_t* stats, int* info, hipStream_t stream) {
+  // The sort pays where the solver's instructions bound the kernel; a launch
+  // that leaves the chip part idle waits for its longest chain instead, which
+  // the sort and its barriers lengthen.  Measured, exact, us (face order /
+  // sorted): 50001 faces 5.5 / 7.3, 200000 7.1 / 7.9, 400000 10.0 / 10.9,
+  // 1000001 19.1 / 19.3, 2000003 32.1 / 30.2, 2^24 213 / 188.
+  const bool plain = METHOD != AST_EXACT ||
+                     (n <= (size_t(1) << 20) && ex.mlp == nullptr && !stats && !info);
+  if (plain) {
+    size_t blocks = (n + FNT - 1) / FNT;
+    if (blocks > 256 * 64) blocks = 256 * 64;
+    hipLaunchKernelGGL((flux_kernel<METHOD>), dim3((unsigned)blocks), dim3(FNT), 0, stream, n, in,
+                       n1, n2, krad, ex, out);
+    AST_LAUNCH_CHECK("ast_flux_f32 launch");
+    return AST_OK;
+  }
   if constexpr (METHOD == AST_EXACT) {
-    // one tile per workgroup (measured on 2^24 faces: 512-face tiles, one per
-    // workgroup, 346 us; 1024-face tiles 367-403 us; 4096 workgroups looping
-    // over the tiles 389-427 us), a loop over tiles beyond 2^20 workgroups
+    // one tile per workgroup (measured on 2^24 faces, before the solver's
+    // present form: 512-face tiles, one per workgroup, 346 us; 1024-face tiles
+    // 367-403 us; 4096 workgroups looping over the tiles 389-427 us), a loop
+    // over tiles beyond 2^20 workgroups
     size_t blocks = (n + STILE - 1) / STILE;
     if (blocks > (size_t(1) << 20)) blocks = size_t(1) << 20;
     const dim3 gr((unsigned)blocks), bl(SORT_NT);
@@ -262,21 +256,7 @@ static int launch(size_t n, const float* in, float n1, float n2, float krad, con
                          krad, ex, out, stats, info);
     }
     AST_LAUNCH_CHECK("ast_flux_f32 launch");
-    return AST_OK;
-  } else {
-    return launch_unsorted<METHOD>(n, in, n1, n2, krad, ex, out, stats, info, stream);
   }
-}
-
-template <int METHOD>
-static int launch_unsorted(size_t n, const float* in, float n1, float n2, float krad,
-                           const ExactCtx& ex, float* out, ast_stats_t* stats, int* info,
-                           hipStream_t stream) {
-  size_t blocks = (n + FNT - 1) / FNT;
-  if (blocks > 256 * 64) blocks = 256 * 64;
-  hipLaunchKernelGGL((flux_kernel<METHOD, false, false>), dim3((unsigned)blocks), dim3(FNT), 0,
-                     stream, n, in, n1, n2, krad, ex, out, stats, info);
-  AST_LAUNCH_CHECK("ast_flux_f32 launch");
   return AST_OK;
 }
 

@@ -64,19 +64,21 @@ int ast_tile_rows_setting(void) { return g_krows; }
 // 2048x1024 20.5 / 22.9, 8192x400 26.9 / 29.1, 4096x2048 55.6 / 63.7.
 //
 // Exact solver: its waves differ by several times (patterns and iterations
-// diverge), so short strips balance them: 1 row up to 9400 wave rows
-// (bands x rows), 2 up to 20000, 4 up to 100000, 8 beyond, where the 5 rows
-// a strip reads and solves over those it holds weigh more.  Measured, us a
-// step (1 / 2 / 4 / 8 rows): 256x128 13.1 / 19.6 / 31.0 / 58.4, 1024x512
-// 20.5 / 21.0 / 32.4 / 56.3, 1500x750 34.5 / 27.6 / 36.0 / 63.5, 2048x1024
-// 58.1 / 43.8 / 40.0 / 61.1, 8192x400 85.3 / 62.5 / 53.5 / 63.6, 4096x2048
-// 209 / 149 / 121 / 111.
+// diverge), so short strips balance them: the strips' extra rows (5 read, one
+// solved) cost in proportion to 1/h, the last wave's lead to h over the
+// grid's wave rows (bands x rows), together least at h ~ sqrt(wave rows):
+// sqrt(wave rows / 2300), 1 to 8.  Measured, us a step (1 / 2 / 3 / 4 / 5 / 6 / 8
+// rows): 256x128 12.7 / 14.5 / 18.1 / 21.6 / 25.1 / 28.7 / 35.6, 1024x512
+// 23.2 / 19.7 / 20.5 / 23.7 / 27.2 / 30.6 / 38.5, 1500x750 35.8 / 28.0 / 25.5
+// / 25.8 / 29.3 / 33.5 / 39.0, 2047x1021 58.4 / 42.2 / 38.3 / 36.5 / 36.9 /
+// 37.0 / 41.1, 8192x400 83.8 / 59.2 / 53.0 / 50.9 / 49.3 / 49.6 / 50.1,
+// 4096x2048 202 / 140 / 119 / 112 / 107 / 105 / 101.
 static int default_tile(const ast_grid_t& g, int method) {
   const long long nbands = (g.N + WOUT - 1) / WOUT;
   int tile = 4;
   if (method == AST_EXACT) {
-    const long long rows = nbands * g.M;
-    tile = rows <= 9400 ? 1 : rows <= 20000 ? 2 : rows <= 100000 ? 4 : 8;
+    const double rows = (double)nbands * g.M;
+    tile = std::min(8, std::max(1, (int)(std::sqrt(rows / 2300.0) + 0.5)));
   } else {
     auto strips = [&](long long waves) { return waves * 1024 / nbands; };
     long long waves = 4;
