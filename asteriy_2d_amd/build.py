@@ -43,6 +43,7 @@ SOURCES = [
     ("step_f32.hip", FAST),
     ("step_f32_hll.hip", FAST),
     ("step_f32_exact.hip", FAST),
+    ("step_f32_exact5.hip", FAST),
     ("step_f32_learned.hip", FAST),
     ("step_f32_detect.hip", FAST),
     ("mlp.hip", FAST),

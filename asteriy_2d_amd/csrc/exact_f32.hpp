@@ -46,6 +46,16 @@ struct ExactCtx {
   // When set, the kernel ORs 1 into *strong when it meets a strong two-shock
   // face (the runtime's learned mode, time_slots.h).
   uint32_t* strong;
+  AST_DEV int order() const { return n; }
+};
+// The same with n known when the code is compiled: the powers are then
+// straight-line products without the scalar tests and branches of the other
+// orders (a fifth of the solver's code; the step at 2047x1021 36.4 -> 33.9 us,
+// 2^24 fluxes 190 -> 183).  n = 5 only, gamma = 5/3; the kernels that count or
+// serve the learned start keep the general code.
+struct ExactCtx5 : ExactCtx {
+  AST_DEV explicit ExactCtx5(const ExactCtx& e) : ExactCtx(e) {}
+  AST_DEV static constexpr int order() { return 5; }
 };
 
 static inline ExactCtx make_exact_ctx(double gamma, const void* mlp) {
@@ -100,19 +110,23 @@ AST_DEV float geom_sum(float x, int n) {
   return s;
 }
 // x^(1/gm): exact products for an integer 1/gm, else exp2/log2
-AST_DEV float pow_igm(const ExactCtx& e, float x) { return e.n ? ipow(x, e.n) : fpow(x, e.igm); }
+template <class E>
+AST_DEV float pow_igm(const E& e, float x) {
+  return e.order() ? ipow(x, e.order()) : fpow(x, e.igm);
+}
 
 // x^(1/gm - 1), the same way
-AST_DEV float pow_igm1(const ExactCtx& e, float x) {
-  if (e.n == 5) {
+template <class E>
+AST_DEV float pow_igm1(const E& e, float x) {
+  if (e.order() == 5) {
     const float x2 = x * x;
     return x2 * x2;
   }
-  if (e.n == 7) {
+  if (e.order() == 7) {
     const float x2 = x * x;
     return x2 * x2 * x2;
   }
-  return e.n ? ipow(x, e.n - 1) : fpow(x, e.igm - 1.f);
+  return e.order() ? ipow(x, e.order() - 1) : fpow(x, e.igm - 1.f);
 }
 AST_DEV float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
 
@@ -252,7 +266,8 @@ AST_DEV float newton_f32(const ExactCtx& e, float du, float pI, float rI, float 
 // operations a step.  q = (pI/pII)^gm; the start takes side I as a
 // rarefaction too, whose root is (cI + cII + (g-1)/2 du)/(cI/q + cII).
 // Returns y and p.
-AST_DEV float shock_raref_f32(const ExactCtx& e, float du, float D, float pI, float rI, float cI,
+template <class E>
+AST_DEV float shock_raref_f32(const E& e, float du, float D, float pI, float rI, float cI,
                               float pII, float cII, float q, float& p, int& iters, bool& capped) {
   const float kI = 0.5f * e.g2 * rI, jI = 0.5f * e.g1 * rI * pI, zI = rI * cI, zzI = zI * zI;
   const float c2 = e.c2g1 * cII, hn = 0.5f * e.igm;
@@ -374,7 +389,8 @@ AST_DEV double sound_speed_d(double g, float p, float r, float c) {
 // 234-544) is one code for all, with the side that holds w = 0 mirrored onto
 // side I, so that lanes of different patterns and regions share it.  Faces
 // outside both rarefactions take a side's state without a p*.
-AST_DEV FaceF exact_solve_f32(const ExactFace& s, const WavePattern& w, const ExactCtx& e,
+template <class E>
+AST_DEV FaceF exact_solve_f32(const ExactFace& s, const WavePattern& w, const E& e,
                               float& UU, FaceInfo& fi, float guess) {
   const float g = e.g, g1 = e.g1, g2 = e.g2, gm = e.gm;
   const float enI = s.enI, enII = s.enII, pI = s.pI, pII = s.pII, rI = s.rI, rII = s.rII;
@@ -425,16 +441,16 @@ AST_DEV FaceF exact_solve_f32(const ExactFace& s, const WavePattern& w, const Ex
     if (shock) {
       aI = fsqrt(rI * fmaf(0.5f * g1, pI, hp));
       dI = enI - aI * frcp(rI);
-    } else if (e.n) {
-      aI = gm * zI * geom_sum(t, e.n);
+    } else if (e.order()) {
+      aI = gm * zI * geom_sum(t, e.order());
     } else if (!(fabsf(p - pI) < 1e-6f * pI)) {
       aI = gm * zI * (1.f - p * frcp(pI)) * frcp(1.f - t);
     }
     if (w.ss) {
       aII = fsqrt(rII * fmaf(0.5f * g1, pII, hp));
       dII = enII + aII * frcp(rII);
-    } else if (e.n) {
-      aII = gm * zII * geom_sum(y, e.n);
+    } else if (e.order()) {
+      aII = gm * zII * geom_sum(y, e.order());
     } else if (!(fabsf(p - pII) < 1e-6f * pII)) {
       aII = gm * zII * (1.f - p * frcp(pII)) * frcp(1.f - y);
     }
@@ -499,8 +515,8 @@ AST_DEV FaceF exact_solve_f32(const ExactFace& s, const WavePattern& w, const Ex
 // all its lanes on MFMA (a wave-uniform branch) and those lanes start
 // newton from it.
 // DETECT: report strong two-shock faces (fi.strong) without the network.
-template <bool LEARNED, bool DETECT = false>
-AST_DEV FaceF exact_frame_f32(const PrimF& L, const PrimF& R, const ExactCtx& e, float& UU,
+template <bool LEARNED, bool DETECT = false, class E>
+AST_DEV FaceF exact_frame_f32(const PrimF& L, const PrimF& R, const E& e, float& UU,
                               FaceInfo& fi, float guess = -1.f) {
   const ExactFace s = exact_sides(L, R, e);
   const WavePattern w = wave_pattern(s, e);
@@ -520,8 +536,8 @@ AST_DEV FaceF exact_frame_f32(const PrimF& L, const PrimF& R, const ExactCtx& e,
 }
 
 // The same flux in the lab frame (face-frame axes).
-template <bool LEARNED, bool DETECT = false>
-AST_DEV FluxF exact_f32(const PrimF& L, const PrimF& R, const ExactCtx& e, float& UU,
+template <bool LEARNED, bool DETECT = false, class E>
+AST_DEV FluxF exact_f32(const PrimF& L, const PrimF& R, const E& e, float& UU,
                         FaceInfo& fi, float guess = -1.f) {
   return lab_flux(exact_frame_f32<LEARNED, DETECT>(L, R, e, UU, fi, guess));
 }

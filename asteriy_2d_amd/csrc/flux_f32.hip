@@ -14,10 +14,12 @@ namespace f32 {
 
 constexpr int FNT = 256;
 
-template <int METHOD>
+// E: the exact solver's constants, with gamma = 5/3 compiled in or not.
+template <int METHOD, class E>
 __global__ __launch_bounds__(FNT) void flux_kernel(size_t n, const float* __restrict__ in,
                                                    float n1, float n2, float krad,
-                                                   ExactCtx ex, float* __restrict__ out) {
+                                                   ExactCtx ex0, float* __restrict__ out) {
+  const E ex(ex0);
   const size_t stride = (size_t)gridDim.x * FNT;
   for (size_t i = (size_t)blockIdx.x * FNT + threadIdx.x; i < n; i += stride) {
     const float rl = in[i], pl = in[n + i], vxl = in[2 * n + i], vyl = in[3 * n + i];
@@ -82,13 +84,14 @@ AST_DEV void face_frame(const float* w, float n1, float n2, PrimF& L, PrimF& R) 
   R = PrimF{w[4], w[5], w[6] * n1 + w[7] * n2, -w[6] * n2 + w[7] * n1};
 }
 
-template <bool STATS, int MODE>
+template <bool STATS, int MODE, class E = ExactCtx>
 __global__ __launch_bounds__(SORT_NT) void exact_sorted_kernel(size_t n,
                                                                const float* __restrict__ in,
                                                                float n1, float n2, float krad,
-                                                               ExactCtx ex, float* out,
+                                                               ExactCtx ex0, float* out,
                                                                ast_stats_t* stats,
                                                                int* __restrict__ info) {
+  const E ex(ex0);
   constexpr bool STRONG = MODE != kSolve;  // strong faces form a group of their own
   __shared__ uint32_t redi[(SORT_NT / 64) * 10];
   // slot -> face of the tile (low bits), its key and its swap
@@ -224,8 +227,10 @@ static int launch(size_t n, const float* in, float n1, float n2, float krad, con
   if (plain) {
     size_t blocks = (n + FNT - 1) / FNT;
     if (blocks > 256 * 64) blocks = 256 * 64;
-    hipLaunchKernelGGL((flux_kernel<METHOD>), dim3((unsigned)blocks), dim3(FNT), 0, stream, n, in,
-                       n1, n2, krad, ex, out);
+    const auto kernel = METHOD == AST_EXACT && ex.n == 5 ? flux_kernel<METHOD, ExactCtx5>
+                                                         : flux_kernel<METHOD, ExactCtx>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(FNT), 0, stream, n, in, n1, n2, krad,
+                       ex, out);
     AST_LAUNCH_CHECK("ast_flux_f32 launch");
     return AST_OK;
   }
@@ -251,6 +256,9 @@ static int launch(size_t n, const float* in, float n1, float n2, float krad, con
     } else if (st) {
       hipLaunchKernelGGL((exact_sorted_kernel<true, kSolve>), gr, bl, 0, stream, n, in, n1, n2,
                          krad, ex, out, stats, info);
+    } else if (ex.n == 5) {
+      hipLaunchKernelGGL((exact_sorted_kernel<false, kSolve, ExactCtx5>), gr, bl, 0, stream, n, in,
+                         n1, n2, krad, ex, out, stats, info);
     } else {
       hipLaunchKernelGGL((exact_sorted_kernel<false, kSolve>), gr, bl, 0, stream, n, in, n1, n2,
                          krad, ex, out, stats, info);

@@ -441,7 +441,7 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
   // exact solver's strips are of 1 to 8 rows (its waves differ too much for
   // taller ones), the FP64 step's of 1 to 32 or the tiling chosen by size
   int dflt[8] = {4, 8, 12, 16};
-  static const int dflt_exact[5] = {1, 2, 3, 4, 8};
+  static const int dflt_exact[7] = {1, 2, 3, 4, 5, 6, 8};
   int dflt64[12] = {0, 1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
   bool own64 = false;
   if ((!candidates || ncand <= 0) && S->precision == 0) {
@@ -452,7 +452,7 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
   }
   if ((!candidates || ncand <= 0) && S->method == AST_EXACT) {
     candidates = dflt_exact;
-    ncand = 5;
+    ncand = 7;
   }
   if (!candidates || ncand <= 0) {
     int nd = 4, dev = 0, cus = 0;

@@ -156,7 +156,7 @@ int ast_step_f32_rows(const ast_grid_t* g, const float* s, const float* u, float
         return tm->learned ? step_launch<kExactLearned>(a) : step_launch<kExactDetect>(a);
       }
       if (mlp != nullptr && !window) return step_launch<kExactLearned>(a);
-      return step_launch<AST_EXACT>(a);
+      return ex.n == 5 && stats == nullptr ? step_launch<kExact5>(a) : step_launch<AST_EXACT>(a);
     default: return ast_fail(AST_ERR_ARG, "ast_step_f32: unknown method %d", method);
   }
 }

@@ -43,6 +43,7 @@ extern template int step_launch<AST_HLLC_A>(const StepArgs&);
 extern template int step_launch<AST_EXACT>(const StepArgs&);
 extern template int step_launch<kExactLearned>(const StepArgs&);
 extern template int step_launch<kExactDetect>(const StepArgs&);
+extern template int step_launch<kExact5>(const StepArgs&);
 
 #ifdef AST_STEP_F32_KERNELS
 
@@ -116,8 +117,9 @@ int launch_f32(const ast_grid_t& g, const Consts& c, const ExactCtx& ex, const f
   // pulsed sides: the PULSE kernels of the HLL family, and of the plain
   // exact solver without counters or source planes (the other exact-solver
   // kernels serve pulsed sides on the boundary strip path)
-  constexpr bool kPulseKernels = !is_exact(METHOD) || METHOD == AST_EXACT;
+  constexpr bool kPulseKernels = !is_exact(METHOD) || METHOD == AST_EXACT || METHOD == kExact5;
   constexpr bool kPulseSrcKernels = !is_exact(METHOD);
+  constexpr bool kCounts = is_exact(METHOD) && METHOD != kExact5;
   const bool pulsed = kPulseKernels && c.pulsed;
 #define AST_LAUNCH_K(STATS_, SRC_, PULSE_, SRCV)                                                    \
   hipLaunchKernelGGL((step_kernel<METHOD, GEOM, WINDOW, STATS_, SRC_, PULSE_>), dim3(grid),        \
@@ -136,9 +138,8 @@ int launch_f32(const ast_grid_t& g, const Consts& c, const ExactCtx& ex, const f
   if (src != nullptr) {
     if constexpr (kSrc) {
       const bool f32 = src->xy != nullptr || src->e != nullptr;
-      const bool counting = is_exact(METHOD) && stats != nullptr;
-      if (counting) {
-        if constexpr (is_exact(METHOD)) {
+      if (kCounts && stats != nullptr) {
+        if constexpr (kCounts) {
           if (f32) AST_LAUNCH_K(true, kSrcF32, false, *src);
           else AST_LAUNCH_K(true, kSrcF64, false, *src);
         }
@@ -150,8 +151,8 @@ int launch_f32(const ast_grid_t& g, const Consts& c, const ExactCtx& ex, const f
     } else {
       return ast_fail(AST_ERR_ARG, "ast_step_f32: source planes with the learned start");
     }
-  } else if (is_exact(METHOD) && stats != nullptr) {
-    if constexpr (is_exact(METHOD)) AST_LAUNCH_K(true, kSrcNone, false, none);
+  } else if (kCounts && stats != nullptr) {
+    if constexpr (kCounts) AST_LAUNCH_K(true, kSrcNone, false, none);
   } else {
     AST_LAUNCH_P(kPulseKernels, false, kSrcNone, none);
   }

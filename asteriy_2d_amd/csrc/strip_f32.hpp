@@ -183,9 +183,12 @@ static inline int check_positive_bc(const ast_grid_t& g) {
 // that reports strong two-shock faces (the other half of a gated launch).
 constexpr int kExactLearned = 16;
 constexpr int kExactDetect = 17;
+// the plain exact solver with gamma = 5/3 compiled in (ExactCtx5)
+constexpr int kExact5 = 18;
 // the exact solver, in any of its kernel variants
 constexpr bool is_exact(int method) {
-  return method == AST_EXACT || method == kExactLearned || method == kExactDetect;
+  return method == AST_EXACT || method == kExactLearned || method == kExactDetect ||
+         method == kExact5;
 }
 
 template <int METHOD>
@@ -194,6 +197,7 @@ AST_DEV FaceF face_flux(const PrimF& L, const PrimF& R, const Consts& c, float& 
   if constexpr (METHOD == AST_HLL) return hll_frame_f32(L, R, c.g, c.ig1, UU);
   else if constexpr (METHOD == AST_HLLC) return hllc_frame_f32<false>(L, R, c.g, c.ig1, UU);
   else if constexpr (METHOD == AST_HLLC_A) return hllc_frame_f32<true>(L, R, c.g, c.ig1, UU);
+  else if constexpr (METHOD == kExact5) return exact_frame_f32<false>(L, R, ExactCtx5(ex), UU, fi);
   else return exact_frame_f32<METHOD == kExactLearned, METHOD == kExactDetect>(L, R, ex, UU, fi);
 }
 
