@@ -226,4 +226,22 @@ AST_DEV void step_dt_commit(double* T, const KTime& kt, double t) {
   }
 }
 
+// The wave's dt candidate after the T that the first step of a run finds:
+// that step lowers T (set_time may have left one below the step's own
+// minimum), so its slots start from it and T[0] is reset, by wave 0 of
+// workgroup 0 (every lane active).  Compared as the atomics compare, by the
+// IEEE bits: a T that is negative or NaN limits nothing.
+AST_DEV double lower_of(double t, double T) {
+  const auto a = (unsigned long long)__double_as_longlong(t);
+  const auto b = (unsigned long long)__double_as_longlong(T);
+  return b < a ? T : t;
+}
+AST_DEV double first_step_min(double tmin, double* T, const KTime& kt) {
+  if (kt.cur != nullptr && kt.prev == nullptr && blockIdx.x == 0 && threadIdx.x < 64) {
+    tmin = lower_of(tmin, T[0]);
+    if ((threadIdx.x & 63) == 0) T[0] = kSlotEmpty;
+  }
+  return tmin;
+}
+
 }  // namespace ast

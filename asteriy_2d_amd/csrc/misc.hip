@@ -19,7 +19,8 @@ __global__ void funk_time_kernel(double* T, double* T_do, double* TT, int* i) {
 
 // The time advance that closes a run of steps on the runtime's time block
 // (time_slots.h): funk_time with T = the minimum of the slots of set `last`
-// (the last step's), and every set cleared for the next run.  With `flags`
+// (the last step's; the first step has put the T it found into its slots),
+// and every set cleared for the next run.  With `flags`
 // (pinned host memory, 2 words), the run's strong-face flag goes to
 // flags[run & 1] and is cleared, and the run is counted.  One wave; lane k
 // folds and clears slot k.
@@ -29,7 +30,6 @@ __global__ void funk_time_fold_kernel(double* T, int last, int nslots, uint32_t*
   double t = k < nslots ? L[kSlotStride * k] : INFINITY;
   t = wave_min(t);
   if (k == 0) {
-    t = fmin(t, *T);  // a step launched without slots lowers T itself
     T[1] = t;
     T[2] = T[2] + t;
     T[0] = kSlotEmpty;
