@@ -70,7 +70,7 @@ AST_DEV void batch_item(const BatchInst& I, int local, int from, int j, double* 
       *i = *i + 1;
     } else {
       // the first step lowers the T it finds, which its slot then holds
-      tmin = fmin(tmin, T[0]);
+      tmin = lower_of(tmin, T[0]);
       T[0] = kSlotEmpty;
     }
   }

@@ -514,12 +514,7 @@ __global__ __launch_bounds__(NT, (step_waves<METHOD, G>())) void strip_kernel(St
   double tmin = any_out ? 1000.0 : INFINITY;
   if (UUx > 0.0) tmin = fmin(tmin, g.krit * g.dx / UUx);
   if (UUy > 0.0) tmin = fmin(tmin, g.krit * g.dy / UUy);
-  // the first step of a run lowers the T it finds (set_time may have left one
-  // below the step's own minimum), which the slots then hold
-  if (A.kt.cur != nullptr && A.kt.prev == nullptr && blockIdx.x == 0 && threadIdx.x < 64) {
-    tmin = fmin(tmin, A.T[0]);
-    if (lane == 0) A.T[0] = kSlotEmpty;
-  }
+  tmin = first_step_min(tmin, A.T, A.kt);
   block_min_uniform<NT>(tmin, red, A.kt.cur ? A.kt.cur : A.T, A.kt.cur ? A.kt.nslots : 0);
   if constexpr (STATS) block_counters_to(cnt, redc, A.stats);
 }

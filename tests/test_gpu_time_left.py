@@ -48,3 +48,25 @@ def test_time_left_below_the_steps_minimum(dev, precision, method):
                 t = sim.time()
                 assert t["T"] == 1e7 and t["T_do"] == t_do and t["TT"] == tt and t["i"] == n
                 assert np.array_equal(a, s) and np.array_equal(b, u)
+
+
+# positive IEEE doubles order like their bits, by which the step's atomic compares (on the
+# protocol's *T as well), so these limit nothing
+@pytest.mark.parametrize("T0", [-1.0, -0.0, float("nan")])
+def test_negative_time_limits_nothing(dev, T0):
+    from asteriy_2d_amd.batch import Batch
+    from asteriy_2d_amd.sim import Simulation
+    import torch
+    p = problems.wind(62, 4)  # one workgroup
+    for precision, dt in (("f32", torch.float32), ("f64", torch.float64)):
+        want = _protocol(p, G.HLLC, dt, 1, T0, dev)[2]
+        assert 0.0 < want < 1000.0
+        with Simulation(p.grid, G.HLLC, precision, p.s, p.u) as sim:
+            sim.set_time(T0, T_DO, 0.0, 0)
+            sim.run(1)
+            assert sim.time()["T_do"] == want, precision
+        if precision == "f32":
+            with Batch([p.grid], G.HLLC, [(p.s, p.u)]) as b:
+                b.set_time(0, T0, T_DO, 0.0, 0)
+                b.run(1)
+                assert b.time(0)["T_do"] == want
