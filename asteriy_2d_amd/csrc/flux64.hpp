@@ -53,13 +53,18 @@ struct FluxD {
 //
 // The compiler's FP64 division is 11 instructions, its square root about 16:
 // both scale their operands so that results near the ends of the exponent
-// range round correctly too.  The solvers' operands lie far inside it, so
-// here the hardware estimate (relative error 2^-24 measured for v_rcp_f64 and
-// v_rsq_f64) takes one Newton step (2^-47) and the quotient or root one
-// residual correction: 7 and 11 instructions, every result equal to the IEEE
-// one on 2^24 random operands over 2^+-200.  v_div_fixup keeps the IEEE
-// results for zeros, infinities and NaN.  rcp64 is the reciprocal to ~2^-47,
-// which one denominator's quotients share (div64 with three arguments).
+// range round correctly too.  Here the hardware estimate (relative error
+// 2^-24 measured for v_rcp_f64 and v_rsq_f64) takes one Newton step (2^-47)
+// and the quotient or root one residual correction: 7 and 11 instructions,
+// equal to the IEEE results on 2^20 random operands over 2^+-200 (tests; 2^22
+// exact fluxes 198 us, 248 with the compiler's; 217 with its scaled operands
+// and this one's steps).  v_div_fixup keeps the IEEE results for zeros,
+// infinities and NaN, and gives the infinity of a quotient that overflows,
+// whose residual is NaN.  What is not IEEE's: a denominator of magnitude 2^-1024
+// or less (its reciprocal overflows) gives an infinity, and a quotient or
+// root whose numerator or argument is below 2^-968 may be off in its last bits.
+// rcp64 is the reciprocal to ~2^-47, which one denominator's quotients share
+// (div64 with three arguments).
 AST_HD double rcp64(double b) {
 #ifdef __HIP_DEVICE_COMPILE__
   const double r = __builtin_amdgcn_rcp(b);

@@ -138,7 +138,12 @@ int ast_grid_check(const ast_grid_t* g);
  * out : 5 planes of n values: Ps.x (mass), Ps.y (energy), Pu.x, Pu.y
  *       (momentum, lab axes), and the operator's return value (local dt).
  * The FP32 variant computes in float; its exact solver keeps the p* solve
- * in FP64 near vacuum and in strong rarefactions. */
+ * in FP64 near vacuum and in strong rarefactions.
+ * The FP64 operators and the FP64 step form quotients and roots equal to the
+ * IEEE ones, zeros, infinities, NaN and overflow included, but for the last
+ * range of the exponents: a denominator (a density, a sum of impedances) of
+ * 2^-1024 = 5.6e-309 or less counts as zero, and a numerator or a root's
+ * argument below 2^-968 = 4e-292 may cost the last bits. */
 int ast_flux_f64(int method, size_t n, const double* in, double n1, double n2,
                  double rad, double gamma, double krit, double* out,
                  ast_stats_t* stats, void* stream);
