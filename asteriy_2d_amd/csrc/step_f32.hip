@@ -37,19 +37,22 @@
 using namespace ast;
 using namespace ast::f32;
 
-// The tiling set by ast_set_tile_rows (0: not set, the step takes
-// default_tile's)
+// The tiling set by ast_set_tile_rows (0: none, the step takes
+// default_tile's).  8 stands for none in both calls, as it was the tiling of a
+// step for which none was set: a caller that saves the setting, changes it
+// and sets it back leaves the choice by size as it found it.
 static int g_krows = 0;
+constexpr int kNoTiling = 8;
 
 // krows > 0: rows per strip; krows = -S: S strips of (nearly) equal height
 // per band (strip_rows)
 extern "C" int ast_set_tile_rows(int krows) {
   if (krows == 0 || krows > 1024 || krows < -(1 << 20))
     return ast_fail(AST_ERR_ARG, "ast_set_tile_rows: %d", krows);
-  g_krows = krows;
+  g_krows = krows == kNoTiling ? 0 : krows;
   return AST_OK;
 }
-extern "C" int ast_get_tile_rows(void) { return g_krows ? g_krows : 8; }
+extern "C" int ast_get_tile_rows(void) { return g_krows ? g_krows : kNoTiling; }
 int ast_tile_rows_setting(void) { return g_krows; }
 
 // The tiling of a step for which none was set, by the grid's size.

@@ -477,9 +477,9 @@ long long ast_batch_cells(const ast_batch_t* b);
 
 /* ---- tile configuration of the stand-alone FP32 step entry point --------
  * Strip tiling as for ast_sim_set_tile_rows, for the steps and for
- * simulations created afterwards.  Until it is set (ast_get_tile_rows then
- * returns 8) each step takes the tiling its rule gives for the grid's size
- * and method; the tiling never changes a result. */
+ * simulations created afterwards.  8, the value before any is set, leaves
+ * each step the tiling its rule gives for the grid's size and method, so
+ * set(get()) changes nothing; the tiling never changes a result. */
 int ast_set_tile_rows(int rows);
 int ast_get_tile_rows(void);
 /* Doubles of device memory ast_conservation_sums needs at `out` (the two
