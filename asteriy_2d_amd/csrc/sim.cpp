@@ -409,12 +409,16 @@ extern "C" int ast_sim_set_mlp(ast_sim_t* S, const ast_mlp_t* mlp) {
   return AST_OK;
 }
 
-// Strip tiling of the FP32 step (its tile shape; see the autotuner): rows
-// per wave strip, or -S for S strips of (nearly) equal height per band.
+// Is it a tiling of the simulation's step: rows per wave strip, or -S for S
+// strips of (nearly) equal height per band?
+static bool tiling(const ast_sim_t* S, int rows) {
+  return rows != 0 && rows <= (S->precision == 0 ? 4096 : 1024) &&
+         (rows > 0 || -(long long)rows <= S->g.M);
+}
+
 extern "C" int ast_sim_set_tile_rows(ast_sim_t* S, int krows) {
   if (!S) return ast_fail(AST_ERR_ARG, "ast_sim_set_tile_rows: null sim");
-  if (S->precision == 0 ? (krows < 1 || krows > 4096)
-                        : (krows == 0 || krows > 1024 || (krows < 0 && -(long long)krows > S->g.M)))
+  if (!tiling(S, krows))
     return ast_fail(AST_ERR_ARG, "ast_sim_set_tile_rows: %d", krows);
   CK(hipStreamSynchronize(S->stream));
   if (S->precision == 0) S->rows64 = krows;
@@ -425,46 +429,40 @@ extern "C" int ast_sim_set_tile_rows(ast_sim_t* S, int krows) {
 
 extern "C" void* ast_sim_stream(ast_sim_t* S) { return S ? (void*)S->stream : nullptr; }
 
-// Tile autotuner of the FP32 step: times `reps` launches of the step kernel
-// for each candidate strip tiling (rows per wave strip, or -S: S strips of
-// (nearly) equal height per band) on the simulation's own
-// state and stream, keeps the fastest, and restores the time scalars (the
-// repeated launches read the current planes and only write the spare ones).
-// best_rows / best_us (may be NULL) report the choice.  The FP64 step has a
-// fixed tile; for it this only reports the step time.
+// Tile autotuner: times `reps` launches of the step kernel for each candidate
+// strip tiling (rows per wave strip, or -S: S strips of (nearly) equal height
+// per band) on the simulation's own state and stream, keeps the fastest, and
+// restores the time scalars (the repeated launches read the current planes
+// and only write the spare ones).  best_rows / best_us (may be NULL) report
+// the choice, which ast_sim_set_tile_rows takes.
 extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, int reps,
                                 int* best_rows, float* best_us) {
   if (!S) return ast_fail(AST_ERR_ARG, "ast_sim_autotune: null sim");
-  // default: strips of 4-16 rows, and the tilings that give every SIMD 2 to
-  // 5 waves of (nearly) equal height, S strips per band with S * bands
-  // waves (a wave strip has 60 output columns; a CU has 4 SIMDs); the FP32
-  // exact solver's strips are of 1 to 8 rows (its waves differ too much for
-  // taller ones), the FP64 step's of 1 to 32 or the tiling chosen by size
-  int dflt[8] = {4, 8, 12, 16};
-  static const int dflt_exact[7] = {1, 2, 3, 4, 5, 6, 8};
-  int dflt64[12] = {0, 1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
-  bool own64 = false;
-  if ((!candidates || ncand <= 0) && S->precision == 0) {
-    dflt64[0] = ast_step_f64_default_tile(&S->g, S->method);
-    own64 = true;
-    candidates = dflt64;
-    ncand = 12;
-  }
-  if ((!candidates || ncand <= 0) && S->method == AST_EXACT) {
-    candidates = dflt_exact;
-    ncand = 7;
-  }
+  // default: FP32 strips of 4-16 rows and the tilings that give every SIMD 2 to
+  // 5 waves of (nearly) equal height, S strips per band with S * bands waves (a
+  // wave strip has 60 output columns; a CU has 4 SIMDs); FP32 exact solver
+  // strips of 1 to 8 rows (its waves differ too much for taller ones); FP64
+  // strips of 1 to 32 rows and the tiling chosen by size
+  std::vector<int> dflt;
   if (!candidates || ncand <= 0) {
-    int nd = 4, dev = 0, cus = 0;
-    CK(hipGetDevice(&dev));
-    CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int nbands = (S->g.N + 59) / 60;
-    for (int waves = 2; waves <= 5; waves++) {
-      const int ns = waves * 4 * cus / nbands;
-      if (ns >= 1 && S->g.M / ns >= 4) dflt[nd++] = -ns;
+    if (S->precision == 0) {
+      dflt.push_back(ast_step_f64_default_tile(&S->g, S->method));
+      for (int r : {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32}) dflt.push_back(r);
+    } else if (S->method == AST_EXACT) {
+      for (int r : {1, 2, 3, 4, 5, 6, 8}) dflt.push_back(r);
+    } else {
+      for (int r : {4, 8, 12, 16}) dflt.push_back(r);
+      int dev = 0, cus = 0;
+      CK(hipGetDevice(&dev));
+      CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+      const int nbands = (S->g.N + 59) / 60;
+      for (int waves = 2; waves <= 5; waves++) {
+        const int ns = waves * 4 * cus / nbands;
+        if (ns >= 1 && S->g.M / ns >= 4) dflt.push_back(-ns);
+      }
     }
-    candidates = dflt;
-    ncand = nd;
+    candidates = dflt.data();
+    ncand = (int)dflt.size();
   }
   if (reps < 1) reps = 10;
   double saved[ast::kGateWord + 1];  // T, T_do, TT, i and the learned-mode words
@@ -495,10 +493,7 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
                                    (double*)u2, S->scal, S->scal + 1, S->scal + 2, S->method,
                                    nullptr, kr, &tm, sources64(S), S->stream);
   };
-  auto valid = [&](int kr) {
-    if (S->precision == 0) return (own64 || kr >= 1) && kr <= 4096;
-    return !(kr == 0 || kr > 1024 || (kr < 0 && -kr > S->g.M));
-  };
+  auto valid = [&](int kr) { return tiling(S, kr); };
   const int n = ncand;
   // warm-up: the clocks of an idle device ramp over the first tens of
   // milliseconds of work, which would slow the first candidates; untimed
@@ -550,8 +545,7 @@ extern "C" int ast_sim_autotune(ast_sim_t* S, const int* candidates, int ncand, 
     S->rows64 = best;
     drop_graph(S);
   }
-  // an FP64 tiling of equal strips is reported by their height
-  if (best_rows) *best_rows = S->precision == 0 && best < 0 ? (S->g.M - best - 1) / -best : best;
+  if (best_rows) *best_rows = best;
   if (best_us) *best_us = best_t;
   return AST_OK;
 }

@@ -158,9 +158,10 @@ class Simulation:
         native.call("ast_sim_set_tile_rows", self.h, int(krows))
 
     def autotune(self, candidates=None, reps: int = 10):
-        """Picks the fastest FP32 strip tiling for this grid (csrc/sim.cpp);
-        returns (tiling, microseconds per step): rows per wave strip, or -S
-        for S strips of (nearly) equal height per 60-column band."""
+        """Picks the fastest strip tiling for this grid (csrc/sim.cpp); returns
+        (tiling, microseconds per step): rows per wave strip, or -S for S
+        strips of (nearly) equal height per 60-column band.  set_tile_rows
+        takes the tiling back."""
         arr, n = None, 0
         if candidates:
             n = len(candidates)

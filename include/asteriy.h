@@ -417,17 +417,17 @@ int ast_sim_learned_modes(ast_sim_t* sim, int* modes);
  * solver / the learned start (for strong faces that last too few steps for
  * the automatic choice to meet them). */
 int ast_sim_set_learned_mode(ast_sim_t* sim, int mode);
-/* Strip tiling of the step.  FP32: rows > 0 rows per wave strip, rows = -S
- * S strips of (nearly) equal height per band of 60 columns; strips of 4 (the
- * exact solver: 1) to 64 rows inside the grid take the fast strip path
- * (default: chosen from the grid's size and the method).  FP64: rows > 0 rows
- * per wave strip (default: chosen from the grid's size and the method). */
+/* Strip tiling of the step: rows > 0 rows per wave strip (FP32 up to 1024,
+ * FP64 4096), rows = -S S strips of (nearly) equal height per band of 60
+ * columns; by default it is chosen from the grid's size and the method.
+ * FP32: strips of 4 (the exact solver: 1) to 64 rows inside the grid take
+ * the fast strip path. */
 int ast_sim_set_tile_rows(ast_sim_t* sim, int rows);
 /* Times the step for each candidate tiling (NULL = a default list: FP32 4,
  * 8, 12, 16 rows and the tilings -S that give every SIMD 2, 3, 4 or 5 equal
- * waves, with the exact solver 1, 2, 3, 4, 8 rows; FP64 1 to 6, 8, 12, 16,
- * 24, 32 rows and the tiling chosen by size, which is reported by its rows),
- * keeps the fastest; reports it (may be NULL).  State and time are left
+ * waves, with the exact solver 1 to 6 and 8 rows; FP64 1 to 6, 8, 12, 16, 24,
+ * 32 rows and the tiling chosen by size), keeps the fastest; reports it (may
+ * be NULL) as ast_sim_set_tile_rows takes it.  State and time are left
  * unchanged. */
 int ast_sim_autotune(ast_sim_t* sim, const int* candidates, int ncand, int reps,
                      int* best_rows, float* best_us);
