@@ -109,8 +109,10 @@ def stream_handle(stream=None) -> int:
     import torch
     if stream is not None:
         return stream.cuda_stream
-    if torch.cuda.is_initialized():
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # not in every torch
+    device = getattr(torch._C, "_cuda_getDevice", None)
+    if raw is not None and device is not None and torch.cuda.is_initialized():
+        return raw(device())
     return torch.cuda.current_stream().cuda_stream
 
 
