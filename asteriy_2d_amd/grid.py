@@ -116,12 +116,33 @@ class Grid:
     def to_c(self) -> CGrid:
         # one packed write: assigning the fields one by one takes twice as long
         bc, st = self.bc, self.bc_state
-        return CGrid.from_buffer_copy(_PACK.pack(
-            self.N, self.M, self.geometry, int(bc[0]), int(bc[1]), int(bc[2]), int(bc[3]),
-            self.x_min, self.dx, self.y_min, self.dy, self.gamma, self.krit,
-            *st[0][:4], *st[1][:4], *st[2][:4], *st[3][:4], *self.bc_vclamp[:4],
-            self.ho_lo, self.ho_hi, self.frozen_x0, self.frozen_ax, self.frozen_ay,
-            *self.bc_pulse[:4]))
+        try:
+            return CGrid.from_buffer_copy(_PACK.pack(
+                self.N, self.M, self.geometry, int(bc[0]), int(bc[1]), int(bc[2]), int(bc[3]),
+                self.x_min, self.dx, self.y_min, self.dy, self.gamma, self.krit,
+                *st[0][:4], *st[1][:4], *st[2][:4], *st[3][:4], *self.bc_vclamp[:4],
+                self.ho_lo, self.ho_hi, self.frozen_x0, self.frozen_ax, self.frozen_ay,
+                *self.bc_pulse[:4]))
+        except Exception:
+            # values that need a conversion (numbers as text in the states), and
+            # the errors of those that have none
+            return self._fields_to_c()
+
+    def _fields_to_c(self) -> CGrid:
+        g = CGrid()
+        g.N, g.M, g.geometry = self.N, self.M, self.geometry
+        for i in range(4):
+            g.bc[i] = int(self.bc[i])
+            g.bc_vclamp[i] = float(self.bc_vclamp[i])
+            for j in range(4):
+                g.bc_state[i][j] = float(self.bc_state[i][j])
+        g.x_min, g.dx, g.y_min, g.dy = self.x_min, self.dx, self.y_min, self.dy
+        g.gamma, g.krit = self.gamma, self.krit
+        g.ho_lo, g.ho_hi = self.ho_lo, self.ho_hi
+        g.frozen_x0, g.frozen_ax, g.frozen_ay = self.frozen_x0, self.frozen_ax, self.frozen_ay
+        for i in range(4):
+            g.bc_pulse[i] = float(self.bc_pulse[i])
+        return g
 
     def replace(self, **kw) -> "Grid":
         d = dict(self.__dict__)
