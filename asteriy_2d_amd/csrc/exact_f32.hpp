@@ -228,7 +228,7 @@ constexpr float kStep = 1e-4f;
 // ones.  dfK/dp = hK (1 + zK^2 hK^2)/2: three transcendental operations a
 // step.  pee: the PVRS-type estimate, kernel.cu:640, the start unless a
 // learned guess is used.  Every iterate is kept at or above pII (p* > pII in
-// this pattern).
+// this pattern); a NaN stays one.
 AST_DEV float newton_f32(const ExactCtx& e, float du, float pI, float rI, float cI, float pII,
                          float rII, float cII, float guess, bool use_guess, int& iters,
                          bool& capped) {
@@ -253,7 +253,8 @@ AST_DEV float newton_f32(const ExactCtx& e, float du, float pI, float rI, float 
     w = fmaxf(w + dw, wlo);
   }
   iters = k;
-  return fmaxf(fmaf(dw, fmaf(2.f, w, dw), p), pII);  // (w + dw)^2
+  const float pn = fmaf(dw, fmaf(2.f, w, dw), p);  // (w + dw)^2
+  return pn < pII ? pII : pn;
 }
 
 // Shock + rarefaction: the root of lev (kernel.cu:751-765) on devtwo's
@@ -467,7 +468,7 @@ AST_DEV FaceF exact_solve_f32(const ExactFace& s, const WavePattern& w, const E&
     en = en0;
     pp = one ? pI : pII;
     r = one ? rI : rII;
-    if (!(0.f <= head)) {
+    if (head < 0.f) {  // (a NaN speed: the side's state)
       if (sh0) {
         const float a0 = one ? aI : aII;
         r = r * a0 * frcp(a0 - r * (en0 - us));
