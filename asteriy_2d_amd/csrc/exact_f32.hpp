@@ -221,12 +221,14 @@ constexpr float kStep = 1e-4f;
 
 // Two shocks: the root of kernel.cu:635-680's equation
 //   fI(p) + fII(p) = enI - enII,  fK = (p - pK) hK,
-//   1/hK^2 = aK^2 = rK ((g+1) p + (g-1) pK)/2
-// (the reference's zK^2 (gp p/pK + gm) with zK = rK cK multiplied out: no
-// division by pK) by Newton in w = sqrt(p): a strong shock's fK grows like
-// sqrt(p), which is linear in w, so strong faces need no more steps than weak
-// ones.  dfK/dp = hK (1 + zK^2 hK^2)/2: three transcendental operations a
-// step.  pee: the PVRS-type estimate, kernel.cu:640, the start unless a
+//   1/hK = zK sqrt(gp p/pK + gm),  zK = rK cK
+// by Newton in w = sqrt(p): a strong shock's fK grows like sqrt(p), which is
+// linear in w, so strong faces need no more steps than weak ones.  With sK =
+// (gp p/pK + gm)^-1/2, dfK/dp = hK (1 + sK^2)/2: three transcendental
+// operations a step.  In ratios of pressures, not as rK ((g+1) p + (g-1) pK)/2:
+// that product leaves the FP32 range first (r = 1e-24, p = 1e-14), and a
+// side without pressure has no p* here, as in the reference; the times are
+// the same.  pee: the PVRS-type estimate, kernel.cu:640, the start unless a
 // learned guess is used.  Every iterate is kept at or above pII (p* > pII in
 // this pattern); a NaN stays one.
 AST_DEV float newton_f32(const ExactCtx& e, float du, float pI, float rI, float cI, float pII,
@@ -234,19 +236,19 @@ AST_DEV float newton_f32(const ExactCtx& e, float du, float pI, float rI, float 
                          bool& capped) {
   const float zI = rI * cI, zII = rII * cII;
   const float pee = (pI * zII + pII * zI + du * zI * zII) * frcp(zI + zII);
-  const float kI = 0.5f * e.g2 * rI, kII = 0.5f * e.g2 * rII;
-  const float jI = 0.5f * e.g1 * rI * pI, jII = 0.5f * e.g1 * rII * pII;
-  const float zzI = zI * zI, zzII = zII * zII, wlo = fsqrt(pII);
+  const float gI = e.gp * frcp(pI), gII = e.gp * frcp(pII), iI = frcp(zI), iII = frcp(zII);
+  const float wlo = fsqrt(pII);
   float w = fmaxf(fsqrt(use_guess ? guess : pee), wlo);
   float p, dw;
   int k = 0;
   for (;;) {
     p = w * w;
     k++;
-    const float hI = frsq(fmaf(kI, p, jI)), hII = frsq(fmaf(kII, p, jII));
+    const float sI = frsq(fmaf(gI, p, e.gm)), sII = frsq(fmaf(gII, p, e.gm));
+    const float hI = iI * sI, hII = iII * sII;
     const float f = fmaf(p - pI, hI, fmaf(p - pII, hII, -du));
     // 2 df/dp
-    const float d = fmaf(hI, fmaf(zzI * hI, hI, 1.f), hII * fmaf(zzII * hII, hII, 1.f));
+    const float d = fmaf(hI, fmaf(sI, sI, 1.f), hII * fmaf(sII, sII, 1.f));
     dw = -f * frcp(w * d);  // df/dw = w d
     if (!(fabsf(dw) > kStep * w)) break;
     if (k >= AST_ITER_CAP) { capped = true; break; }
@@ -260,18 +262,19 @@ AST_DEV float newton_f32(const ExactCtx& e, float du, float pI, float rI, float 
 // Shock + rarefaction: the root of lev (kernel.cu:751-765) on devtwo's
 // bracket [pI, pII] (kernel.cu:682-749) by safeguarded Newton in
 // y = (p/pII)^gm, in which the rarefaction is linear and p = pII y^n,
-// n = 1/gm (5 for gamma 5/3: products, no power function):
-//   (p - pI) hI + c2 y - D = 0,  c2 = 2 cII/(g - 1),  D = c2 + enI - enII
-// (D from the caller: FP64-formed in strong rarefactions).  hI and the
-// shock's derivative are newton_f32's, dp/dy = n p/y: two transcendental
-// operations a step.  q = (pI/pII)^gm; the start takes side I as a
-// rarefaction too, whose root is (cI + cII + (g-1)/2 du)/(cI/q + cII).
-// Returns y and p.
+// n = 1/gm (5 for gamma 5/3: products, no power function).  With x = p/pII,
+// xI = pI/pII and the shock's 1/hI = (rI pII ((g+1) x + (g-1) xI)/2)^1/2,
+//   (rI/pII)^-1/2 (x - xI) s + c2 y - D = 0,  s = (((g+1) x + (g-1) xI)/2)^-1/2,
+//   c2 = 2 cII/(g - 1),  D = c2 + enI - enII
+// (D from the caller: FP64-formed in strong rarefactions); d/dx of (x - xI) s is
+// s (1 + g xI s^2)/2, dx/dy = n x/y: two transcendental operations a step.
+// q = (pI/pII)^gm; the start takes side I as a rarefaction too, whose root is
+// (cI + cII + (g-1)/2 du)/(cI/q + cII).  Returns y and p.
 template <class E>
 AST_DEV float shock_raref_f32(const E& e, float du, float D, float pI, float rI, float cI,
                               float pII, float cII, float q, float& p, int& iters, bool& capped) {
-  const float kI = 0.5f * e.g2 * rI, jI = 0.5f * e.g1 * rI * pI, zI = rI * cI, zzI = zI * zI;
-  const float c2 = e.c2g1 * cII, hn = 0.5f * e.igm;
+  const float xI = pI * frcp(pII), k2 = 0.5f * e.g2, j = 0.5f * e.g1 * xI, gx = e.g * xI;
+  const float A = fsqrt(pII) * frsq(rI), c2 = e.c2g1 * cII, hn = 0.5f * e.igm * A;
   float lo = q, hi = 1.f;
   float y = q * fmaf(0.5f * e.g1, du, cI + cII) * frcp(fmaf(q, cII, cI));
   y = fminf(fmaxf(y, lo), hi);
@@ -279,11 +282,11 @@ AST_DEV float shock_raref_f32(const E& e, float du, float D, float pI, float rI,
   int k = 0;
   for (;;) {
     k++;
-    const float m = pII * pow_igm1(e, y);  // p/y
-    p = m * y;
-    const float h = frsq(fmaf(kI, p, jI));
-    const float f = fmaf(p - pI, h, fmaf(c2, y, -D));
-    const float df = fmaf(hn * m * h, fmaf(zzI * h, h, 1.f), c2);
+    const float m = pow_igm1(e, y);  // x/y
+    const float x = m * y;
+    const float s = frsq(fmaf(k2, x, j));
+    const float f = fmaf(x - xI, A * s, fmaf(c2, y, -D));
+    const float df = fmaf(hn * m * s, fmaf(gx * s, s, 1.f), c2);
     const float dy = -f * frcp(df);
     if (f < 0.f) lo = y;
     else hi = y;
