@@ -172,7 +172,8 @@ static int batch_layout(ast_batch_t* B) {
 // its rows, so that all instances together give every SIMD 4 equal waves, or
 // 3, 2, 1 if the strips would be shorter than 4 rows (then strips of 4), or
 // 8-row strips taken in rounds where they would be taller than 64.  Exact
-// solver: rows by the wave rows of the sweep, as for one grid.
+// solver: 1, 2, 4 or 8 rows by the wave rows of the sweep, more rows the more
+// of them there are, as in a single grid's rule.
 static void batch_default_tiles(ast_batch_t* B) {
   long long rows = 0;  // wave rows of the sweep
   for (const auto& I : B->h) rows += (long long)((I.g.N + WOUT - 1) / WOUT) * I.g.M;

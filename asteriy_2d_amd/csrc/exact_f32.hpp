@@ -52,7 +52,9 @@ struct ExactCtx {
 // straight-line products without the scalar tests and branches of the other
 // orders (a fifth of the solver's code; the step at 2047x1021 36.4 -> 33.9 us,
 // 2^24 fluxes 190 -> 183).  n = 5 only, gamma = 5/3; the kernels that count or
-// serve the learned start keep the general code.
+// serve the learned start, and the batch's, keep the general code.  Measured
+// at gamma = 5/3 / 7/5 / 1.3: the step at 1021x509 15.4 / 16.4 / 16.1 us, 2^21
+// fluxes 31 / 35 / 34.
 struct ExactCtx5 : ExactCtx {
   AST_DEV explicit ExactCtx5(const ExactCtx& e) : ExactCtx(e) {}
   AST_DEV static constexpr int order() { return 5; }

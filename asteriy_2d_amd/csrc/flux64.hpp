@@ -109,6 +109,8 @@ struct GasD {
 // registers it holds stay out of the kernel (the FP64 exact kernels: 231 ->
 // 180 VGPRs in the step, 147 -> 96 in the flux batch, 1.17x and 1.32x the
 // speed).  n = 5 only, gamma = 5/3: every other gas takes the general code.
+// Measured at gamma = 5/3 / 7/5 / 1.3 (the last with pow): the step at 1021x509
+// 43 / 63 / 79 us, 2^21 fluxes 98 / 134 / 217.
 template <int N>
 struct GasN : GasD {
   AST_HDM explicit GasN(const GasD& a) : GasD(a) {}
@@ -374,17 +376,18 @@ AST_HD double two_shock_root(const GasD& a, double du, double pI, double rI, dou
 //
 // The replay: f increases, so its root r decides the sign of
 // f at every midpoint, and near the root |f(mid)| = f'(r) |mid - r|, which
-// decides the stopping test but for midpoints within 2% of its edge (more
-// where speeds above 1e4 round f by more); there f is evaluated.  The root comes from Newton in t = (p/p_II)^gm, in which
-// the fan's function is linear and the shock's a mild power, from the
+// decides the stopping test but for midpoints near its edge (`doubt`: within
+// 2% of it, more in proportion to speeds above 1250, which round f by more);
+// there f is evaluated.  The root comes from Newton in t = (p/p_II)^gm, in
+// which the fan's function is linear and the shock's a mild power, from the
 // chord's zero, kept inside the bracket.  A face takes the plain bisection
 // when the replay could decide otherwise than it: where Newton has not
-// converged to 1e-9 relative (leaving f(r) at rounding level), where f's
-// rounding, about 1e-15 of the speeds, is half of 1e-9 or more (speeds above
-// 5e5), or where f bends within the stopping window (p f' below 1e-6).  A
-// wave with one plain face takes its 50 evaluations after the others' Newton:
-// with speeds above 1e4 left to the bisection too, 65536 faces of gamma = 1.1
-// took 73 us, 1% of them plain (30 now; 50 for bisections alone).
+// converged to 1e-9 relative (leaving f(r) at rounding level), where the doubt
+// would be the whole window (speeds above 6e4), or where f bends within the
+// window (p f' below 1e-6).  A wave with one plain face takes its 50
+// evaluations after the others' Newton: with speeds above 1e4 left to the
+// bisection too, 65536 faces of gamma = 1.1 took 73 us, 1% of them plain (30
+// now; 50 for bisections alone).
 // Measured on the microbenchmark's faces: 33.5 iterations a face either way,
 // about 6 evaluations of f instead of 35 (with the powers as roots: the flux
 // batch of 2^22 faces 701 -> 251 us).

@@ -220,8 +220,10 @@ static int launch(size_t n, const float* in, float n1, float n2, float krad, con
   // The sort pays where the solver's instructions bound the kernel; a launch
   // that leaves the chip part idle waits for its longest chain instead, which
   // the sort and its barriers lengthen.  Measured, exact, us (face order /
-  // sorted): 50001 faces 5.5 / 7.3, 200000 7.1 / 7.9, 400000 10.0 / 10.9,
-  // 1000001 19.1 / 19.3, 2000003 32.1 / 30.2, 2^24 213 / 188.
+  // sorted), gamma = 5/3: 50001 faces 6.1 / 6.4, 200000 6.7 / 7.6, 400000 9.1 /
+  // 10.3, 1000001 17.4 / 18.0, 1200001 19.9 / 20.9, 2000003 29.3 / 28.9, 2^24
+  // 220 / 207; gamma = 7/5: 50001 6.1 / 7.4, 1000001 18.9 / 20.0, 2000003 31.3 /
+  // 31.7, 2^24 230 / 220.
   const bool plain = METHOD != AST_EXACT ||
                      (n <= (size_t(1) << 20) && ex.mlp == nullptr && !stats && !info);
   if (plain) {

@@ -107,8 +107,8 @@ struct Star {
   double r, q, v, w, bt, bm, e;
 };
 
-// Bound by HBM from 2^21 faces on (224 B/face): HLLD 2^21 faces in 99 us, 2^23
-// in 330 us (5.7 TB/s), 104 and 353 us with the compiler's divisions and
+// Bound by HBM from 2^21 faces on (224 B/face): HLLD 2^21 faces in 95 us, 2^23
+// in 330 us (5.7 TB/s), 101 and 353 us with the compiler's divisions and
 // square roots; the chain of ~16 quotients and 6 roots is what few waves
 // expose below that (2^20: 54 / 58 us).  Three waves a SIMD (156 VGPRs): a
 // fourth spills 100 B a lane (168 us at 2^21).
